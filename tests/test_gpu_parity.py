@@ -186,6 +186,20 @@ def test_pcg_matches_oracle(pv, ne, levels, fmg, nu):
     assert abs(c - cref) <= 1e-12 * abs(cref)
 
 
+@pytest.mark.parametrize("ne", [(64, 32, 32), (48, 40, 32), (72, 32, 32)])
+def test_pcg_product_partials_fit(pv, ne):
+    """Grids whose fused <d, K d> writes more partial sums (one per workgroup, up to tiles x node planes) than the
+    vector reductions (two sets): the launch refuses a buffer that they do not fit."""
+    tiles = -(-(ne[1] + 1) // 15) * -(-(ne[2] + 1) // 15)
+    sets = 2 * 3 * (ne[0] + 1) * -(-(ne[1] + 1) * (ne[2] + 1) // 2048) + 2
+    assert tiles * (ne[0] + 1) > sets
+    tps, s = make_pair(pv, ne, seed=7)
+    f = tps.buildLoadVector()
+    u = tps.multigridSolver(2).preconditionedConjugateGradient(np.zeros_like(f), f, 200, 1e-8)
+    ref, _ = orc.MG(s, 2).pcg(np.zeros_like(f), f, 200, 1e-8)
+    assert rel(u, ref) < 1e-10
+
+
 def test_pcg_fp32_preconditioner(pv):
     ne = (64, 32, 32)
     tps, s = make_pair(pv, ne)

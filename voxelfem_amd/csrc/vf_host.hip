@@ -854,7 +854,7 @@ struct vf_mg {
 
     // Ad = K d on the fine level (Dirichlet rows zero) and *dAd = <d, Ad> over the active nodes, fused into
     // the Walsh-basis product when that family is in use
-    void apply_dot(const double *d, double *Ad, double *partials, double *dAd);
+    void apply_dot(const double *d, double *Ad, double *partials, size_t npart, double *dAd);
     template <typename T>
     void apply(int l, const T *u, T *y, const T *b, int mode, bool useMask) {
         const uint8_t *mask = useMask ? dm(l) : nullptr;
@@ -1488,7 +1488,10 @@ struct vf_mg {
         pr.resize(n0); ps.resize(n0); pd.resize(n0); pAd.resize(n0);
         double *r = pr.data(), *sv = ps.data(), *d = pd.data(), *Ad = pAd.data();
         double *sc = sim->scalars();
-        double *part = sim->red_partials(2 * (size_t)reduction_partials(g) + 2);
+        // the vector reductions write up to two sets of partials, the fused <d, K d> one per workgroup of the product
+        // (more than both sets on small grids: 585 against 392 on 64x32x32)
+        const size_t npart = std::max(2 * (size_t)reduction_partials(g) + 2, walsh_partials(g));
+        double *part = sim->red_partials(npart);
         std::vector<double> hx, hr;
         auto callback = [&](int64_t it) {
             if (!cb) return;
@@ -1567,7 +1570,7 @@ struct vf_mg {
                     launch_pcg_direction_x<double>(g, sv, d, x, sc, flexible ? 1 : 0, firstIt ? 1 : 0, s);
                 }
                 if (timeKd) VF_HIP(hipEventRecord(kdEv[0], s));
-                apply_dot(d, Ad, part, sc + 3);
+                apply_dot(d, Ad, part, npart, sc + 3);
                 if (timeKd) VF_HIP(hipEventRecord(kdEv[1], s));
                 launch_pcg_scalars(sc, 1, s);  // alpha of this iteration
                 launch_pcg_residual(g, r, Ad, sc, part, sc + 4, r32, s);
@@ -1686,10 +1689,10 @@ template <> const float *vf_mg::blocksp<float>(int l) const {
 }
 template <> DBuf<double> &vf_mg::block_buf<double>(int l) { return lv[l]->blocks; }
 template <> DBuf<float> &vf_mg::block_buf<float>(int l) { return lv[l]->blocks32; }
-void vf_mg::apply_dot(const double *d, double *Ad, double *partials, double *dAd) {
+void vf_mg::apply_dot(const double *d, double *Ad, double *partials, size_t npart, double *dAd) {
     if (ku_family<double>() == 2) {
         launch_fine_apply_walsh<double>(lv[0]->g, Wp<double>(), Ep<double>(), d, Ad, nullptr, dm(0), AM_SET, st(),
-                                        partials, dAd);
+                                        partials, dAd, 0, npart);
     } else {
         apply<double>(0, d, Ad, nullptr, AM_SET, true);
         launch_dot_active(lv[0]->g, d, Ad, partials, dAd, st());
@@ -3371,7 +3374,7 @@ static void lbl_stacked_batch(vf_mg *base, std::vector<std::shared_ptr<StackedBa
                                            s);
         }
         launch_fine_apply_walsh<double>(g, S->Wtab.data(), S->E.data(), d, Ad, nullptr, m.dm(0), AM_SET, s, part.data(),
-                                        xx.data(), P);
+                                        xx.data(), P, part.size());
         launch_seg_sum_chunks(part.data(), tiles, xc, nch, P, nseg, sc.data(), 3, s);
         launch_seg_scalars(sc.data(), dstate.data(), nseg, 1, s);
         launch_seg_residual(g, r, Ad, sc.data(), dstate.data(), P, nseg, part.data(), r32, s);

@@ -138,14 +138,17 @@ int resident_workgroups(const void *kernel, int threads);
 int plane_chunks(int tiles, int n, int want, int resident);
 // Element-centric fine K u in the Walsh basis (AM_SET or AM_RESIDUAL); C = the 8 x 16 table of the
 // nonzero Walsh-basis element stiffness entries divided by 64 (see vf_kernels_walsh.hip).
-// With dotOut (SET mode only), *dotOut = <u, y> is also formed from per-workgroup partials (dotPartials
-// needs one entry per workgroup, at most tiles x nn[0]); the partials are stored chunk-major (entry
+// With dotOut (SET mode only), *dotOut = <u, y> is also formed from per-workgroup partials (dotPartials holds
+// dotCapacity entries, one per workgroup needed, at most walsh_partials(g); the launch throws if they do not fit);
+// the partials are stored chunk-major (entry
 // chunk * tiles + tile, tiles = ceil(ydet / 15) * ceil(nn[2] / 15), chunk c owning node planes
 // [c xchunk, (c + 1) xchunk)). alignX > 0: xchunk divides alignX.
 template <typename T>
 void launch_fine_apply_walsh(const Grid &g, const T *C, const T *E, const T *u, T *y, const T *b,
                              const uint8_t *dmask, int mode, hipStream_t s, double *dotPartials = nullptr,
-                             double *dotOut = nullptr, int alignX = 0);
+                             double *dotOut = nullptr, int alignX = 0, size_t dotCapacity = 0);
+// most partial sums of <u, K u> that launch on g writes (one x-plane per chunk)
+size_t walsh_partials(const Grid &g);
 // x-chunk length the Walsh K u uses on g with alignX (as above)
 int walsh_xchunk(const Grid &g, int mode, int alignX);
 // fixed-order sum of count partials into *out

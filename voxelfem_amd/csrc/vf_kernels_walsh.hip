@@ -296,10 +296,12 @@ int walsh_xchunk(const Grid &g, int mode, int alignX) {
     return walsh_xchunk_of(g, kern, alignX);
 }
 
+size_t walsh_partials(const Grid &g) { return (size_t)cdiv(g.ydet, TN) * cdiv(g.nn[2], TN) * g.nn[0]; }
+
 template <typename T>
 void launch_fine_apply_walsh(const Grid &g, const T *C, const T *E, const T *u, T *y, const T *b,
                              const uint8_t *dmask, int mode, hipStream_t s, double *dotPartials, double *dotOut,
-                             int alignX) {
+                             int alignX, size_t dotCapacity) {
     if (mode != AM_SET && mode != AM_RESIDUAL) throw std::runtime_error("Walsh K u supports the SET and RESIDUAL modes");
     if (dotOut && (mode != AM_SET || !dotPartials)) throw std::runtime_error("the fused <u, K u> needs SET mode and partials");
     if (dotOut && g.ydet <= 0) launch_fill<double>(1, dotOut, 0.0, s);
@@ -311,6 +313,9 @@ void launch_fine_apply_walsh(const Grid &g, const T *C, const T *E, const T *u, 
         const int xchunk = walsh_xchunk_of(g, kern, alignX);
         const int chunks = cdiv(g.nn[0], xchunk);
         if (chunks > 65535) throw std::runtime_error("grid too large for the Walsh K u");
+        if (dotOut && (size_t)tiles * chunks > dotCapacity)
+            throw std::runtime_error("Walsh K u: " + std::to_string((size_t)tiles * chunks) +
+                                     " partial sums do not fit the buffer of " + std::to_string(dotCapacity));
         const dim3 grid(tiles, chunks);
         if (mode == AM_RESIDUAL)
             hipLaunchKernelGGL((k_ku_walsh<T, AM_RESIDUAL>), grid, dim3(NTW), 0, s, g, C, E, u, y, b, dmask, ntZ, xchunk,
@@ -329,8 +334,9 @@ void launch_fine_apply_walsh(const Grid &g, const T *C, const T *E, const T *u, 
 
 template void launch_fine_apply_walsh<double>(const Grid &, const double *, const double *, const double *, double *,
                                               const double *, const uint8_t *, int, hipStream_t, double *, double *,
-                                              int);
+                                              int, size_t);
 template void launch_fine_apply_walsh<float>(const Grid &, const float *, const float *, const float *, float *,
-                                             const float *, const uint8_t *, int, hipStream_t, double *, double *, int);
+                                             const float *, const uint8_t *, int, hipStream_t, double *, double *, int,
+                                             size_t);
 
 }  // namespace vf
