@@ -1,0 +1,57 @@
+"""GPU tests of the coarse-level kernels at the sizes where their work split can go wrong, against the oracle.
+
+Tolerances: a level's rows are sums of 81 products in FP64, so two orders of the sum agree to a few 1e-15 of the
+row's largest term; 1e-12 (products) and 1e-11 (after a sweep's 3 x 3 solves) leave room for the cancellation in
+the rows, as in test_gpu_parity."""
+import numpy as np
+import pytest
+
+from oracle import oracle as orc
+from voxelfem_amd import workloads as wl
+
+pytestmark = pytest.mark.gpu
+
+
+def rel(a, b):
+    return np.abs(np.asarray(a) - np.asarray(b)).max() / max(np.abs(np.asarray(b)).max(), 1e-300)
+
+
+def pair(ne, levels, layer=None, seed=0):
+    """A solver and the oracle's on the same cantilever."""
+    import voxelfem_amd
+
+    rho = wl.noise_density(ne, seed)
+    tps = wl.configure(voxelfem_amd.pyVoxelFEM, ne, wl.CANTILEVER_BC, rho)
+    mg = tps.multigridSolver(levels)
+    s = orc.Sim(ne)
+    s.set_etensor(1.0, 0.3)
+    s.set_law(0, 1.0, 1e-9, 3.0, 3.0)
+    s.set_densities(rho)
+    s.set_dirichlet(wl.cantilever_mask(ne))
+    om = orc.MG(s, levels)
+    if layer is not None:
+        mg.setFabricationMaskHeightByLayer(layer)
+        om.set_mask_layer(layer)
+    mg.updateStiffnessMatrices()
+    om.update_stiffness()
+    return mg, om
+
+
+# level 1 has (ne / 2 + 1) nodes per axis: colour classes of 1 to 45 nodes, with every remainder modulo the four nodes
+# that the block rows interleave and the sixteen that a workgroup holds; with layers masked, rows end inside a class
+@pytest.mark.parametrize("ne,levels,layer", [((4, 4, 4), 2, None), ((8, 4, 4), 2, None), ((8, 12, 4), 2, None),
+                                             ((16, 8, 12), 2, None), ((4, 12, 20), 2, 5), ((16, 16, 8), 3, 9)])
+def test_block_rows(ne, levels, layer):
+    mg, om = pair(ne, levels, layer)
+    rng = np.random.default_rng(5)
+    for l in range(1, levels):
+        nn = om.num_nodes(l)
+        u, b = rng.normal(size=(nn, 3)), rng.normal(size=(nn, 3))
+        ny = (ne[1] >> l) + 1
+        iy = (np.arange(nn) // ((ne[2] >> l) + 1)) % ny
+        act = np.ones(nn, bool) if layer is None else iy < -(-layer >> l) + 1
+        u[~act] = 0
+        assert rel(mg.applyK(l, u)[act], om.apply_K(l, u)[act]) < 1e-12, l
+        assert rel(mg.computeResidual(l, u, b)[act], om.residual(l, u, b)[act]) < 1e-12, l
+        for fwd in (True, False):
+            assert rel(mg._smooth(l, u, b, fwd)[act], om.smooth(l, u, b, fwd)[act]) < 1e-11, (l, fwd)

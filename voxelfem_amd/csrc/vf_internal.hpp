@@ -93,31 +93,28 @@ struct DBuf {
 // ---------------------------------------------------------------------------------------------
 enum ApplyMode { AM_SET = 0, AM_ADD = 1, AM_SUB = 2, AM_RESIDUAL = 3 };
 
-// Assembled block rows (levels 2..L-1) are stored colour-major: the nodes of colour
+// Assembled block rows (levels 1..L-1) are stored colour-major: the nodes of colour
 // c = 4(ix%2) + 2(iy%2) + (iz%2) form a class of cnt_c nodes numbered j = ((ix/2) my + iy/2) mz + iz/2
-// (m_ = nodes of that parity along each axis), classes follow each other in colour order, and inside a
-// class entry k of neighbour slot s sits at (s*9 + k) * cnt_c + j. A smoothing pass over one colour then
-// streams contiguous memory.
-struct BlockSlot {
-    size_t base;  // first entry of the node's colour class
-    int cnt;      // nodes in the class
-    int j;        // node index inside the class
-};
-__host__ __device__ inline BlockSlot block_slot(const Grid &g, int ix, int iy, int iz) {
-    const int cx = ix & 1, cy = iy & 1, cz = iz & 1;
-    const int c = 4 * cx + 2 * cy + cz;
+// (m_ = nodes of that parity along each axis) and classes follow each other in colour order, each padded to a
+// multiple of BLOCK_GROUP nodes. Inside a class the rows of four consecutive nodes are interleaved: entry k = 3 a + c
+// of neighbour slot s of node j sits at ((j / 4 * 9 + k) * 27 + s) * 4 + j % 4. A wavefront that gives each of four
+// nodes sixteen lanes, one per neighbour slot, so reads contiguous memory, and a pass over one colour streams it.
+constexpr int BLOCK_GROUP = 4;
+__host__ __device__ inline size_t block_class_nodes(const Grid &g, int c) {  // padded node count of a class
+    const size_t mx = (g.nn[0] - ((c >> 2) & 1) + 1) / 2, my = (g.nn[1] - ((c >> 1) & 1) + 1) / 2,
+                 mz = (g.nn[2] - (c & 1) + 1) / 2;
+    return (mx * my * mz + BLOCK_GROUP - 1) / BLOCK_GROUP * BLOCK_GROUP;
+}
+__host__ __device__ inline size_t block_class_base(const Grid &g, int c) {  // padded nodes of the classes before c
     size_t before = 0;
-    for (int q = 0; q < c; ++q) {
-        const long mx = (g.nn[0] - ((q >> 2) & 1) + 1) / 2, my = (g.nn[1] - ((q >> 1) & 1) + 1) / 2,
-                   mz = (g.nn[2] - (q & 1) + 1) / 2;
-        before += (size_t)(mx * my * mz);
-    }
-    const int my = (g.nn[1] - cy + 1) / 2, mz = (g.nn[2] - cz + 1) / 2, mx = (g.nn[0] - cx + 1) / 2;
-    BlockSlot r;
-    r.base = before * 243;
-    r.cnt = mx * my * mz;
-    r.j = ((ix >> 1) * my + (iy >> 1)) * mz + (iz >> 1);
-    return r;
+    for (int q = 0; q < c; ++q) before += block_class_nodes(g, q);
+    return before;
+}
+inline size_t block_storage(const Grid &g) { return block_class_base(g, 8) * 243; }  // values of a whole level
+// offset of entry 0 of slot 0 of node j inside a level whose class starts at padded node `base`; entry k of slot s
+// is (k * 27 + s) * BLOCK_GROUP further on
+__host__ __device__ inline size_t block_offset(size_t base, int j) {
+    return (base + (size_t)(j / BLOCK_GROUP) * BLOCK_GROUP) * 243 + j % BLOCK_GROUP;
 }
 
 // fine level (TPSStencils.hh:431-728).  AM_SET: y = K u (detached rows zeroed);
@@ -179,7 +176,7 @@ void launch_l1_gs_mfma(const Grid &gc, const Grid &gf, const T *Chat, const T *E
 // zero the rows of y at and above the first detached row (ydet)
 template <typename T>
 void launch_zero_detached(const Grid &g, T *y, hipStream_t s);
-// assembled 27-point block rows (levels >= 2)
+// assembled 27-point block rows (levels >= 1)
 template <typename T>
 void launch_block_apply(const Grid &g, const T *blocks, const T *u, T *y, const T *b, const uint8_t *dmask, int mode,
                         hipStream_t s);

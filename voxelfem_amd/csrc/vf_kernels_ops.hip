@@ -516,206 +516,118 @@ __global__ void __launch_bounds__(TPB) k_l1_gs_r2(Grid gc, Grid gf, const T *__r
 }
 
 // ------------------------------------------------------------------ assembled block rows
-// Colour-major block storage (see BlockSlot). The neighbours are visited GROUP at a time with the
-// accumulators pinned after each group, which bounds how many of the 243 block entries and 81 u values
-// the compiler keeps in flight (and so the register count) while still overlapping memory latency.
-// Large levels use groups of 3 (occupancy); small levels, whose launches are latency-bound, groups of 9
-// (three dependent memory rounds per row instead of nine).
-template <typename T, bool WANT_M, int GROUP = 3>
-__device__ __forceinline__ void block_row(const Grid &g, const T *__restrict__ blocks, const BlockSlot &bs, int ix,
-                                          int iy, int iz, const T *__restrict__ u, T f[3], T M[9]) {
-    const int N = g.nnodes, sx = g.nn[1] * g.nn[2], sy = g.nn[2];
-    const int n = (ix * g.nn[1] + iy) * g.nn[2] + iz;
-    const T *__restrict__ bp = blocks + bs.base + bs.j;
-    const size_t st = (size_t)bs.cnt;
+// One node is worked on by the sixteen lanes of one DPP row: lane p holds neighbour slots p and p + 16 (27 in all), so
+// a node's 243 block entries and 81 neighbour values are requested at once, in one round of loads, and the row is
+// summed by four DPP exchanges without LDS. A colour pass over a small level is bound by that one memory round
+// instead of the three dependent rounds (and 81 loads per work-item) of four work-items per node; over a large level
+// it streams the interleaved rows (105 x 57 x 49 nodes in FP64: 20 us per colour, 3.6 TB/s). Time per colour, before
+// and after, averaged over the block levels of a hierarchy: 64 x 32 x 32 FP64 10.4 -> 4.3 us, 176 x 88 x 72 FP64
+// 13.6 -> 7.5 us, 208 x 112 x 96 FP64 16.2 -> 9.9 us, 384 x 192 x 192 FP32 9.5 -> 7.6 us.
+template <int CTRL>
+__device__ __forceinline__ float dpp_get(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_get(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+// sum over the sixteen lanes of a DPP row, the same in every lane
+template <typename T>
+__device__ __forceinline__ T row16_sum(T v) {
+    v += dpp_get<0xB1>(v);   // quad_perm [1, 0, 3, 2]
+    v += dpp_get<0x4E>(v);   // quad_perm [2, 3, 0, 1]
+    v += dpp_get<0x141>(v);  // row_half_mirror
+    v += dpp_get<0x140>(v);  // row_mirror
+    return v;
+}
+
+constexpr int RL = 16;       // lanes per node
+constexpr int RN16 = TPB / RL;  // nodes per workgroup
+constexpr int DIAG_LANE = 13;   // the lane that holds the node's own slot
+
+// this lane's part of row f = sum_s B_s u_s of the node (ix, iy, iz) whose rows start at bp; M: the entries of slot p
+template <typename T>
+__device__ __forceinline__ void block_row16(const Grid &g, const T *__restrict__ bp, int p, int ix, int iy, int iz,
+                                            const T *__restrict__ u, T f[3], T M[9]) {
+    const int N = g.nnodes, sy = g.nn[2], sx = g.nn[1] * sy;
+    const int n = ix * sx + iy * sy + iz;
+    T B[2][9], un[2][3];
 #pragma unroll
-    for (int s = 0; s < 27; ++s) {
-        const int dx = s / 9 - 1, dy = (s / 3) % 3 - 1, dz = s % 3 - 1;
-        const bool ok = (unsigned)(ix + dx) < (unsigned)g.nn[0] && (unsigned)(iy + dy) < (unsigned)g.nn[1] &&
+    for (int h = 0; h < 2; ++h) {
+        const bool real = p + RL * h < 27;
+        const int s = real ? p + RL * h : 26;  // the idle lanes of the second half repeat slot 26 with u = 0
+        const int q = (s * 171) >> 9;          // s / 3
+        const int dx = ((s * 57) >> 9) - 1, dy = q - 3 * (dx + 1) - 1, dz = s - 3 * q - 1;
+        const bool ok = real && (unsigned)(ix + dx) < (unsigned)g.nn[0] && (unsigned)(iy + dy) < (unsigned)g.nn[1] &&
                         (unsigned)(iz + dz) < (unsigned)g.nn[2];
-        const int m = n + dx * sx + dy * sy + dz;
-        T un[3];
+        const int m = ok ? n + dx * sx + dy * sy + dz : n;
 #pragma unroll
-        for (int c = 0; c < 3; ++c) un[c] = ok ? u[(size_t)c * N + m] : T(0);
+        for (int k = 0; k < 9; ++k) B[h][k] = bp[(k * 27 + s) * BLOCK_GROUP];
 #pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            T acc = 0;
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-                const T B = bp[(size_t)(s * 9 + 3 * a + c) * st];
-                acc += B * un[c];
-                if (WANT_M && s == 13) M[3 * a + c] = B;
-            }
-            f[a] += acc;
-        }
-        if (s % GROUP == GROUP - 1) {
-            asm volatile("" : "+v"(f[0]), "+v"(f[1]), "+v"(f[2]));
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    }
-}
-
-template <typename T, int MODE, int GROUP>
-__device__ __forceinline__ void block_apply_row(const Grid &g, const T *__restrict__ blocks, const T *__restrict__ u,
-                                                T *__restrict__ y, const T *__restrict__ b,
-                                                const uint8_t *__restrict__ dmask) {
-    const int nz = g.nn[2], slab = g.ydet * nz;
-    const int t = blockIdx.x * TPB + threadIdx.x;
-    if (t >= g.nn[0] * slab) return;
-    const int ix = t / slab, r = t - ix * slab, iy = r / nz, iz = r - iy * nz;
-    const int n = (ix * g.nn[1] + iy) * nz + iz;
-    const BlockSlot bs = block_slot(g, ix, iy, iz);
-    T f[3] = {0, 0, 0};
-    T M[9];
-    block_row<T, false, GROUP>(g, blocks, bs, ix, iy, iz, u, f, M);
-    store_out(y, b, g.nnodes, n, f, MODE, dmask ? dmask[n] : uint8_t(0));
-}
-
-// Block-row product on a small level with four work-items per node (see k_block_gs_x4); work-item 0
-// writes the row.
-template <typename T, int MODE>
-__global__ void __launch_bounds__(TPB) k_block_apply_x4(Grid g, const T *__restrict__ blocks, const T *__restrict__ u,
-                                                        T *__restrict__ y, const T *__restrict__ b,
-                                                        const uint8_t *__restrict__ dmask) {
-    const int nz = g.nn[2], slab = g.ydet * nz;
-    const int t = blockIdx.x * TPB + threadIdx.x;
-    const int node = t >> 2, part = t & 3;
-    const bool valid = node < g.nn[0] * slab;
-    const int ix = valid ? node / slab : 0, r = valid ? node - ix * slab : 0, iy = r / nz, iz = r - iy * nz;
-    const int N = g.nnodes, n = (ix * g.nn[1] + iy) * nz + iz;
-    T f[3] = {0, 0, 0};
-    if (valid && part < 3) {
-        const BlockSlot bs = block_slot(g, ix, iy, iz);
-        const T *__restrict__ bp = blocks + bs.base + bs.j;
-        const size_t st = (size_t)bs.cnt;
-        const int sx = g.nn[1] * nz;
-        const int dx = part - 1;
-        const bool okx = (unsigned)(ix + dx) < (unsigned)g.nn[0];
-#pragma unroll
-        for (int q = 0; q < 9; ++q) {
-            const int s = 9 * part + q, dy = q / 3 - 1, dz = q % 3 - 1;
-            const bool ok = okx && (unsigned)(iy + dy) < (unsigned)g.nn[1] && (unsigned)(iz + dz) < (unsigned)nz;
-            const int m = n + dx * sx + dy * nz + dz;
-            T un[3];
-#pragma unroll
-            for (int c = 0; c < 3; ++c) un[c] = ok ? u[(size_t)c * N + m] : T(0);
-#pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                T acc = 0;
-#pragma unroll
-                for (int c = 0; c < 3; ++c) acc += bp[(size_t)(s * 9 + 3 * a + c) * st] * un[c];
-                f[a] += acc;
-            }
+        for (int c = 0; c < 3; ++c) {
+            const T v = u[(size_t)c * N + m];
+            un[h][c] = ok ? v : T(0);
         }
     }
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        f[c] += __shfl_xor(f[c], 1, 64);
-        f[c] += __shfl_xor(f[c], 2, 64);
+    for (int a = 0; a < 3; ++a) {
+        T acc = B[0][3 * a] * un[0][0];
+        acc += B[0][3 * a + 1] * un[0][1];
+        acc += B[0][3 * a + 2] * un[0][2];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) acc += B[1][3 * a + c] * un[1][c];
+        f[a] = row16_sum(acc);
     }
-    if (valid && part == 0) store_out(y, b, N, n, f, MODE, dmask ? dmask[n] : uint8_t(0));
+#pragma unroll
+    for (int k = 0; k < 9; ++k) M[k] = B[0][k];
 }
 
-template <typename T, int MODE>
-__global__ void __launch_bounds__(TPB) k_block_apply_g9(Grid g, const T *__restrict__ blocks, const T *__restrict__ u,
-                                                        T *__restrict__ y, const T *__restrict__ b,
-                                                        const uint8_t *__restrict__ dmask) {
-    block_apply_row<T, MODE, 9>(g, blocks, u, y, b, dmask);
-}
-
+// grid.y = colour class (the rows are stored by class)
 template <typename T, int MODE>
 __global__ void __launch_bounds__(TPB) k_block_apply(Grid g, const T *__restrict__ blocks, const T *__restrict__ u,
                                                      T *__restrict__ y, const T *__restrict__ b,
                                                      const uint8_t *__restrict__ dmask) {
-    const int nz = g.nn[2], slab = g.ydet * nz;
-    const int t = blockIdx.x * TPB + threadIdx.x;
-    if (t >= g.nn[0] * slab) return;
-    const int ix = t / slab, r = t - ix * slab, iy = r / nz, iz = r - iy * nz;
-    const int n = (ix * g.nn[1] + iy) * nz + iz;
-    const BlockSlot bs = block_slot(g, ix, iy, iz);
-    T f[3] = {0, 0, 0};
-    T M[9];
-    block_row<T, false>(g, blocks, bs, ix, iy, iz, u, f, M);
-    store_out(y, b, g.nnodes, n, f, MODE, dmask ? dmask[n] : uint8_t(0));
+    const int col = blockIdx.y, cx = (col >> 2) & 1, cy = (col >> 1) & 1, cz = col & 1;
+    const int mx = (g.nn[0] - cx + 1) / 2, my = (g.ydet - cy + 1) / 2, mz = (g.nn[2] - cz + 1) / 2;
+    const int node = blockIdx.x * RN16 + threadIdx.x / RL, p = threadIdx.x % RL;
+    if (node >= mx * my * mz) return;
+    const int jx = node / (my * mz), r = node - jx * my * mz, jy = r / mz, jz = r - jy * mz;
+    const int ix = 2 * jx + cx, iy = 2 * jy + cy, iz = 2 * jz + cz;
+    const int n = (ix * g.nn[1] + iy) * g.nn[2] + iz;
+    const int j = (jx * ((g.nn[1] - cy + 1) / 2) + jy) * mz + jz;
+    T f[3], M[9];
+    block_row16<T>(g, blocks + block_offset(block_class_base(g, col), j), p, ix, iy, iz, u, f, M);
+    if (p == DIAG_LANE) store_out(y, b, g.nnodes, n, f, MODE, dmask ? dmask[n] : uint8_t(0));
 }
 
-// One colour of the block Gauss-Seidel sweep on a small level, four work-items per node: work-item
-// g < 3 of a node gathers the nine block rows of neighbour plane x + g - 1, the partial rows are summed
-// across the four with two lane exchanges, and work-item 1 (which holds the diagonal block) updates the
-// node. The per-node dependency chain is a third of the one-work-item form, which bounds these
-// latency-limited launches.
+// One colour of the block Gauss-Seidel sweep; lane 13 of a node's sixteen, which holds the diagonal block, updates it.
 template <typename T>
-__global__ void __launch_bounds__(TPB) k_block_gs_x4(Grid g, const T *__restrict__ blocks, T *__restrict__ u,
-                                                     const T *__restrict__ b, const uint8_t *__restrict__ dmask,
-                                                     int cx, int cy, int cz, int forward) {
+__global__ void __launch_bounds__(TPB) k_block_gs(Grid g, const T *__restrict__ blocks, T *__restrict__ u,
+                                                  const T *__restrict__ b, const uint8_t *__restrict__ dmask,
+                                                  size_t base, int cx, int cy, int cz, int forward) {
     const int mx = (g.nn[0] - cx + 1) / 2, my = (g.ydet - cy + 1) / 2, mz = (g.nn[2] - cz + 1) / 2;
-    const int t = blockIdx.x * TPB + threadIdx.x;
-    const int node = t >> 2, part = t & 3;
-    const bool valid = node < mx * my * mz;
-    const int jx = valid ? node / (my * mz) : 0, r = valid ? node - jx * my * mz : 0, jy = r / mz, jz = r - jy * mz;
+    const int node = blockIdx.x * RN16 + threadIdx.x / RL, p = threadIdx.x % RL;
+    if (node >= mx * my * mz) return;
+    const int jx = node / (my * mz), r = node - jx * my * mz, jy = r / mz, jz = r - jy * mz;
     const int ix = 2 * jx + cx, iy = 2 * jy + cy, iz = 2 * jz + cz;
     const int N = g.nnodes, n = (ix * g.nn[1] + iy) * g.nn[2] + iz;
-    const uint8_t dm = valid ? (dmask ? dmask[n] : uint8_t(0)) : uint8_t(7);
-    T f[3] = {0, 0, 0};
-    T M[9];
-    if (dm != 7 && part < 3) {
-        const BlockSlot bs = block_slot(g, ix, iy, iz);
-        const T *__restrict__ bp = blocks + bs.base + bs.j;
-        const size_t st = (size_t)bs.cnt;
-        const int sx = g.nn[1] * g.nn[2], sy = g.nn[2];
-        const int dx = part - 1;
-        const bool okx = (unsigned)(ix + dx) < (unsigned)g.nn[0];
+    const int j = (jx * ((g.nn[1] - cy + 1) / 2) + jy) * mz + jz;
+    // requested with the row, so that the update waits for no second round
+    uint8_t dm = 0;
+    T bn[3] = {0, 0, 0};
+    if (p == DIAG_LANE) {
+        if (dmask) dm = dmask[n];
 #pragma unroll
-        for (int q = 0; q < 9; ++q) {
-            const int s = 9 * part + q, dy = q / 3 - 1, dz = q % 3 - 1;
-            const bool ok = okx && (unsigned)(iy + dy) < (unsigned)g.nn[1] && (unsigned)(iz + dz) < (unsigned)g.nn[2];
-            const int m = n + dx * sx + dy * sy + dz;
-            T un[3];
-#pragma unroll
-            for (int c = 0; c < 3; ++c) un[c] = ok ? u[(size_t)c * N + m] : T(0);
-#pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                T acc = 0;
-#pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    const T B = bp[(size_t)(s * 9 + 3 * a + c) * st];
-                    acc += B * un[c];
-                    if (q == 4) M[3 * a + c] = B;  // slot 13 (the node itself) when part == 1
-                }
-                f[a] += acc;
-            }
-        }
+        for (int c = 0; c < 3; ++c) bn[c] = b[(size_t)c * N + n];
     }
-    // every lane takes part in the exchanges (idle ones contribute zeros)
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        f[c] += __shfl_xor(f[c], 1, 64);
-        f[c] += __shfl_xor(f[c], 2, 64);
-    }
-    if (dm != 7 && part == 1) {
-        const T bms[3] = {b[n] - f[0], b[N + n] - f[1], b[2 * N + n] - f[2]};
+    T f[3], M[9];
+    block_row16<T>(g, blocks + block_offset(base, j), p, ix, iy, iz, u, f, M);
+    if (p == DIAG_LANE && dm != 7) {
+        const T bms[3] = {bn[0] - f[0], bn[1] - f[1], bn[2] - f[2]};
         gs_update(u, N, n, bms, M, dm, forward);
     }
-}
-
-template <typename T, int GROUP = 3>
-__global__ void __launch_bounds__(TPB) k_block_gs(Grid g, const T *__restrict__ blocks, T *__restrict__ u,
-                                                  const T *__restrict__ b, const uint8_t *__restrict__ dmask, int cx,
-                                                  int cy, int cz, int forward) {
-    const int mx = (g.nn[0] - cx + 1) / 2, my = (g.ydet - cy + 1) / 2, mz = (g.nn[2] - cz + 1) / 2;
-    const int t = blockIdx.x * TPB + threadIdx.x;
-    if (t >= mx * my * mz) return;
-    const int jx = t / (my * mz), r = t - jx * my * mz, jy = r / mz, jz = r - jy * mz;
-    const int ix = 2 * jx + cx, iy = 2 * jy + cy, iz = 2 * jz + cz;
-    const int N = g.nnodes, n = (ix * g.nn[1] + iy) * g.nn[2] + iz;
-    const uint8_t dm = dmask ? dmask[n] : uint8_t(0);
-    if (dm == 7) return;
-    const BlockSlot bs = block_slot(g, ix, iy, iz);
-    T f[3] = {0, 0, 0};
-    T M[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    block_row<T, true, GROUP>(g, blocks, bs, ix, iy, iz, u, f, M);
-    const T bms[3] = {b[n] - f[0], b[N + n] - f[1], b[2 * N + n] - f[2]};
-    gs_update(u, N, n, bms, M, dm, forward);
 }
 
 // ------------------------------------------------------------------ cached element matrices
@@ -907,23 +819,12 @@ void launch_l1_apply(const Grid &gc, const Grid &gf, const T *Chat, const T *Cw,
     VF_HIP(hipGetLastError());
 }
 
-// levels below this many nodes use the latency-oriented grouping of block_row
-constexpr int SMALL_LEVEL = 65536;
-// levels below this many nodes smooth with four work-items per node (latency-bound launches); up to
-// GS_G9_LEVEL nodes, one work-item per node with nine block rows requested at a time
-constexpr int GS_X4_LEVEL = 1 << 19, GS_G9_LEVEL = 1 << 22;
-
 template <typename T>
 void launch_block_apply(const Grid &g, const T *blocks, const T *u, T *y, const T *b, const uint8_t *dmask, int mode,
                         hipStream_t s) {
-    const long count = (long)g.nn[0] * g.ydet * g.nn[2];
-    if (count > 0 && g.nnodes < GS_X4_LEVEL) {
-        VF_DISPATCH_MODE(k_block_apply_x4, T, mode, dim3(nblocks(4 * count)), g, blocks, u, y, b, dmask);
-    } else if (count > 0 && g.nnodes < SMALL_LEVEL) {
-        VF_DISPATCH_MODE(k_block_apply_g9, T, mode, dim3(nblocks(count)), g, blocks, u, y, b, dmask);
-    } else if (count > 0) {
-        VF_DISPATCH_MODE(k_block_apply, T, mode, dim3(nblocks(count)), g, blocks, u, y, b, dmask);
-    }
+    const long most = (long)((g.nn[0] + 1) / 2) * ((g.ydet + 1) / 2) * ((g.nn[2] + 1) / 2);
+    if (most > 0)
+        VF_DISPATCH_MODE(k_block_apply, T, mode, dim3((unsigned)((most + RN16 - 1) / RN16), 8), g, blocks, u, y, b, dmask);
     if (mode == AM_SET && g.ydet < g.nn[1]) {
         const long cz = (long)g.nn[0] * (g.nn[1] - g.ydet) * g.nn[2];
         hipLaunchKernelGGL(k_zero_detached<T>, dim3(nblocks(cz)), dim3(TPB), 0, s, g, y);
@@ -976,15 +877,8 @@ void launch_block_gs(const Grid &g, const T *blocks, T *u, const T *b, const uin
     const int cx = (color >> 2) & 1, cy = (color >> 1) & 1, cz = color & 1;
     const long count = color_count(g, cx, cy, cz);
     if (!count) return;
-    if (g.nnodes < GS_X4_LEVEL)
-        hipLaunchKernelGGL(k_block_gs_x4<T>, dim3(nblocks(4 * count)), dim3(TPB), 0, s, g, blocks, u, b, dmask, cx, cy,
-                           cz, forward);
-    else if (g.nnodes < GS_G9_LEVEL)
-        hipLaunchKernelGGL((k_block_gs<T, 9>), dim3(nblocks(count)), dim3(TPB), 0, s, g, blocks, u, b, dmask, cx, cy, cz,
-                           forward);
-    else
-        hipLaunchKernelGGL((k_block_gs<T, 3>), dim3(nblocks(count)), dim3(TPB), 0, s, g, blocks, u, b, dmask, cx, cy, cz,
-                           forward);
+    hipLaunchKernelGGL(k_block_gs<T>, dim3((unsigned)((count + RN16 - 1) / RN16)), dim3(TPB), 0, s, g, blocks, u, b, dmask,
+                       block_class_base(g, color), cx, cy, cz, forward);
     VF_HIP(hipGetLastError());
 }
 

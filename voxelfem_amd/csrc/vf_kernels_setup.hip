@@ -133,28 +133,22 @@ __global__ void __launch_bounds__(576) k_galerkin_recurse(Grid gc, Grid gf, cons
 // lm = 4 (i + ox) + 2 (jj + oy) + (k + oz). The 27 slots split into three groups of nine by ox; in group ox
 // only the elements with lx = i + ox in {0, 1} contribute, and for one element and one matrix row 3 ln + a
 // the twelve entries 3 lm + c of that group (lx fixed) are contiguous. A work-item holds one group's 81
-// FP64 sums in registers, so every element datum it needs is read once per group, and the colour-major
-// block layout (BlockSlot) makes each slot entry a contiguous run over the class.
+// FP64 sums in registers, so every element datum it needs is read once per group; four neighbouring
+// work-items' rows are interleaved in the block layout (block_offset).
 struct ClassNode {
-    int ix, iy, iz, j, cnt;
-    size_t before;  // nodes of the lower colour classes
+    int ix, iy, iz;
+    size_t at;  // entry 0 of slot 0 of the node's block rows
 };
 __device__ inline bool class_node(const Grid &g, int colour, ClassNode &r) {
     const int cx = (colour >> 2) & 1, cy = (colour >> 1) & 1, cz = colour & 1;
     const int mx = (g.nn[0] - cx + 1) / 2, my = (g.nn[1] - cy + 1) / 2, mz = (g.nn[2] - cz + 1) / 2;
-    r.cnt = mx * my * mz;
-    r.j = blockIdx.x * TPB + threadIdx.x;
-    if (r.j >= r.cnt) return false;
-    const int jx = r.j / (my * mz), q = r.j - jx * my * mz, jy = q / mz, jz = q - jy * mz;
+    const int j = blockIdx.x * TPB + threadIdx.x;
+    if (j >= mx * my * mz) return false;
+    const int jx = j / (my * mz), q = j - jx * my * mz, jy = q / mz, jz = q - jy * mz;
     r.ix = 2 * jx + cx;
     r.iy = 2 * jy + cy;
     r.iz = 2 * jz + cz;
-    r.before = 0;
-    for (int p = 0; p < colour; ++p) {
-        const long px = (g.nn[0] - ((p >> 2) & 1) + 1) / 2, py = (g.nn[1] - ((p >> 1) & 1) + 1) / 2,
-                   pz = (g.nn[2] - (p & 1) + 1) / 2;
-        r.before += (size_t)(px * py * pz);
-    }
+    r.at = block_offset(block_class_base(g, colour), j);
     return true;
 }
 
@@ -166,7 +160,7 @@ __global__ void __launch_bounds__(TPB) k_assemble_blocks(Grid g, const double *_
     ClassNode n;
     if (!class_node(g, blockIdx.y, n)) return;
     if (n.iy < nylo || n.iy > nyhi) return;
-    OutT *out = blocks + n.before * 243 + n.j;
+    OutT *out = blocks + n.at;
     for (int gx = 0; gx < 3; ++gx) {
         const int ox = gx - 1;
         double acc[81];
@@ -207,7 +201,7 @@ __global__ void __launch_bounds__(TPB) k_assemble_blocks(Grid g, const double *_
                 }
         }
 #pragma unroll
-        for (int q = 0; q < 81; ++q) out[(size_t)(gx * 81 + q) * n.cnt] = (OutT)acc[q];
+        for (int q = 0; q < 81; ++q) out[((q % 9) * 27 + gx * 9 + q / 9) * BLOCK_GROUP] = (OutT)acc[q];
     }
 }
 
@@ -231,7 +225,7 @@ __global__ void __launch_bounds__(TPB) k_assemble_l1_blocks(Grid gc, Grid gf, co
     if (n.iy < nylo || n.iy > nyhi) return;
     const int eyEnd = min(gc.ne[1], gc.ymask);
     const int fz = gf.ne[2], fyz = gf.ne[1] * gf.ne[2];
-    OutT *out = blocks + n.before * 243 + n.j;
+    OutT *out = blocks + n.at;
     // slot groups (ox, oy): three slots (oz) of nine entries each, 27 FP64 sums in registers
     for (int gxy = 0; gxy < 9; ++gxy) {
         const int ox = gxy / 3 - 1, oy = gxy % 3 - 1;
@@ -312,7 +306,7 @@ __global__ void __launch_bounds__(TPB) k_assemble_l1_blocks(Grid gc, Grid gf, co
             }
         }
 #pragma unroll
-        for (int q = 0; q < 27; ++q) out[(size_t)(gxy * 27 + q) * n.cnt] = (OutT)acc[q];
+        for (int q = 0; q < 27; ++q) out[((q % 9) * 27 + gxy * 3 + q / 9) * BLOCK_GROUP] = (OutT)acc[q];
     }
 }
 
