@@ -55,3 +55,35 @@ def test_block_rows(ne, levels, layer):
         assert rel(mg.computeResidual(l, u, b)[act], om.residual(l, u, b)[act]) < 1e-12, l
         for fwd in (True, False):
             assert rel(mg._smooth(l, u, b, fwd)[act], om.smooth(l, u, b, fwd)[act]) < 1e-11, (l, fwd)
+
+
+# the marching smoothing filter: tiles of 8 or 16 rows by 64 columns, reaches 1 to 4, sides below the reach (repeated
+# reflection), real radii, constant weights; sums of up to 729 positive terms in another order: 1e-13
+@pytest.mark.parametrize("dims", [(1, 1, 1), (2, 3, 1), (5, 8, 64), (7, 9, 65), (3, 17, 130), (40, 16, 63)])
+@pytest.mark.parametrize("rmin,linear", [(2.0, True), (3.0, True), (4.0, True), (5.0, True), (2.5, True), (3.7, True),
+                                         (3.0, False), (4.0, False), (6.0, True)])
+def test_smoothing_march(dims, rmin, linear):
+    import voxelfem_amd
+
+    pv = voxelfem_amd.pyVoxelFEM
+    x = np.random.default_rng(9).uniform(size=int(np.prod(dims)))
+    sf = pv.SmoothingFilter(1, pv.SmoothingFilter.Type.Linear if linear else pv.SmoothingFilter.Type.Const)
+    sf.setInputDimensions(list(dims))
+    sf.rmin = rmin
+    assert rel(sf.apply(x), orc.smoothing_filter(x, dims, rmin, linear)) < 1e-13
+
+
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_smoothing_march_non_finite(bad):
+    """A value that is not finite reaches the voxels within the kernel and no others."""
+    import voxelfem_amd
+
+    pv = voxelfem_amd.pyVoxelFEM
+    dims = (11, 12, 13)
+    for rmin, linear in ((4.0, True), (3.7, True), (3.0, False)):
+        x = np.random.default_rng(9).uniform(size=int(np.prod(dims)))
+        x[np.ravel_multi_index((5, 6, 6), dims)] = bad
+        sf = pv.SmoothingFilter(1, pv.SmoothingFilter.Type.Linear if linear else pv.SmoothingFilter.Type.Const)
+        sf.setInputDimensions(list(dims))
+        sf.rmin = rmin
+        assert np.array_equal(np.isfinite(sf.apply(x)), np.isfinite(orc.smoothing_filter(x, dims, rmin, linear)))

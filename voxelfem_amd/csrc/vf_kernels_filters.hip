@@ -1,8 +1,9 @@
-// vf_kernels_filters.hip -- the grid-changing and build-direction density filters of
-// TopologyOptimizationFilter.hh: UpsampleFilter (419-525), VertexToCellFilter (527-597) and, on planar grids,
+// vf_kernels_filters.hip -- the density filters of TopologyOptimizationFilter.hh: SmoothingFilter (285-400), the
+// grid-changing and build-direction filters UpsampleFilter (419-525), VertexToCellFilter (527-597) and, on planar grids,
 // LangelaarFilter (600-712). One work-item per output value (or per input value for the adjoints, gathered,
 // so every sum has one writer and a fixed order); grids are C order with the last index fastest.
 #include <cmath>
+#include <type_traits>
 
 #include "vf_internal.hpp"
 
@@ -391,7 +392,170 @@ __global__ void __launch_bounds__(TPB) k_langelaar_out(int nx, int ny, const dou
     out[i] = i % ny == 0 ? lam[i] : lam[i] * lg_dsmin_dx1(vars[i], smax[i]);
 }
 
+// SmoothingFilter on a 3D grid for kernels reaching R <= 4 voxels. The weight w(a, b, c) depends on |a|, |b|, |c| only
+// and is symmetric in b and c, so the tap sum folds: a workgroup owns a (y, z) tile of 64 columns along z and marches
+// along x with each input plane once in LDS; a work-item folds its rows along z, then along y, then over the swap
+// (b, c) <-> (c, b), forms the R + 1 weighted in-plane sums P_|a| of the plane for each of its YB outputs along y and
+// adds P_|a| to the partial sums of the output planes x - a and x + a, which it keeps in registers. For R = 3 that is
+// about 66 FP64 operations and 18 LDS reads per voxel in place of 251 taps, each with its own reflected index and
+// square root. The march re-reads 2 R planes per x-chunk. Bound by FP64 issue and LDS reads: 384 x 192 x 192, R = 3:
+// 4012 -> 85 us (2.7 TB/s of the 16 bytes a voxel needs); two outputs per work-item instead of four: 92 us. The folded
+// order is also the more exact one: 1.2e-16 rms against 4.9e-16 for the sum tap by tap (251 taps, 80-bit reference).
+struct SmoothWeights {
+    double w[75];      // w[a * NC + b (b + 1) / 2 + c], 0 <= c <= b <= R, NC = (R + 1)(R + 2) / 2 (R <= 4)
+    unsigned mask[5];  // bit b (b + 1) / 2 + c of mask[a]: the tap is inside the kernel (w > 0)
+};
+__device__ __forceinline__ int reflect_cell(int i, int n) {
+    while (i < 0 || i >= n) {
+        if (i >= n) i = 2 * n - i - 1;
+        if (i < 0) i = -i - 1;
+    }
+    return i;
+}
+constexpr int ST = 256, STZ = 64;
+// HAT: the support is that of the linear kernel of radius R + 1 (known at compile time); otherwise taps outside the
+// kernel are skipped by the mask (they must not contribute, not even 0 * x, where x is not finite)
+template <int R, int YB, bool HAT>
+__global__ void __launch_bounds__(ST) k_smoothing_march(int d0, int d1, int d2, SmoothWeights sw, double W,
+                                                        const double *__restrict__ in, double *__restrict__ out, int ntZ,
+                                                        int xchunk) {
+    constexpr int TY = ST / STZ * YB, RY = TY + 2 * R, RZ = STZ + 2 * R, PLANE = RY * RZ, NL = (PLANE + ST - 1) / ST;
+    constexpr int NC = (R + 1) * (R + 2) / 2, NR = 2 * R + 1;
+    __shared__ double sp[2][PLANE];
+    const int tiles = gridDim.x;
+    const int logical = xcd_remap(blockIdx.x + blockIdx.y * tiles, tiles * gridDim.y);
+    const int tile = logical % tiles, chunk = logical / tiles;
+    const int y0 = tile / ntZ * TY, z0 = tile % ntZ * STZ;
+    const int x0 = chunk * xchunk, x1 = min(x0 + xchunk, d0);
+    const int t = threadIdx.x, tz = t % STZ, ty = t / STZ * YB;
+    int off[NL];
+#pragma unroll
+    for (int q = 0; q < NL; ++q) {
+        const int e = min(t + q * ST, PLANE - 1);
+        off[q] = reflect_cell(y0 - R + e / RZ, d1) * d2 + reflect_cell(z0 - R + e % RZ, d2);
+    }
+    double pf[NL];
+    auto fetch = [&](int p) {
+        const double *src = in + (size_t)reflect_cell(p, d0) * d1 * d2;
+#pragma unroll
+        for (int q = 0; q < NL; ++q) pf[q] = src[off[q]];
+    };
+    double acc[YB][NR];  // partial sums of the output planes p - R .. p + R
+#pragma unroll
+    for (int y = 0; y < YB; ++y)
+#pragma unroll
+        for (int j = 0; j < NR; ++j) acc[y][j] = 0;
+    const int steps = x1 - x0 + 2 * R;
+    fetch(x0 - R);
+#pragma unroll 1
+    for (int st = 0; st < steps; ++st) {
+        const int p = x0 - R + st;  // input plane
+        double *cur = sp[st & 1];
+#pragma unroll
+        for (int q = 0; q < NL; ++q)
+            if (t + q * ST < PLANE) cur[t + q * ST] = pf[q];
+        if (st + 1 < steps) fetch(p + 1);
+        __syncthreads();
+        // S[y][class of (b, c)]: the plane's values at offsets (+-b, +-c) and (+-c, +-b) of output y, rows in turn
+        double S[YB][NC];
+#pragma unroll
+        for (int r = 0; r < YB + 2 * R; ++r) {
+            const double *row = cur + (ty + r) * RZ + tz + R;
+            double T[R + 1];
+            T[0] = row[0];
+#pragma unroll
+            for (int c = 1; c <= R; ++c) T[c] = row[c] + row[-c];
+#pragma unroll
+            for (int y = 0; y < YB; ++y) {
+                const int db = r - y - R, b = db < 0 ? -db : db;
+                if (b > R) continue;
+#pragma unroll
+                for (int c = 0; c <= R; ++c) {
+                    const int k = b > c ? b * (b + 1) / 2 + c : c * (c + 1) / 2 + b;
+                    // the first row to reach class (h, l), l <= h, is the one at offset -h, with c = l
+                    if (db < 0 && b >= c) {
+                        S[y][k] = T[c];
+                    } else if (k == 0) {
+                        S[y][0] = T[0];
+                    } else {
+                        S[y][k] += T[c];
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int y = 0; y < YB; ++y)
+#pragma unroll
+            for (int a = 0; a <= R; ++a) {
+                double P = 0;
+#pragma unroll
+                for (int k = 0; k < NC; ++k) {
+                    const int b = k < 1 ? 0 : k < 3 ? 1 : k < 6 ? 2 : k < 10 ? 3 : 4, c = k - b * (b + 1) / 2;
+                    if (HAT ? a * a + b * b + c * c < (R + 1) * (R + 1) : (bool)((sw.mask[a] >> k) & 1))
+                        P += sw.w[a * NC + k] * S[y][k];
+                }
+                acc[y][R - a] += P;
+                if (a) acc[y][R + a] += P;
+            }
+        const int o = p - R;  // complete now
+        if (o >= x0 && z0 + tz < d2) {
+#pragma unroll
+            for (int y = 0; y < YB; ++y)
+                if (y0 + ty + y < d1) out[((size_t)o * d1 + y0 + ty + y) * d2 + z0 + tz] = acc[y][0] / W;
+        }
+#pragma unroll
+        for (int y = 0; y < YB; ++y) {
+#pragma unroll
+            for (int j = 0; j + 1 < NR; ++j) acc[y][j] = acc[y][j + 1];
+            acc[y][NR - 1] = 0;
+        }
+    }
+}
+
 }  // namespace
+
+template <int R, int YB, bool HAT>
+static void launch_smoothing_march(const int d[3], const SmoothWeights &sw, double W, const double *in, double *out,
+                                   hipStream_t s) {
+    constexpr int TY = ST / STZ * YB;
+    const int ntY = (d[1] + TY - 1) / TY, ntZ = (d[2] + STZ - 1) / STZ, tiles = ntY * ntZ;
+    const int chunks = plane_chunks(tiles, d[0], 1024, resident_workgroups((const void *)k_smoothing_march<R, YB, HAT>, ST));
+    const int xchunk = (d[0] + chunks - 1) / chunks;
+    hipLaunchKernelGGL((k_smoothing_march<R, YB, HAT>), dim3(tiles, (d[0] + xchunk - 1) / xchunk), dim3(ST), 0, s, d[0],
+                       d[1], d[2], sw, W, in, out, ntZ, xchunk);
+    VF_HIP(hipGetLastError());
+}
+
+bool launch_smoothing_filter_march(const int dims[3], int R, double rmin, int type, double W, const double *in, double *out,
+                                   hipStream_t s) {
+    const long n = (long)dims[0] * dims[1] * dims[2];
+    if (R < 1 || R > 4 || n <= 0) return false;
+    const int NC = (R + 1) * (R + 2) / 2;
+    SmoothWeights sw = {};
+    bool hat = true;
+    for (int a = 0; a <= R; ++a)
+        for (int b = 0; b <= R; ++b)
+            for (int c = 0; c <= b; ++c) {
+                const int k = b * (b + 1) / 2 + c;
+                const double w = type == 1 ? rmin - std::sqrt((double)(a * a + b * b + c * c)) : 1.0;
+                const bool inside = w > 0;
+                if (inside) {
+                    sw.w[a * NC + k] = w;
+                    sw.mask[a] |= 1u << k;
+                }
+                hat = hat && inside == (a * a + b * b + c * c < (R + 1) * (R + 1));
+            }
+    auto go = [&](auto r, auto yb) {
+        if (hat) launch_smoothing_march<decltype(r)::value, decltype(yb)::value, true>(dims, sw, W, in, out, s);
+        else launch_smoothing_march<decltype(r)::value, decltype(yb)::value, false>(dims, sw, W, in, out, s);
+    };
+    // four outputs per work-item along y; two for R = 4, whose folded rows would not fit the registers
+    if (R == 1) go(std::integral_constant<int, 1>(), std::integral_constant<int, 4>());
+    else if (R == 2) go(std::integral_constant<int, 2>(), std::integral_constant<int, 4>());
+    else if (R == 3) go(std::integral_constant<int, 3>(), std::integral_constant<int, 4>());
+    else go(std::integral_constant<int, 4>(), std::integral_constant<int, 2>());
+    return true;
+}
 
 void upsample_dims(int nd, const int64_t *in, int factor, int64_t *out) {
     for (int k = 0; k < nd; ++k) out[k] = (in[k] - 1) * factor + 1;

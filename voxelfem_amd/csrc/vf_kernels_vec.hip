@@ -956,6 +956,8 @@ void launch_smoothing_filter(const int dims[3], double rmin, int type, const dou
                 const double w = type == 1 ? rmin - sqrt((double)(a * a + b * b + c * c)) : 1.0;
                 if (w > 0) W += w;
             }
+    // reaches of one to four voxels march with the folded kernel; wider ones (and R = 0) sum tap by tap
+    if (launch_smoothing_filter_march(dims, R, rmin, type, W, in, out, s)) return;
     const long n = (long)dims[0] * dims[1] * dims[2];
     hipLaunchKernelGGL(k_smoothing, dim3(nblocks(n)), dim3(TPB), 0, s, dims[0], dims[1], dims[2], R, rmin, type, W, in,
                        out);
