@@ -87,3 +87,18 @@ def test_smoothing_march_non_finite(bad):
         sf.setInputDimensions(list(dims))
         sf.rmin = rmin
         assert np.array_equal(np.isfinite(sf.apply(x)), np.isfinite(orc.smoothing_filter(x, dims, rmin, linear)))
+
+
+# the factorization's launches: one block and a padded remainder, no block below the diagonal, a band of several blocks;
+# the coarse solve multiplies the relative rounding by the operator's condition number, as in test_gpu_parity: 1e-9
+@pytest.mark.parametrize("ne,levels", [((2, 2, 2), 1), ((4, 4, 2), 1), ((16, 2, 2), 1), ((32, 4, 4), 1), ((8, 16, 16), 1),
+                                       ((48, 16, 16), 1)])
+@pytest.mark.parametrize("graphs", [False, True])
+def test_coarse_factor(ne, levels, graphs):
+    mg, om = pair(ne, levels)
+    mg.useGraphs = graphs
+    rng = np.random.default_rng(6)
+    for _ in range(3):  # with graphs: captured, then replayed
+        mg.updateStiffnessMatrices()
+        b = rng.normal(size=(om.num_nodes(levels), 3))
+        assert rel(mg._coarseSolve(b), om.coarse_solve(b)) < 1e-9

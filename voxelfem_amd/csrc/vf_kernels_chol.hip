@@ -4,12 +4,13 @@
 // after every stiffness update. Here the reduced operator (fixed and detached DoFs removed, natural node
 // order, so its half-bandwidth is about 3 (nny nnz + nnz + 1)) is stored as 64 x 64 blocks of its lower
 // band and factored by a blocked right-looking band Cholesky A = L L^T:
-//   for each block column k: L_kk = chol(A_kk) (one workgroup, LDS), L_ik = A_ik L_kk^-T for the kb blocks
-//   below, A_ij -= L_ik L_jk^T for the trailing triangle of the band.
+//   for each block column k: L_kk^-1 from A_kk, L_ik = A_ik L_kk^-T for the kb blocks below, A_ij -= L_ik L_jk^T for
+//   the trailing triangle of the band.
 // The work is O(n bw^2) instead of the O(n^3) of a dense factorisation. For the solves, the explicit dense
-// lower-triangular X = L^-1 is formed (one workgroup per block column, sequential down the column), so a
-// coarse solve x = X^T (X b) is two bandwidth-bound triangular matrix-vector products instead of a chain of
-// small sequential triangular solves.
+// lower-triangular X = L^-1 is formed block row by block row, so a coarse solve x = X^T (X b) is two bandwidth-bound
+// triangular matrix-vector products instead of a chain of small sequential triangular solves.
+// One launch per block column (k_band_step) does all of that: the chain of block columns is what bounds the
+// factorisation, so nothing that the next diagonal block does not need sits between two links of it.
 #include "vf_internal.hpp"
 
 namespace vf {
@@ -80,308 +81,395 @@ __global__ void k_band_pad_b(const int *__restrict__ n, int nb, int kb, double *
     if (i >= n[blockIdx.y] && i < nb * NB) bandblk(B, kb, blockIdx.x, 0)[(i % NB) * NB + i % NB] = 1.0;
 }
 
-// ---- L_kk = chol(A_kk) and Linv_kk = L_kk^-1 by one workgroup of 256 work-items, four per row.
-// Work-item t holds row r = t % 64 at the columns [16 q, 16 q + 16), q = t / 64 (one quarter of the
-// columns per wavefront), in registers. The factorisation runs in the unscaled (LDL^T) form
-//   A[r][c] -= A[r][j] A[c][j] / A[j][j]   for c > j, r >= c,   j = 0 .. 63,
-// with one barrier per step: the wavefront owning column j (q = j / 16, known at compile time in the
-// unrolled loop) publishes the column in LDS (double-buffered, so the next step's publication cannot
-// overwrite entries still being read) and every work-item then updates its own entries. The pivots
-// d_j = A[j][j] give L[r][c] = A[r][c] / sqrt(d_c). The inverse is X = L^-1 = D^-1/2 Y with Y the inverse of
-// the unit lower factor L1[r][m] = A[r][m] / d_m, formed right-looking from Y = I:
-//   Y[r][c] -= L1[r][m] Y[m][c]   for r > m, c <= m,   m = 0 .. 63,
-// again one barrier per step (row m of Y and column m of L1 published in LDS).
-// flag != 0 on a non-positive pivot.
-constexpr int PTPB = 4 * NB;
-constexpr int PQ = NB / 4;  // columns per work-item
-// returns false (uniformly) on a non-positive pivot; the block is then left partly factored
-__device__ __forceinline__ bool potrf_block(int k, int kb, double *__restrict__ B, double *__restrict__ Linv) {
-    __shared__ double sCol[2][NB];
-    __shared__ double sRow[2][NB];
-    __shared__ double sPiv[NB], sInvPiv[NB], sSqrt[NB], sInvSqrt[NB];
-    // q is uniform over the wavefront: the column-range tests below are scalar branches
-    const int t = threadIdx.x, r = t % NB, q = __builtin_amdgcn_readfirstlane(t / NB);
-    const int c0 = PQ * q;
-    double *Dk = bandblk(B, kb, k, 0);
-    double a[PQ];
+// FP64 MFMA 16x16x4 operand layout: A[i][k] at lane i + 16 k, B[k][j] at lane j + 16 k, result D[4 v + l / 16][l % 16]
+// in element v of lane l (the FP64 form interleaves the four result rows of a lane, unlike the FP32 16x16 forms).
+typedef double dx4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ dx4 mfma(double a, double b, dx4 c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
+// row stride of 64 x 64 blocks in LDS: the sixteen lanes served at once (one entry of sixteen rows) meet no bank twice
+constexpr int LS = 66;
+
+// 1/d to full precision: the hardware estimate x (24 bits) corrected by its residual e = 1 - d x to third order,
+// x (1 + e + e^2); a fraction of the latency of a division, which would bound the chain of pivots
+__device__ __forceinline__ double recip(double d) {
+    const double x = __builtin_amdgcn_rcp(d), e = __builtin_fma(-d, x, 1.0);
+    return __builtin_fma(x, __builtin_fma(e, e, e), x);
+}
+// d^-1/2 the same way: x (1 + e / 2 + 3 e^2 / 8) with e = 1 - d x^2
+__device__ __forceinline__ double rsqrt_full(double d) {
+    const double x = __builtin_amdgcn_rsq(d), e = __builtin_fma(-(d * x), x, 1.0);
+    return __builtin_fma(x, e * __builtin_fma(0.375, e, 0.5), x);
+}
+__device__ __forceinline__ double lane_value(double v, int lane) {  // lane is uniform
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+template <int J>
+__device__ __forceinline__ double row_bcast(double v) {  // lane J of the lane's DPP row of sixteen
+    return __builtin_amdgcn_update_dpp(0.0, v, 0x150 + J, 0xf, 0xf, true);
+}
+__device__ __forceinline__ double even_lane(double v) {  // quad_perm [0, 0, 2, 2]
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0xA0, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0xA0, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+// One elimination step of the wavefront's 16 x 16 block (see chol16) by the 2 x 2 pivot at rows J, J + 1: the rows below
+// lose their combination of the two. The old columns and the pivot come from the lanes that hold them. One wavefront
+// alone is bound by the instructions it issues one after the other, so two rows go per step, and A and Y share one array.
+template <int J>
+__device__ __forceinline__ void chol16_step(double (&a)[4], int r, int part, double (&piv)[3], bool &ok) {
+    constexpr int h = J / 4, i0 = J % 4;
+    const double p00 = lane_value(a[i0], J + 16 * h), p01 = lane_value(a[i0], J + 1 + 16 * h),
+                 p11 = lane_value(a[i0 + 1], J + 1 + 16 * h);
+    const double c0 = __shfl(a[i0], r + 16 * h, 64), c1 = __shfl(a[i0 + 1], r + 16 * h, 64);
+    // the combination of the two rows is formed without the determinant, so that only one product follows its reciprocal
+    const double g0 = r > J + 1 ? c0 * p11 - c1 * p01 : 0.0, g1 = r > J + 1 ? c1 * p00 - c0 * p01 : 0.0;
+    double u[4];
 #pragma unroll
-    for (int i = 0; i < PQ; ++i) a[i] = Dk[r * NB + c0 + i];
+    for (int i = 0; i < 4; ++i) u[i] = __builtin_fma(g1, row_bcast<J + 1>(a[i]), g0 * row_bcast<J>(a[i]));
+    if (part == h) {  // columns J, J + 1 of Y start here: rows J, J + 1 of it are (1, 0), (0, 1)
+        u[i0] = g0;
+        u[i0 + 1] = g1;
+        a[i0] = 0.0;
+        a[i0 + 1] = 0.0;
+    }
+    const double det = __builtin_fma(p00, p11, -(p01 * p01)), id = -recip(det);
+    ok = ok && p00 > 0 && det > 0;
+    if ((r >> 1) == J / 2) {
+        piv[0] = p00;
+        piv[1] = p01;
+        piv[2] = det;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) a[i] = __builtin_fma(id, u[i], a[i]);
+}
+// U = L^-1 of the 16 x 16 symmetric block whose lower triangle is at S (row stride LS), by one wavefront: lane l holds
+// columns 4 (l / 16) .. + 3 of row l % 16. Eliminating two rows at a time turns [A | I] into [.. | Y] with Y A Y^T = D
+// block diagonal with the 2 x 2 pivots P = [p00 p01; p01 p11]; after the step at J the columns up to J + 1 of A are not
+// used again and hold those of Y instead. U = M Y with M = chol(P)^-1 per pivot: M00 = p00^-1/2, M11 = (det / p00)^-1/2,
+// M10 = -p01 / p00 M11. Writes U (zero above its diagonal) to X (row stride LS).
+__device__ __forceinline__ bool chol16(const double *S, double *X, int l) {
+    const int r = l & 15, part = l >> 4, c0 = 4 * part;
+    double a[4], piv[3] = {1.0, 0.0, 1.0};
     bool ok = true;
 #pragma unroll
-    for (int j = 0; j < NB; ++j) {
-        const int b = j & 1;
-        if (q == j / PQ) {
-            if (r >= j) sCol[b][r] = a[j % PQ];
-            if (r == j) sPiv[j] = a[j % PQ];
-        }
-        __syncthreads();
-        const double piv = sCol[b][j];
-        ok = ok && piv > 0;
-        // rows at or above j take f = 0 (a select: their sCol entries are stale); entries right of the
-        // diagonal (c > r) are updated too but never used
-        const double f = r > j ? sCol[b][r] * (1.0 / (piv > 0 ? piv : 1.0)) : 0.0;
-        if (q > j / PQ) {
+    for (int i = 0; i < 4; ++i) a[i] = S[max(r, c0 + i) * LS + min(r, c0 + i)];
+    chol16_step<0>(a, r, part, piv, ok);
+    chol16_step<2>(a, r, part, piv, ok);
+    chol16_step<4>(a, r, part, piv, ok);
+    chol16_step<6>(a, r, part, piv, ok);
+    chol16_step<8>(a, r, part, piv, ok);
+    chol16_step<10>(a, r, part, piv, ok);
+    chol16_step<12>(a, r, part, piv, ok);
+    chol16_step<14>(a, r, part, piv, ok);
+    const bool odd = r & 1;
+    const double ip = recip(piv[0]), scale = rsqrt_full(odd ? piv[2] * ip : piv[0]), m = odd ? -piv[1] * ip : 0.0;
 #pragma unroll
-            for (int i = 0; i < PQ; ++i) a[i] -= f * sCol[b][c0 + i];
-        } else if (q == j / PQ) {
-#pragma unroll
-            for (int i = j % PQ + 1; i < PQ; ++i) a[i] -= f * sCol[b][c0 + i];
-        }
-    }
-    if (!ok) return false;  // uniform: every work-item saw the same pivots
-    if (t < NB) {
-        const double d = sPiv[t], sq = sqrt(d);
-        sSqrt[t] = sq;
-        sInvSqrt[t] = 1.0 / sq;
-        sInvPiv[t] = 1.0 / d;
-    }
-    __syncthreads();
-    double y[PQ];
-#pragma unroll
-    for (int i = 0; i < PQ; ++i) y[i] = (c0 + i == r) ? 1.0 : 0.0;
-#pragma unroll
-    for (int m = 0; m < NB; ++m) {
-        const int b = m & 1;
-        if (r == m) {
-#pragma unroll
-            for (int i = 0; i < PQ; ++i) sRow[b][c0 + i] = y[i];
-        }
-        if (q == m / PQ && r > m) sCol[b][r] = a[m % PQ] * sInvPiv[m];
-        __syncthreads();
-        const double f = r > m ? sCol[b][r] : 0.0;
-        if (q < m / PQ) {
-#pragma unroll
-            for (int i = 0; i < PQ; ++i) y[i] -= f * sRow[b][c0 + i];
-        } else if (q == m / PQ) {
-#pragma unroll
-            for (int i = 0; i <= m % PQ; ++i) y[i] -= f * sRow[b][c0 + i];
-        }
-    }
-    double *Lk = Linv + (size_t)k * BB;
-    const double isr = sInvSqrt[r];
-#pragma unroll
-    for (int i = 0; i < PQ; ++i) {
+    for (int i = 0; i < 4; ++i) {
         const int c = c0 + i;
-        Dk[r * NB + c] = c < r ? a[i] * sInvSqrt[c] : (c == r ? sSqrt[r] : 0.0);
-        Lk[r * NB + c] = c <= r ? y[i] * isr : 0.0;
+        const double y = c == r ? 1.0 : c < (r & ~1) ? a[i] : 0.0;  // row r of Y
+        X[r * LS + c] = scale * __builtin_fma(m, even_lane(y), y);
     }
-    return true;
+    return ok;
 }
-// nbz (batched, optional): system z uses only its first nbz[z] blocks (the rest is padding nothing reads)
-__global__ void __launch_bounds__(PTPB) k_potrf_diag(int k, int kb, double *__restrict__ B, double *__restrict__ Linv,
-                                                     int *__restrict__ flag, size_t zB, size_t zL,
-                                                     const int *__restrict__ nbz) {
-    if (nbz && k >= nbz[blockIdx.z]) return;
-    B += blockIdx.z * zB;
-    Linv += blockIdx.z * zL;
-    if (!potrf_block(k, kb, B, Linv) && threadIdx.x == 0) atomicOr(flag + blockIdx.z, 1);
-}
-
-// C (+)= alpha * P * Q^T for 64 x 64 row-major blocks, 256 work-items with 4 x 4 register tiles.
-// sP and sQ are LDS staging (P, Q copied in); accumulates into acc[4][4] for rows 4*(t/16).., cols 4*(t%16)..
-__device__ __forceinline__ void gemm_nt_64(const double (*sP)[NB + 1], const double (*sQ)[NB + 1], int t,
-                                           double acc[4][4]) {
-    const int r0 = 4 * (t / 16), c0 = 4 * (t % 16);
-    for (int m = 0; m < NB; ++m) {
-        double p[4], q[4];
+// D (16 x 16) = P Q^T (NT) or P Q (NN) over K = 16 columns of P, both in LDS with row stride LS, added to acc
+__device__ __forceinline__ dx4 mul16_nt(const double *P, const double *Q, dx4 acc, int li, int lk) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            p[i] = sP[r0 + i][m];
-            q[i] = sQ[c0 + i][m];
+    for (int s = 0; s < 4; ++s) acc = mfma(P[li * LS + 4 * s + lk], Q[li * LS + 4 * s + lk], acc);
+    return acc;
+}
+__device__ __forceinline__ dx4 mul16_nn(const double *P, const double *Q, dx4 acc, int li, int lk) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) acc = mfma(P[li * LS + 4 * s + lk], Q[(4 * s + lk) * LS + li], acc);
+    return acc;
+}
+// X = L^-1 of the 64 x 64 block whose lower triangle is in S, by a workgroup of four wavefronts, in 16 x 16 blocks.
+// Step p: wavefront 0 updates diagonal block p and inverts its factor (the serial chain) while the others update the
+// remaining tiles with panel p - 1 and form the sums T_pj = sum_m L_pm X_mj of row p of the inverse (in the unused blocks
+// above the diagonal of S); then the panel L_ip = S_ip U_p^T below and the row X_pj = -U_p T_pj take one wavefront each.
+// The upper triangle of X is zeroed. Returns false (in wavefront 0) on a non-positive pivot.
+__device__ __forceinline__ bool potrf_inverse(double *S, double *X, int t) {
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6), l = t & 63, li = l & 15, lk = l >> 4;
+    auto blk = [](double *M, int i, int j) { return M + (16 * i) * LS + 16 * j; };
+    auto put = [&](double *D, dx4 v, double sign) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) D[(4 * q + lk) * LS + li] = sign * v[q];
+    };
+    auto trail = [&](int i, int j, int p) {  // S_ij -= L_ip L_jp^T
+        const dx4 v = mul16_nt(blk(S, i, p), blk(S, j, p), dx4{0, 0, 0, 0}, li, lk);
+        double *D = blk(S, i, j);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) D[(4 * q + lk) * LS + li] -= v[q];
+    };
+    bool ok = true;
+    for (int e = t; e < 6 * 256; e += TPB) {  // the blocks above the diagonal
+        const int q = e >> 8, i = q < 3 ? 0 : q < 5 ? 1 : 2, j = q < 3 ? q + 1 : q < 5 ? q - 1 : 3;
+        X[(16 * i + ((e >> 4) & 15)) * LS + 16 * j + (e & 15)] = 0.0;
+    }
+#pragma unroll 1
+    for (int p = 0; p < 4; ++p) {
+        if (w == 0) {
+            if (p) trail(p, p, p - 1);
+            __builtin_amdgcn_wave_barrier();
+            ok = chol16(blk(S, p, p), blk(X, p, p), l) && ok;
+        } else if (p) {
+            int q = 0;
+            for (int j = p; j < 4; ++j)
+                for (int i = j + (j == p); i < 4; ++i)
+                    if (q++ % 3 == w - 1) trail(i, j, p - 1);
+            for (int j = 0; j < p; ++j)
+                if (q++ % 3 == w - 1) {
+                    dx4 v = {0, 0, 0, 0};
+#pragma unroll 1
+                    for (int m = j; m < p; ++m) v = mul16_nn(blk(S, p, m), blk(X, m, j), v, li, lk);
+                    put(blk(S, j, p), v, 1.0);
+                }
         }
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc[i][j] += p[i] * q[j];
+        __syncthreads();
+        if (w < 3) {
+            if (w < p) {
+                put(blk(X, p, w), mul16_nn(blk(X, p, p), blk(S, w, p), dx4{0, 0, 0, 0}, li, lk), -1.0);
+            } else {
+                double *D = blk(S, w + 1, p);
+                put(D, mul16_nt(D, blk(X, p, p), dx4{0, 0, 0, 0}, li, lk), 1.0);
+            }
+        }
+        __syncthreads();
     }
+    return ok;
 }
 
-// ---- L_ik = A_ik Linv_kk^T for i = k+1 .. min(k+kb, nb-1)   (grid: one workgroup per block)
-__global__ void __launch_bounds__(TPB) k_trsm_panel(int k, int nb, int kb, double *__restrict__ B,
-                                                    const double *__restrict__ Linv, size_t zB, size_t zL,
-                                                    const int *__restrict__ nbz) {
-    if (nbz) nb = min(nb, nbz[blockIdx.z]);
-    B += blockIdx.z * zB;
-    Linv += blockIdx.z * zL;
-    __shared__ double sP[NB][NB + 1];
-    __shared__ double sQ[NB][NB + 1];
-    const int q = 1 + blockIdx.x, I = k + q;
-    if (I >= nb) return;
+// writes X = L^-1 of diagonal block k from LDS to Linv (64 x 64, row-major)
+__device__ __forceinline__ void store_linv(const double *sX, double *__restrict__ Linv, int k, int t) {
+    double *Lk = Linv + (size_t)k * BB;
+    for (int e = t; e < BB; e += TPB) Lk[e] = sX[(e / NB) * LS + e % NB];
+}
+
+// ---- the first diagonal block (grid: systems); nbz (batched, optional): system z uses its first nbz[z] blocks only
+__global__ void __launch_bounds__(TPB) k_band_first(int kb, const double *__restrict__ B, double *__restrict__ Linv,
+                                                    int *__restrict__ flag, size_t zB, size_t zL) {
+    B += blockIdx.x * zB;
+    Linv += blockIdx.x * zL;
+    __shared__ double sA[NB * LS], sX[NB * LS];
     const int t = threadIdx.x;
-    double *Aik = bandblk(B, kb, I, q);
-    const double *Lk = Linv + (size_t)k * BB;
-    for (int w = t; w < BB; w += TPB) {
-        sP[w / NB][w % NB] = Aik[w];
-        sQ[w / NB][w % NB] = Lk[w];
-    }
-    __syncthreads();
-    double acc[4][4] = {};
-    gemm_nt_64(sP, sQ, t, acc);
-    __syncthreads();
-    const int r0 = 4 * (t / 16), c0 = 4 * (t % 16);
+    const double *D = bandblk(B, kb, 0, 0);
+    double v[BB / TPB];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int q = 0; q < BB / TPB; ++q) v[q] = D[q * TPB + t];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) Aik[(r0 + i) * NB + c0 + j] = acc[i][j];
+    for (int q = 0; q < BB / TPB; ++q) sA[(q * TPB + t) / NB * LS + t % NB] = v[q];
+    __syncthreads();
+    if (!potrf_inverse(sA, sX, t) && t == 0) atomicOr(flag + blockIdx.x, 1);
+    store_linv(sX, Linv, 0, t);
 }
 
-// ---- A_IJ -= L_Ik L_Jk^T for k < J <= I <= min(k+kb, nb-1)  (grid: one workgroup per pair)
-__global__ void __launch_bounds__(TPB) k_band_update(int k, int nb, int kb, double *__restrict__ B, size_t zB,
-                                                     const int *__restrict__ nbz) {
-    if (nbz) nb = min(nb, nbz[blockIdx.z]);
-    B += blockIdx.z * zB;
-    __shared__ double sP[NB][NB + 1];
-    __shared__ double sQ[NB][NB + 1];
-    // decode pair index -> (a, b) with 1 <= b <= a <= m
-    int p = blockIdx.x, a = 1;
-    while (p >= a) { p -= a; ++a; }
-    const int b = p + 1;
-    const int I = k + a, J = k + b;
-    if (I >= nb) return;
-    const int t = threadIdx.x;
-    const double *Lik = bandblk(B, kb, I, a), *Ljk = bandblk(B, kb, J, b);
-    double *Aij = bandblk(B, kb, I, a - b);
-    for (int w = t; w < BB; w += TPB) {
-        sP[w / NB][w % NB] = Lik[w];
-        sQ[w / NB][w % NB] = Ljk[w];
+// L = A Linv^T for one 64 x 64 block A of the panel, into LDS and, where wanted, to Lp (leading dimension ld): wavefront
+// w forms rows 16 w .. (Linv is lower triangular, so column tile j needs the first 16 (j + 1) terms only)
+__device__ __forceinline__ void panel_put(dx4 v, int j, double *sL, double *__restrict__ Lp, size_t ld, int w, int li, int lk) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) sL[(16 * w + 4 * q + lk) * LS + 16 * j + li] = v[q];
+    if (Lp)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) Lp[(size_t)(16 * w + 4 * q + lk) * ld + 16 * j + li] = v[q];
+}
+__device__ __forceinline__ void panel_block(const double *__restrict__ A, const double *__restrict__ Lk, double *sL,
+                                            double *__restrict__ Lp, size_t ld, int w, int li, int lk) {
+    double a[16];
+#pragma unroll
+    for (int s = 0; s < 16; ++s) a[s] = A[(16 * w + li) * NB + 4 * s + lk];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        dx4 v = {0, 0, 0, 0};
+#pragma unroll
+        for (int s = 0; s < 4 * (j + 1); ++s) v = mfma(a[s], Lk[(16 * j + li) * NB + 4 * s + lk], v);
+        panel_put(v, j, sL, Lp, ld, w, li, lk);
     }
-    __syncthreads();
-    double acc[4][4] = {};
-    gemm_nt_64(sP, sQ, t, acc);
-    const int r0 = 4 * (t / 16), c0 = 4 * (t % 16);
+}
+// the same with A in sP (replaced by L; each wavefront touches its own rows only) and Linv in sL
+__device__ __forceinline__ void panel_rows(double *sP, const double *sL, double *__restrict__ Lp, size_t ld, int w, int li,
+                                           int lk) {
+    double a[16];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int s = 0; s < 16; ++s) a[s] = sP[(16 * w + li) * LS + 4 * s + lk];
+    dx4 v[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) Aij[(r0 + i) * NB + c0 + j] -= acc[i][j];
+    for (int j = 0; j < 4; ++j) v[j] = dx4{0, 0, 0, 0};
+#pragma unroll
+    for (int s = 0; s < 16; ++s)
+#pragma unroll
+        for (int j = s / 4; j < 4; ++j) v[j] = mfma(a[s], sL[(16 * j + li) * LS + 4 * s + lk], v[j]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) panel_put(v[j], j, sP, Lp, ld, w, li, lk);
 }
 
-// ---- X = L^-1 (dense lower triangular, row-major, ld = nb*64), one workgroup per 16-column strip of a
-//      block column J: X_JJ = Linv_JJ; X_IJ = -Linv_II * sum_{q=1..min(kb,I-J)} L_{I,I-q} X_{I-q,J}.
-// Columns of X are independent, so the strips of one block column run in parallel and each workgroup's
-// sequential chain down the column is four times shorter in work than a whole block column's. Both products
-// are FP64 MFMA (v_mfma_f64_16x16x4f64): wave w owns rows 16w..16w+15 of the 64 x 16 strip; operand lane
-// layout A[i][k] at lane i + 16k, B[k][j] at lane j + 16k, result D[4 v + l / 16][l % 16] in element v of
-// lane l (the FP64 form interleaves the four result rows of a lane, unlike the FP32 16x16 forms). The operands come straight from global memory (L2-resident band blocks and earlier strips of X);
-// T = sum_q L X goes through LDS once so every wave sees all 64 of its rows as the K dimension of Linv T.
-typedef double dx4 __attribute__((ext_vector_type(4)));
-constexpr int SW = 16;
-__global__ void __launch_bounds__(TPB) k_band_inverse(int nb, int kb, const double *__restrict__ B,
-                                                      const double *__restrict__ Linv, double *__restrict__ X,
-                                                      size_t zB, size_t zL, size_t zX, const int *__restrict__ nbz) {
-    const size_t ld = (size_t)nb * NB;  // leading dimension of X (the padded size)
-    if (nbz) nb = min(nb, nbz[blockIdx.z]);
-    B += blockIdx.z * zB;
-    Linv += blockIdx.z * zL;
-    X += blockIdx.z * zX;
-    __shared__ double sT[NB][SW + 1];
-    const int J = blockIdx.x / (NB / SW), cs = (blockIdx.x % (NB / SW)) * SW;  // strip columns J*NB+cs ..
-    if (J >= nb) return;
+// ---- everything that block column k allows once Linv_k is known (grid: systems x roles):
+//   roles 0 .. m (m + 1) / 2 - 1, m = min(kb, nb - 1 - k): the pair (a, b), 1 <= b <= a <= m, forms L_{k+a,k} and
+//     L_{k+b,k} from the panel (each pair for itself: the products cost less than a launch between panel and update)
+//     and subtracts their product from A_{k+a,k+b}. Pairs with b = 1 store L_{k+a,k} in the lower block triangle of XT,
+//     which nothing else uses. Role 0 is the pair (1, 1), which goes on to invert the factor of diagonal block k + 1:
+//     that is the chain from launch to launch;
+//   the roles after them: strips of 16 CT columns of block row k of X, X_kJ = -Linv_k sum_q L_{k,k-q} X_{k-q,J}
+//     (J < k), X_kk = Linv_k, and their transposes into XT. They are off the chain and fill the chip beside it. CT = 1
+//     spreads a row over four times the workgroups; CT = 4 reads each band block a quarter as often.
+// 4131 unknowns, kb = 5: 61 launches of 16.0 us against 183 of 13.0 (panel), 13.1 (update) and 52.2 us (diagonal block)
+// and 61 of 14.8 us for the rows of X: 0.99 against 5.66 ms. Of the 16 us the loads take 1.7, the panel 1.7, the update
+// 1.9, the diagonal block 8.3 (four 16 x 16 factors of 1.3 us one after the other) and the launch the rest.
+template <int CT>
+__global__ void __launch_bounds__(TPB) k_band_step(int k, int nb, int kb, double *__restrict__ B, double *__restrict__ Linv,
+                                                   double *__restrict__ X, double *__restrict__ XT, int *__restrict__ flag,
+                                                   size_t zB, size_t zL, size_t zX, const int *__restrict__ nbz) {
+    const size_t ld = (size_t)nb * NB;  // leading dimension of X and XT (the padded size)
+    const int mPairs = min(kb, nb - 1 - k), npairs = mPairs * (mPairs + 1) / 2;
+    const int z = blockIdx.x;
+    if (nbz) nb = min(nb, nbz[z]);
+    if (k >= nb) return;
+    B += z * zB;
+    Linv += z * zL;
+    X += z * zX;
+    XT += z * zX;
+    __shared__ double sP[NB * LS], sQ[NB * LS];
     const int t = threadIdx.x, w = t >> 6, l = t & 63, li = l & 15, lk = l >> 4;
-    const int col0 = J * NB + cs;
-    {
-        const double *Lj = Linv + (size_t)J * BB;
-        for (int e = t; e < NB * SW; e += TPB) {
-            const int r = e / SW, c = e % SW;
-            X[(size_t)(J * NB + r) * ld + col0 + c] = Lj[r * NB + cs + c];
-        }
-    }
-    __threadfence();
-    __syncthreads();
-    const int rowA = 16 * w + li;
-    for (int I = J + 1; I < nb; ++I) {
-        dx4 acc = {0.0, 0.0, 0.0, 0.0};
-        const int qmax = min(kb, I - J);
-        for (int q = 1; q <= qmax; ++q) {
-            const double *Lb = bandblk(B, kb, I, q) + rowA * NB + lk;
-            const double *Xb = X + ((size_t)(I - q) * NB + lk) * ld + col0 + li;
-            double a[16], b[16];
+    const double *Lk = Linv + (size_t)k * BB;
+    int role = blockIdx.y;
+    if (role < npairs) {
+        int a = 1;
+        while (role >= a) { role -= a; ++a; }
+        const int b = role + 1, I = k + a, J = k + b;
+        if (I >= nb) return;
+        double *Aij = bandblk(B, kb, I, a - b), *Lp = XT + (size_t)I * NB * ld + (size_t)k * NB;
+        if (a == b) {
+            // both operands of the panel product go through LDS, requested at once with the block to update: this is
+            // the path of the chain, which waits for one round of loads. Of A_II only the tiles on and below the
+            // diagonal are needed: tile q = w, w + 4, w + 8 of the ten goes to wavefront w
+            constexpr uint64_t tr = 0x3323213210, tc = 0x3221110000;  // row and column of tile q, a nibble each
+            const double *A = bandblk(B, kb, I, a);
+            double va[16], vl[16], old[3][4];
 #pragma unroll
-            for (int s = 0; s < 16; ++s) {
-                a[s] = Lb[4 * s];
-                b[s] = Xb[(size_t)(4 * s) * ld];
+            for (int q = 0; q < 16; ++q) {
+                va[q] = A[q * TPB + t];
+                vl[q] = Lk[q * TPB + t];
+            }
+            const int wu = __builtin_amdgcn_readfirstlane(w);
+            int ti[3], tj[3];
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+                const int id = min(wu + 4 * q, 9);
+                ti[q] = (int)(tr >> (4 * id)) & 15;
+                tj[q] = (int)(tc >> (4 * id)) & 15;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) old[q][v] = Aij[(16 * ti[q] + 4 * v + lk) * NB + 16 * tj[q] + li];
             }
 #pragma unroll
-            for (int s = 0; s < 16; ++s) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s], b[s], acc, 0, 0, 0);
-        }
+            for (int q = 0; q < 16; ++q) {
+                sP[(q * TPB + t) / NB * LS + t % NB] = va[q];
+                sQ[(q * TPB + t) / NB * LS + t % NB] = vl[q];
+            }
+            __syncthreads();
+            panel_rows(sP, sQ, a == 1 ? Lp : nullptr, ld, w, li, lk);
+            __syncthreads();
+            dx4 v[3];
 #pragma unroll
-        for (int v = 0; v < 4; ++v) sT[16 * w + 4 * v + lk][li] = acc[v];
+            for (int q = 0; q < 3; ++q) v[q] = dx4{0, 0, 0, 0};
+#pragma unroll
+            for (int s = 0; s < 16; ++s)  // the sums side by side: a product waits for the one before it in its sum
+#pragma unroll
+                for (int q = 0; q < 3; ++q)
+                    v[q] = mfma(sP[(16 * ti[q] + li) * LS + 4 * s + lk], sP[(16 * tj[q] + li) * LS + 4 * s + lk], v[q]);
+            if (a != 1) {
+#pragma unroll
+                for (int q = 0; q < 3; ++q)
+                    if (wu + 4 * q <= 9)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            Aij[(16 * ti[q] + 4 * e + lk) * NB + 16 * tj[q] + li] = old[q][e] - v[q][e];
+                return;
+            }
+            __syncthreads();  // the panel block in sP has been read by every wavefront
+#pragma unroll
+            for (int q = 0; q < 3; ++q)
+                if (wu + 4 * q <= 9)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        sP[(16 * ti[q] + 4 * e + lk) * LS + 16 * tj[q] + li] = old[q][e] - v[q][e];
+            __syncthreads();
+            if (!potrf_inverse(sP, sQ, t) && t == 0) atomicOr(flag + z, 1);
+            store_linv(sQ, Linv, k + 1, t);
+            return;
+        }
+        double old[4][4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) old[j][q] = Aij[(16 * w + 4 * q + lk) * NB + 16 * j + li];
+        panel_block(bandblk(B, kb, I, a), Lk, sP, b == 1 ? Lp : nullptr, ld, w, li, lk);
+        panel_block(bandblk(B, kb, J, b), Lk, sQ, nullptr, ld, w, li, lk);
         __syncthreads();
-        const double *Li = Linv + (size_t)I * BB + rowA * NB + lk;
-        double a[16], b[16];
+        dx4 v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = dx4{0, 0, 0, 0};
 #pragma unroll
         for (int s = 0; s < 16; ++s) {
-            a[s] = Li[4 * s];
-            b[s] = sT[4 * s + lk][li];
+            const double x = sP[(16 * w + li) * LS + 4 * s + lk];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = mfma(x, sQ[(16 * j + li) * LS + 4 * s + lk], v[j]);
         }
-        dx4 out = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-        for (int s = 0; s < 16; ++s) out = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s], b[s], out, 0, 0, 0);
-        double *Xi = X + ((size_t)I * NB + 16 * w + lk) * ld + col0 + li;
+        for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) Xi[(size_t)(4 * v) * ld] = -out[v];
-        // the strip is read back by the other waves in the next kb steps; sT is rewritten next step
-        __threadfence();
-        __syncthreads();
+            for (int q = 0; q < 4; ++q) Aij[(16 * w + 4 * q + lk) * NB + 16 * j + li] = old[j][q] - v[j][q];
+        return;
     }
-}
-
-// ---- block row I of X = L^-1 for every block column J <= I at once (batched systems): the same products as
-//      one step of k_band_inverse, so X is identical. Row by row, each band block L_{I,I-q} is read by the
-//      strips of one launch while it is hot in the caches, instead of once per strip and row as in the
-//      column-walking form, whose re-reads of the band dominate when nb is large (grid: (I + 1) * 4 strips,
-//      systems; a system with nbz[z] <= I is done).
-__global__ void __launch_bounds__(TPB) k_band_inverse_row(int I, int nb, int kb, const double *__restrict__ B,
-                                                          const double *__restrict__ Linv, double *__restrict__ X,
-                                                          size_t zB, size_t zL, size_t zX,
-                                                          const int *__restrict__ nbz) {
-    const size_t ld = (size_t)nb * NB;
-    if (nbz && I >= nbz[blockIdx.z]) return;
-    B += blockIdx.z * zB;
-    Linv += blockIdx.z * zL;
-    X += blockIdx.z * zX;
-    __shared__ double sT[NB][SW + 1];
-    const int J = blockIdx.x / (NB / SW), cs = (blockIdx.x % (NB / SW)) * SW;
-    const int t = threadIdx.x, w = t >> 6, l = t & 63, li = l & 15, lk = l >> 4;
-    const int col0 = J * NB + cs;
-    if (J == I) {
-        const double *Lj = Linv + (size_t)J * BB;
-        for (int e = t; e < NB * SW; e += TPB) {
-            const int r = e / SW, c = e % SW;
-            X[(size_t)(J * NB + r) * ld + col0 + c] = Lj[r * NB + cs + c];
+    // ---- a strip of block row k of X
+    constexpr int CW = 16 * CT;
+    role -= npairs;
+    const int J = role / (NB / CW), cs = role % (NB / CW) * CW, col0 = J * NB + cs;
+    if (J > k) return;
+    double *Xr = X + (size_t)k * NB * ld + col0, *XTr = XT + (size_t)col0 * ld + (size_t)k * NB;
+    if (J == k) {
+        for (int e = t; e < NB * CW; e += TPB) {
+            Xr[(size_t)(e / CW) * ld + e % CW] = Lk[(e / CW) * NB + cs + e % CW];
+            XTr[(size_t)(e / NB) * ld + e % NB] = Lk[(e % NB) * NB + cs + e / NB];
         }
         return;
     }
-    const int rowA = 16 * w + li;
-    dx4 acc = {0.0, 0.0, 0.0, 0.0};
-    const int qmax = min(kb, I - J);
+    dx4 v[CT];
+#pragma unroll
+    for (int j = 0; j < CT; ++j) v[j] = dx4{0, 0, 0, 0};
+    const int qmax = min(kb, k - J);
     for (int q = 1; q <= qmax; ++q) {
-        const double *Lb = bandblk(B, kb, I, q) + rowA * NB + lk;
-        const double *Xb = X + ((size_t)(I - q) * NB + lk) * ld + col0 + li;
-        double a[16], b[16];
+        const double *Lb = XT + (size_t)(k * NB + 16 * w + li) * ld + (size_t)(k - q) * NB + lk;
+        const double *Xb = X + ((size_t)(k - q) * NB + lk) * ld + col0 + li;
+        double a[16];
 #pragma unroll
-        for (int s = 0; s < 16; ++s) {
-            a[s] = Lb[4 * s];
-            b[s] = Xb[(size_t)(4 * s) * ld];
+        for (int s = 0; s < 16; ++s) a[s] = Lb[4 * s];
+#pragma unroll
+        for (int j = 0; j < CT; ++j) {
+            double b[16];
+#pragma unroll
+            for (int s = 0; s < 16; ++s) b[s] = Xb[(size_t)(4 * s) * ld + 16 * j];
+#pragma unroll
+            for (int s = 0; s < 16; ++s) v[j] = mfma(a[s], b[s], v[j]);
         }
-#pragma unroll
-        for (int s = 0; s < 16; ++s) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s], b[s], acc, 0, 0, 0);
     }
+    // the sum goes through LDS once, so that every wavefront sees all 64 of its rows as the K dimension of Linv_k T
 #pragma unroll
-    for (int v = 0; v < 4; ++v) sT[16 * w + 4 * v + lk][li] = acc[v];
+    for (int j = 0; j < CT; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) sP[(16 * w + 4 * q + lk) * LS + 16 * j + li] = v[j][q];
     __syncthreads();
-    const double *Li = Linv + (size_t)I * BB + rowA * NB + lk;
-    double a[16], b[16];
+    double a[16];
 #pragma unroll
-    for (int s = 0; s < 16; ++s) {
-        a[s] = Li[4 * s];
-        b[s] = sT[4 * s + lk][li];
+    for (int s = 0; s < 16; ++s) a[s] = Lk[(16 * w + li) * NB + 4 * s + lk];
+#pragma unroll
+    for (int j = 0; j < CT; ++j) {
+        dx4 o = {0, 0, 0, 0};
+#pragma unroll
+        for (int s = 0; s < 16; ++s) o = mfma(a[s], sP[(4 * s + lk) * LS + 16 * j + li], o);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            Xr[(size_t)(16 * w + 4 * q + lk) * ld + 16 * j + li] = -o[q];
+            XTr[(size_t)(16 * j + li) * ld + 16 * w + 4 * q + lk] = -o[q];
+        }
     }
-    dx4 out = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int s = 0; s < 16; ++s) out = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s], b[s], out, 0, 0, 0);
-    double *Xi = X + ((size_t)I * NB + 16 * w + lk) * ld + col0 + li;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) Xi[(size_t)(4 * v) * ld] = -out[v];
 }
 
 // ---- y = X b over the lower triangle (one wavefront per row)
@@ -395,27 +483,6 @@ __global__ void __launch_bounds__(TPB) k_trmv_lower(int n, int ld, const double 
     for (int j = lane; j <= row; j += 64) s += Xr[j] * b[j];
     for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
     if (lane == 0) y[row] = s;
-}
-
-// ---- XT = X^T for the 64 x 64 tiles on and below the diagonal of X (so XT is filled on and above
-//      its diagonal; the upper triangle of X is zero)
-__global__ void __launch_bounds__(TPB) k_transpose_lower(int ld, const double *__restrict__ X, double *__restrict__ XT,
-                                                         size_t zX, const int *__restrict__ nbz) {
-    X += blockIdx.z * zX;
-    XT += blockIdx.z * zX;
-    const int bi = blockIdx.y, bj = blockIdx.x;  // tile row / column of X
-    if (bj > bi || (nbz && bi >= nbz[blockIdx.z])) return;
-    __shared__ double tl[NB][NB + 1];
-    const int t = threadIdx.x;
-    for (int w = t; w < NB * NB; w += TPB) {
-        const int r = w / NB, c = w % NB;
-        tl[r][c] = X[(size_t)(bi * NB + r) * ld + bj * NB + c];
-    }
-    __syncthreads();
-    for (int w = t; w < NB * NB; w += TPB) {
-        const int r = w / NB, c = w % NB;
-        XT[(size_t)(bj * NB + r) * ld + bi * NB + c] = tl[c][r];
-    }
 }
 
 // ---- x = XT y over the upper triangle of XT (one wavefront per row, coalesced row reads)
@@ -529,30 +596,29 @@ void band_cholesky_inverse(const Grid &g, const double *Ke, const int *red, int 
     band_factor_inverse(n, kb, B, Linv, X, XT, flag, s);
 }
 
+// the launches of the factorization and the inverse for nsys systems (see k_band_step). Rows of X with many strips in
+// flight take the wide ones, which read each band block a quarter as often: above 512 narrow strips (two workgroups on
+// every CU, as many as the LDS holds at once) a row of 8 x 7623 unknowns took 65 us in narrow strips and takes 50 us.
+static void band_steps(int nsys, const int *nbz, int nb, int kb, double *B, double *Linv, double *X, double *XT, int *flags,
+                       size_t zB, size_t zL, size_t zX, hipStream_t s) {
+    hipLaunchKernelGGL(k_band_first, dim3(nsys), dim3(TPB), 0, s, kb, B, Linv, flags, zB, zL);
+    for (int k = 0; k < nb; ++k) {
+        const int m = std::min(kb, nb - 1 - k), pairs = m * (m + 1) / 2;
+        if ((long)nsys * (k + 1) * 4 <= 512)
+            hipLaunchKernelGGL(k_band_step<1>, dim3(nsys, pairs + (k + 1) * 4), dim3(TPB), 0, s, k, nb, kb, B, Linv, X, XT,
+                               flags, zB, zL, zX, nbz);
+        else
+            hipLaunchKernelGGL(k_band_step<4>, dim3(nsys, pairs + k + 1), dim3(TPB), 0, s, k, nb, kb, B, Linv, X, XT, flags,
+                               zB, zL, zX, nbz);
+    }
+    VF_HIP(hipGetLastError());
+}
+
 void band_factor_inverse(int n, int kb, double *B, double *Linv, double *X, double *XT, int *flag, hipStream_t s) {
     const int nb = (n + NB - 1) / NB;
-    const size_t ld = (size_t)nb * NB;
-    launch_fill<double>(ld * ld, X, 0.0, s);
     launch_fill<int>(1, flag, 0, s);
-    if ((int)ld > n) hipLaunchKernelGGL(k_band_pad, dim3(1), dim3(NB), 0, s, n, nb, kb, B);
-    for (int k = 0; k < nb; ++k) {
-        hipLaunchKernelGGL(k_potrf_diag, dim3(1), dim3(PTPB), 0, s, k, kb, B, Linv, flag, 0, 0, nullptr);
-        const int m = std::min(kb, nb - 1 - k);
-        if (m > 0) {
-            hipLaunchKernelGGL(k_trsm_panel, dim3(m), dim3(TPB), 0, s, k, nb, kb, B, Linv, 0, 0, nullptr);
-            hipLaunchKernelGGL(k_band_update, dim3(m * (m + 1) / 2), dim3(TPB), 0, s, k, nb, kb, B, 0, nullptr);
-        }
-    }
-    // small systems: one launch whose strips walk down their block columns; large ones (where re-reading the
-    // band per strip and row dominates): one launch per block row
-    if (nb <= 32)
-        hipLaunchKernelGGL(k_band_inverse, dim3(nb * (NB / SW)), dim3(TPB), 0, s, nb, kb, B, Linv, X, 0, 0, 0, nullptr);
-    else
-        for (int I = 0; I < nb; ++I)
-            hipLaunchKernelGGL(k_band_inverse_row, dim3((I + 1) * (NB / SW)), dim3(TPB), 0, s, I, nb, kb, B, Linv, X, 0,
-                               0, 0, nullptr);
-    hipLaunchKernelGGL(k_transpose_lower, dim3(nb, nb), dim3(TPB), 0, s, (int)ld, X, XT, 0, nullptr);
-    VF_HIP(hipGetLastError());
+    if (nb * NB > n) hipLaunchKernelGGL(k_band_pad, dim3(1), dim3(NB), 0, s, n, nb, kb, B);
+    band_steps(1, nullptr, nb, kb, B, Linv, X, XT, flag, 0, 0, 0, s);
 }
 
 void band_cholesky_inverse_batched(const Grid &g, const double *Ke, size_t keStride, const int *red, size_t redStride,
@@ -561,24 +627,11 @@ void band_cholesky_inverse_batched(const Grid &g, const double *Ke, size_t keStr
     if (nsys < 1 || nsys > 65535 || nb < 1) throw std::runtime_error("batched band Cholesky: bad system count or size");
     const size_t ld = (size_t)nb * NB, zB = band_storage(nb * NB, kb), zL = (size_t)nb * BB, zX = ld * ld;
     launch_fill<double>(zB * nsys, B, 0.0, s);
-    launch_fill<double>(zX * nsys, X, 0.0, s);
     launch_fill<int>(nsys, flags, 0, s);
     hipLaunchKernelGGL(k_band_assemble, dim3(nblk((long)g.nnodes * 81), 1, nsys), dim3(TPB), 0, s, g, Ke, red, kb, B,
                        keStride, redStride, zB);
     hipLaunchKernelGGL(k_band_pad_b, dim3(nb, nsys), dim3(NB), 0, s, n, nb, kb, B, zB);
-    for (int k = 0; k < nb; ++k) {
-        hipLaunchKernelGGL(k_potrf_diag, dim3(1, 1, nsys), dim3(PTPB), 0, s, k, kb, B, Linv, flags, zB, zL, nbz);
-        const int m = std::min(kb, nb - 1 - k);
-        if (m > 0) {
-            hipLaunchKernelGGL(k_trsm_panel, dim3(m, 1, nsys), dim3(TPB), 0, s, k, nb, kb, B, Linv, zB, zL, nbz);
-            hipLaunchKernelGGL(k_band_update, dim3(m * (m + 1) / 2, 1, nsys), dim3(TPB), 0, s, k, nb, kb, B, zB, nbz);
-        }
-    }
-    for (int I = 0; I < nb; ++I)
-        hipLaunchKernelGGL(k_band_inverse_row, dim3((I + 1) * (NB / SW), 1, nsys), dim3(TPB), 0, s, I, nb, kb, B, Linv,
-                           X, zB, zL, zX, nbz);
-    hipLaunchKernelGGL(k_transpose_lower, dim3(nb, nb, nsys), dim3(TPB), 0, s, (int)ld, X, XT, zX, nbz);
-    VF_HIP(hipGetLastError());
+    band_steps(nsys, nbz, nb, kb, B, Linv, X, XT, flags, zB, zL, zX, s);
 }
 
 template <typename T>
