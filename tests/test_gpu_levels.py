@@ -102,3 +102,51 @@ def test_coarse_factor(ne, levels, graphs):
         mg.updateStiffnessMatrices()
         b = rng.normal(size=(om.num_nodes(levels), 3))
         assert rel(mg._coarseSolve(b), om.coarse_solve(b)) < 1e-9
+
+
+# level 1 on the fly: every side of the grid within reach of every node, sides of different length and element size,
+# masked layers, a partially filled workgroup; variant 1 keeps level 1 on the fly
+@pytest.mark.parametrize("ne,levels,layer", [((4, 4, 4), 2, None), ((8, 4, 12), 2, None), ((12, 20, 8), 2, None),
+                                             ((8, 24, 16), 3, 13), ((40, 8, 8), 3, None)])
+@pytest.mark.parametrize("size", [(1.0, 1.0, 1.0), (0.5, 1.5, 2.0)])
+def test_level1_on_the_fly(ne, levels, layer, size):
+    import voxelfem_amd
+    from voxelfem_amd import capi
+
+    pv = voxelfem_amd.pyVoxelFEM
+    rng = np.random.default_rng(8)
+    rho = rng.uniform(0.1, 1.0, int(np.prod(ne)))
+    hi = [n * h for n, h in zip(ne, size)]
+    tps = pv.TensorProductSimulator([1, 1, 1], [[0.0, 0.0, 0.0], hi], list(ne))
+    tps.readMaterial(wl.write_json(wl.MATERIAL, name="material.json"))
+    tps.E_0, tps.E_min, tps.gamma = 1.0, 1e-9, 3.0
+    tps.applyDisplacementsAndLoadsFromFile(wl.write_json(wl.CANTILEVER_BC))
+    tps.setDensities(rho)
+    s = orc.Sim(ne, [0.0, 0.0, 0.0], hi)
+    s.set_etensor(1.0, 0.3)
+    s.set_law(0, 1.0, 1e-9, 3.0, 3.0)
+    s.set_densities(rho)
+    s.set_dirichlet(wl.cantilever_mask(ne))
+    capi.set_kernel_variant(1)
+    try:
+        mg, om = tps.multigridSolver(levels), orc.MG(s, levels)
+        if layer is not None:
+            mg.setFabricationMaskHeightByLayer(layer)
+            om.set_mask_layer(layer)
+        mg.updateStiffnessMatrices()
+        om.update_stiffness()
+        nn = om.num_nodes(1)
+        u, b = rng.normal(size=(nn, 3)), rng.normal(size=(nn, 3))
+        iy = (np.arange(nn) // (ne[2] // 2 + 1)) % (ne[1] // 2 + 1)
+        act = np.ones(nn, bool) if layer is None else iy < -(-layer >> 1) + 1
+        u[~act] = 0
+        assert rel(mg.applyK(1, u)[act], om.apply_K(1, u)[act]) < 1e-12
+        assert rel(mg.computeResidual(1, u, b)[act], om.residual(1, u, b)[act]) < 1e-12
+        for fwd in (True, False):
+            assert rel(mg._smooth(1, u, b, fwd)[act], om.smooth(1, u, b, fwd)[act]) < 1e-11, fwd
+        if layer is None:  # single precision rounds the same sums: 1e-5, as the V-cycles of test_gpu_tiled
+            r = rng.normal(size=(om.num_nodes(0), 3))
+            r[np.arange(len(r)) // ((ne[1] + 1) * (ne[2] + 1)) == 0] = 0
+            assert rel(mg._precondition(r, 1, 1, False, "fp32"), mg._precondition(r, 1, 1, False, "fp64")) < 1e-5
+    finally:
+        capi.set_kernel_variant(0)

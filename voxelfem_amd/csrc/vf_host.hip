@@ -408,8 +408,9 @@ struct vf_mg {
     std::vector<std::unique_ptr<LevelData>> lv;  // lv[0] mirrors the fine simulator
     double phi[512];
     double Chat[8 * 576];
-    DBuf<double> dChat, dphi, dM2, dKe0, dCw;
-    DBuf<float> dChat32, dCw32;
+    L1Coef l1c;  // constants of the level-1 rows formed from the fine moduli
+    DBuf<double> dChat, dphi, dM2, dKe0;
+    DBuf<float> dChat32;
     bool symmetricGS = true;
     bool useGraphs = false;  // replay the steady-state PCG iteration from a captured HIP graph
     // the last solve's iteration graph, destroyed during the next solve's capture (while the device is busy)
@@ -506,17 +507,17 @@ struct vf_mg {
     // hierarchy buffers and work vectors are reused by the next evaluation with the same layers and
     // constraints (the moduli, hierarchy and factors are recomputed every time)
     std::vector<std::shared_ptr<StackedBatch>> stackCache;
-    // the coarsened element matrices (Chat, the level-2 path matrices and the Walsh form of Chat_0) of
+    // the coarsened element matrices (Chat and the level-2 path matrices) of
     // another solver, so that both build identical level operators from the same moduli
     void copy_coarsening(const vf_mg &o) {
         std::copy(o.Chat, o.Chat + 8 * 576, Chat);
+        l1c = o.l1c;
         std::copy(o.phi, o.phi + 512, phi);
         auto dup = [&](auto &dst, const auto &src) {
             dst.resize(src.size());
             d2d(dst.data(), src.data(), src.size(), st());
         };
         dup(dChat, o.dChat); dup(dChat32, o.dChat32); dup(dphi, o.dphi); dup(dM2, o.dM2);
-        dup(dCw, o.dCw); dup(dCw32, o.dCw32);
     }
     // level-0 views used by the cycles (set per preconditioner call)
     double *x0v = nullptr, *b0v = nullptr;
@@ -616,37 +617,13 @@ struct vf_mg {
         child_phi(phi);
         std::fill(Chat, Chat + 8 * 576, 0.0);
         for (int fi = 0; fi < 8; ++fi) coarsen_into(phi, fi, sim->K0h, Chat + fi * 576);
+        l1c = l1_coef_of(sim->young, sim->poisson, sim->h);
         dChat.resize(8 * 576);
         dChat32.resize(8 * 576);
         dphi.resize(512);
         std::vector<float> c32(Chat, Chat + 8 * 576);
         h2d(dChat.data(), Chat, 8 * 576, st());
         h2d(dChat32.data(), c32.data(), 8 * 576, st());
-        // child 0's matrix in the Walsh basis for the element-wise level-1 product: Cw = W^T Chat_0 W / 64
-        {
-            auto wal = [](int l, int k) {
-                int v = 1;
-                for (int a = 0; a < 3; ++a)
-                    if ((k >> (2 - a)) & 1) v *= ((l >> (2 - a)) & 1) ? 1 : -1;
-                return v;
-            };
-            std::vector<double> cw(576, 0.0);
-            for (int k = 0; k < 8; ++k)
-                for (int a = 0; a < 3; ++a)
-                    for (int kp = 0; kp < 8; ++kp)
-                        for (int c = 0; c < 3; ++c) {
-                            double acc = 0;
-                            for (int l = 0; l < 8; ++l)
-                                for (int m = 0; m < 8; ++m)
-                                    acc += wal(l, k) * Chat[(3 * l + a) * 24 + 3 * m + c] * wal(m, kp);
-                            cw[(3 * k + a) * 24 + 3 * kp + c] = acc / 64.0;
-                        }
-            std::vector<float> cw32(cw.begin(), cw.end());
-            dCw.resize(576);
-            dCw32.resize(576);
-            h2d(dCw.data(), cw.data(), 576, st());
-            h2d(dCw32.data(), cw32.data(), 576, st());
-        }
         h2d(dphi.data(), phi, 512, st());
         if (L >= 2) {
             std::vector<double> M2(64 * 576, 0.0);
@@ -693,8 +670,6 @@ struct vf_mg {
     const T *Ep() const;
     template <typename T>
     const T *Chatp() const;
-    template <typename T>
-    const T *Cwp() const;
     template <typename T>
     const T *blocksp(int l) const;
 
@@ -809,7 +784,7 @@ struct vf_mg {
             float tr[3], ts[3];
             tr[0] = best([&] { launch_block_apply<T>(g1, blocksp<T>(1), u.data(), y.data(), rhs.data(), dm(1),
                                                      AM_RESIDUAL, s); });
-            tr[1] = best([&] { launch_l1_apply<T>(g1, g, Chatp<T>(), Cwp<T>(), Ep<T>(), u.data(), y.data(), rhs.data(), dm(1),
+            tr[1] = best([&] { launch_l1_apply<T>(g1, g, Chatp<T>(), l1c, Ep<T>(), u.data(), y.data(), rhs.data(), dm(1),
                                                   AM_RESIDUAL, sim->structured, s); });
             tr[2] = best([&] { launch_l1_apply_mfma<T>(g1, g, Chatp<T>(), Ep<T>(), u.data(), y.data(), rhs.data(),
                                                        dm(1), AM_RESIDUAL, s); });
@@ -822,7 +797,7 @@ struct vf_mg {
                 for (int c = 0; c < 8; ++c) {
                     if (form == 0) launch_block_gs<T>(g1, blocksp<T>(1), u1.data(), b1.data(), dm(1), c, 1, s);
                     else if (form == 1)
-                        launch_l1_gs<T>(g1, g, Chatp<T>(), Ep<T>(), u1.data(), b1.data(), dm(1), c, 1, sim->structured, s);
+                        launch_l1_gs<T>(g1, g, Chatp<T>(), l1c, Ep<T>(), u1.data(), b1.data(), dm(1), c, 1, sim->structured, s);
                     else launch_l1_gs_mfma<T>(g1, g, Chatp<T>(), Ep<T>(), u1.data(), b1.data(), dm(1), c, 1, s);
                 }
             };
@@ -863,7 +838,7 @@ struct vf_mg {
         else if (l == 0 && fam == 1) launch_fine_apply_tiled<T>(lv[0]->g, Fp<T>(), Ep<T>(), u, y, b, mask, mode, st());
         else if (l == 0) launch_fine_apply<T>(lv[0]->g, K0p<T>(), Ep<T>(), u, y, b, mask, mode, st());
         else if (l == 1 && l1_form(pidx<T>(), 0) == 1)
-            launch_l1_apply<T>(lv[1]->g, lv[0]->g, Chatp<T>(), Cwp<T>(), Ep<T>(), u, y, b, mask, mode, sim->structured,
+            launch_l1_apply<T>(lv[1]->g, lv[0]->g, Chatp<T>(), l1c, Ep<T>(), u, y, b, mask, mode, sim->structured,
                                st());
         else if (l == 1 && l1_form(pidx<T>(), 0) == 2)
             launch_l1_apply_mfma<T>(lv[1]->g, lv[0]->g, Chatp<T>(), Ep<T>(), u, y, b, mask, mode, st());
@@ -908,7 +883,7 @@ struct vf_mg {
                 launch_fine_gs_gather_f<T>(lv[0]->g, Fp<T>(), Ep<T>(), u, b, dm(0), color, forward, st());
             else if (l == 0) launch_fine_gs<T>(lv[0]->g, K0p<T>(), Ep<T>(), u, b, dm(0), color, forward, st());
             else if (l == 1 && l1_form(pidx<T>(), 1) == 1)
-                launch_l1_gs<T>(lv[1]->g, lv[0]->g, Chatp<T>(), Ep<T>(), u, b, dm(1), color, forward, sim->structured,
+                launch_l1_gs<T>(lv[1]->g, lv[0]->g, Chatp<T>(), l1c, Ep<T>(), u, b, dm(1), color, forward, sim->structured,
                                 st());
             else if (l == 1 && l1_form(pidx<T>(), 1) == 2)
                 launch_l1_gs_mfma<T>(lv[1]->g, lv[0]->g, Chatp<T>(), Ep<T>(), u, b, dm(1), color, forward, st());
@@ -1677,8 +1652,6 @@ template <> const double *vf_mg::Ep<double>() const { return sim->E.data(); }
 template <> const float *vf_mg::Ep<float>() const { return sim->E32.data(); }
 template <> const double *vf_mg::Chatp<double>() const { return dChat.data(); }
 template <> const float *vf_mg::Chatp<float>() const { return dChat32.data(); }
-template <> const double *vf_mg::Cwp<double>() const { return dCw.data(); }
-template <> const float *vf_mg::Cwp<float>() const { return dCw32.data(); }
 template <> const double *vf_mg::blocksp<double>(int l) const {
     if (!blocksReady[0]) throw std::runtime_error("internal: FP64 block rows used before assembly");
     return lv[l]->blocks.data();

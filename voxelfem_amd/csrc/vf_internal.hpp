@@ -160,11 +160,30 @@ void launch_fine_gs_gather_f(const Grid &g, const T *F, const T *E, T *u, const 
 template <typename T>
 void launch_fine_gs_phase(const Grid &g, const T *K0, const T *E, const T *uin, const T *unb, T *uout, const T *b,
                           const uint8_t *dmask, int parity, int forward, hipStream_t s, int zin = 0);
-// level-1 operator on the fly from the fine moduli (reflect: the element matrix is reflection-symmetric;
-// the product then runs element by element in the Walsh basis from Cw = W^T Chat_0 W / 64, rows (3 k + a),
-// columns (3 k' + c), W[l][k] = prod over the axes a in k of the side of node l along a; otherwise from Chat)
+// constants of the sum-factorised level-1 rows (see l1_row_sep): mu k_p, (lambda + mu) k_p for k_p = the scale of I_pp,
+// mu k_pq for the pairs xy, xz, yz, lambda / mu
+struct L1Coef {
+    double mu[3], lm[3], cm[3], ratio;
+};
+// of an isotropic material on fine elements of size h
+inline L1Coef l1_coef_of(double young, double nu, const double h[3]) {
+    const double lam = young * nu / ((1 + nu) * (1 - 2 * nu)), mu = young / (2 * (1 + nu));
+    const double H[3] = {2 * h[0], 2 * h[1], 2 * h[2]};
+    L1Coef c;
+    for (int p = 0; p < 3; ++p) {
+        // I_pp = int phi' phi' (D / 2) times two int phi phi (M / 12 each); I_pq = int phi' phi (G / 8, T / 8) times M / 12
+        const double k = H[(p + 1) % 3] * H[(p + 2) % 3] / H[p] / 288, kc = H[2 - p] / 768;
+        c.mu[p] = mu * k;
+        c.lm[p] = (lam + mu) * k;
+        c.cm[p] = mu * kc;
+    }
+    c.ratio = lam / mu;
+    return c;
+}
+// level-1 operator on the fly from the fine moduli (reflect: the element matrix is that of an isotropic box element,
+// whose rows are formed by sum factorisation from `sep`; otherwise from Chat)
 template <typename T>
-void launch_l1_apply(const Grid &gc, const Grid &gf, const T *Chat, const T *Cw, const T *Ef, const T *u, T *y,
+void launch_l1_apply(const Grid &gc, const Grid &gf, const T *Chat, const L1Coef &sep, const T *Ef, const T *u, T *y,
                      const T *b, const uint8_t *dmask, int mode, bool reflect, hipStream_t s);
 // level-1 operator on the fly with the matrix cores (full Chat, any element matrix)
 template <typename T>
@@ -189,8 +208,8 @@ template <typename T>
 void launch_fine_gs(const Grid &g, const T *K0, const T *E, T *u, const T *b, const uint8_t *dmask, int color,
                     int forward, hipStream_t s);
 template <typename T>
-void launch_l1_gs(const Grid &gc, const Grid &gf, const T *Chat, const T *Ef, T *u, const T *b, const uint8_t *dmask,
-                  int color, int forward, bool reflect, hipStream_t s);
+void launch_l1_gs(const Grid &gc, const Grid &gf, const T *Chat, const L1Coef &sep, const T *Ef, T *u, const T *b,
+                  const uint8_t *dmask, int color, int forward, bool reflect, hipStream_t s);
 template <typename T>
 void launch_block_gs(const Grid &g, const T *blocks, T *u, const T *b, const uint8_t *dmask, int color, int forward,
                      hipStream_t s);

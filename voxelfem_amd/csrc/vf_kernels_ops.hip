@@ -9,6 +9,7 @@
 #include "vf_internal.hpp"
 
 #include <climits>
+#include <type_traits>
 
 namespace vf {
 namespace {
@@ -273,256 +274,6 @@ __global__ void __launch_bounds__(TPB) k_l1_gs(Grid gc, Grid gf, const T *__rest
     gs_update(u, N, n, bms, M, dm, forward);
 }
 
-// ---- level-1 K u element by element in the Walsh basis (reflection-symmetric element matrix).
-// With the Walsh basis W[l, k] = prod_{axes a in k} s_a(l) (s_a(l) = +-1 the side of local node l along a,
-// per displacement component), the child matrices Chat_fi = R_fi Chat_0 R_fi (R_fi: reflection across the
-// axes of fi, which permutes the nodes and flips the reflected displacement components) become sign flips
-// of Chat_0 in that basis, so the coarse element matrix sum_fi E_fi Chat_fi reads
-//   (W^T K_E W)[(k, a), (k', c)] = Cw[(k, a), (k', c)] Ehat[k ^ k' ^ e_a ^ e_c],
-//   Cw = W^T Chat_0 W,  Ehat[d] = sum_fi (-1)^popcount(d & fi) E_fi,  e_a = the bit of axis a,
-// and K_E u_E = W (Cw o Ehat) W^T u_E / 64 costs about 800 operations for all 24 outputs instead of
-// 8 x 576 for the child products (W W^T = 8 I; the 1/64 is folded into the table Cw).
-// A workgroup owns a tile of WX x WY x WZ nodes, evaluates every element touching it into LDS and sums
-// each owned node's eight element contributions in a fixed order (no atomics: deterministic).
-constexpr int WX = 4, WY = 8, WZ = 8, WNT = WX * WY * WZ;
-constexpr int WEX = WX + 1, WEY = WY + 1, WEZ = WZ + 1, WNE = WEX * WEY * WEZ;
-static_assert(WNT == TPB, "one owned node per work-item");
-
-// v: the element's nodal values [l][a] on entry, K_E v on exit
-template <typename T>
-__device__ __forceinline__ void l1_walsh_element(const T *__restrict__ Cw, const T Ef8[8], T v[8][3]) {
-    T Eh[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) Eh[i] = Ef8[i];
-    // Ehat = H E (H[d][fi] = (-1)^popcount(d & fi)), and w = W^T v, one axis at a time
-#pragma unroll
-    for (int bit = 4; bit >= 1; bit >>= 1)
-#pragma unroll
-        for (int lo = 0; lo < 8; ++lo) {
-            if (lo & bit) continue;
-            const int hi = lo | bit;
-            const T e0 = Eh[lo], e1 = Eh[hi];
-            Eh[lo] = e0 + e1;
-            Eh[hi] = e0 - e1;
-#pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                const T x0 = v[lo][a], x1 = v[hi][a];
-                v[lo][a] = x0 + x1;
-                v[hi][a] = x1 - x0;
-            }
-        }
-    // out[k][a] = sum_d Ehat[d] sum_c Cw[(k, a), (k', c)] w[k'][c] with k' = k ^ d ^ e_a ^ e_c; rows and
-    // columns of the constant mode k = 0 vanish (rigid translations)
-    T out[8][3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a) out[0][a] = T(0);
-#pragma unroll
-    for (int k = 1; k < 8; ++k)
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            T acc = T(0);
-#pragma unroll
-            for (int d = 0; d < 8; ++d) {
-                T inner = T(0);
-                bool any = false;
-#pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    const int kp = k ^ d ^ (4 >> a) ^ (4 >> c);
-                    if (kp == 0) continue;
-                    inner += Cw[(3 * k + a) * 24 + 3 * kp + c] * v[kp][c];
-                    any = true;
-                }
-                if (any) acc += Eh[d] * inner;
-            }
-            out[k][a] = acc;
-        }
-    // back to the nodes: v = W out
-#pragma unroll
-    for (int bit = 4; bit >= 1; bit >>= 1)
-#pragma unroll
-        for (int lo = 0; lo < 8; ++lo) {
-            if (lo & bit) continue;
-            const int hi = lo | bit;
-#pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                const T x0 = out[lo][a], x1 = out[hi][a];
-                out[lo][a] = x0 - x1;
-                out[hi][a] = x0 + x1;
-            }
-        }
-#pragma unroll
-    for (int l = 0; l < 8; ++l)
-#pragma unroll
-        for (int a = 0; a < 3; ++a) v[l][a] = out[l][a];
-}
-
-// y (mode) K u over the nodes of rows below ydet (detached rows are left to the launcher); grid: one
-// workgroup per node tile
-template <typename T, int MODE>
-__global__ void __launch_bounds__(TPB) k_l1_apply_w(Grid gc, Grid gf, const T *__restrict__ Cw,
-                                                    const T *__restrict__ Ef, const T *__restrict__ u,
-                                                    T *__restrict__ y, const T *__restrict__ b,
-                                                    const uint8_t *__restrict__ dmask, int ntY, int ntZ) {
-    __shared__ T sY[WNE * 24];
-    const int N = gc.nnodes, sx = gc.nn[1] * gc.nn[2], sy = gc.nn[2];
-    const int fz = gf.ne[2], fyz = gf.ne[1] * gf.ne[2];
-    const int tz = blockIdx.x % ntZ, r0 = blockIdx.x / ntZ, ty = r0 % ntY, tx = r0 / ntY;
-    const int x0 = tx * WX, y0 = ty * WY, z0 = tz * WZ;
-    const int t = threadIdx.x;
-    for (int el = t; el < WNE; el += TPB) {
-        const int lx = el / (WEY * WEZ), rr = el - lx * WEY * WEZ, ly = rr / WEZ, lz = rr - ly * WEZ;
-        const int ex = x0 - 1 + lx, ey = y0 - 1 + ly, ez = z0 - 1 + lz;
-        T v[8][3];
-        if ((unsigned)ex < (unsigned)gc.ne[0] && (unsigned)ey < (unsigned)gc.ne[1] && (unsigned)ez < (unsigned)gc.ne[2]) {
-            const int n0 = (ex * gc.nn[1] + ey) * gc.nn[2] + ez;
-            T Ef8[8];
-            const int fb = eidx(gf, 2 * ex, 2 * ey, 2 * ez);
-#pragma unroll
-            for (int l = 0; l < 8; ++l) {
-                const int nm = n0 + ((l >> 2) & 1) * sx + ((l >> 1) & 1) * sy + (l & 1);
-#pragma unroll
-                for (int a = 0; a < 3; ++a) v[l][a] = u[(size_t)a * N + nm];
-                Ef8[l] = Ef[fb + ((l >> 2) & 1) * fyz + ((l >> 1) & 1) * fz + (l & 1)];
-            }
-            l1_walsh_element(Cw, Ef8, v);
-        } else {
-#pragma unroll
-            for (int l = 0; l < 8; ++l)
-#pragma unroll
-                for (int a = 0; a < 3; ++a) v[l][a] = T(0);
-        }
-#pragma unroll
-        for (int l = 0; l < 8; ++l)
-#pragma unroll
-            for (int a = 0; a < 3; ++a) sY[el * 24 + 3 * l + a] = v[l][a];
-    }
-    __syncthreads();
-    const int ox = t / (WY * WZ), orr = t - ox * WY * WZ, oy = orr / WZ, oz = orr - oy * WZ;
-    const int ix = x0 + ox, iy = y0 + oy, iz = z0 + oz;
-    if (ix >= gc.nn[0] || iy >= gc.ydet || iz >= gc.nn[2]) return;
-    T f[3] = {0, 0, 0};
-#pragma unroll
-    for (int l = 0; l < 8; ++l) {
-        // the element with this node at local corner l: local element coordinates (o + 1 - bit)
-        const int el = ((ox + 1 - ((l >> 2) & 1)) * WEY + (oy + 1 - ((l >> 1) & 1))) * WEZ + (oz + 1 - (l & 1));
-#pragma unroll
-        for (int a = 0; a < 3; ++a) f[a] += sY[el * 24 + 3 * l + a];
-    }
-    const int n = (ix * gc.nn[1] + iy) * gc.nn[2] + iz;
-    store_out(y, b, N, n, f, MODE, dmask ? dmask[n] : uint8_t(0));
-}
-
-// Level-1 node row from the fine moduli when the element matrix is reflection-symmetric (box element,
-// orthotropic tensor): Chat_fi[(l, a), (m, c)] = S_fi(a) S_fi(c) Chat_0[(l ^ fi, a), (m ^ fi, c)] with
-// S_fi(a) = -1 iff fi has the bit of axis a set. With g = ln ^ fi and m' = m ^ fi the row of the centre
-// node (local index ln = e in element e) reads
-//   f[a] = sum_g sum_e E_{e, e^g} S(a) sum_{m', c} Chat_0[(g, a), (m', c)] S(c) u_{e, m' ^ e ^ g, c},
-// so each Chat_0 entry (a uniform, scalar operand) serves the eight elements in turn, the scalar working set
-// is one child's 24 x 24 matrix, and the signs are free source negations. Absent elements read zero moduli.
-// The row is split over two work-items: work-item h of a pair takes the four elements with x bit i = h.
-// Its element loop stays unrolled over (j, k); the runtime x bit is folded away by loading the element's
-// node values in x-mirrored order when h = 1 (node m' holds local node m' ^ 4h, x component negated), so
-// Chat_0 rows, register indices and signs stay compile-time, and the remaining runtime sign (-1)^h is
-// applied once to the x-row of f and the x-off-diagonal entries of M. The pair sums its halves with one
-// lane exchange: twice the work-items per colour and half the work each, so a colour's launch has twice as
-// many waves in flight (the smoother's launches cover one colour, an eighth of the nodes, each).
-template <typename T, bool WANT_M>
-__device__ __forceinline__ void l1_row_refl_half(const Grid &gc, const Grid &gf, const T *__restrict__ C0,
-                                                 const T *__restrict__ Ef, const T *__restrict__ u, int ix, int iy,
-                                                 int iz, int h, T f[3], T M[9]) {
-    const int N = gc.nnodes, sx = gc.nn[1] * gc.nn[2], sy = gc.nn[2];
-    const int fz = gf.ne[2], fyz = gf.ne[1] * gf.ne[2];
-    const int n = (ix * gc.nn[1] + iy) * gc.nn[2] + iz;
-    const int sxh = h ? -sx : sx;
-    const int fyzA = h ? fyz : 0, fyzB = h ? 0 : fyz;  // x offset of a child whose reflected x bit is 0 / 1
-    const T hs = h ? T(-1) : T(1);
-    const int ex = ix - h;
-    const bool xin = (unsigned)ex < (unsigned)gc.ne[0];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const int j = (e >> 1) & 1, k = e & 1;
-        const int ey = iy - j, ez = iz - k;
-        const bool ok = xin && (unsigned)ey < (unsigned)gc.ne[1] && (unsigned)ez < (unsigned)gc.ne[2];
-        if (!ok) continue;
-        T ue[8][3];
-#pragma unroll
-        for (int m = 0; m < 8; ++m) {
-            // local node m ^ 4h of the element at x offset (m_x - h) = (m >> 2 & 1) * (h ? -1 : 1)
-            const int nm = n + ((m >> 2) & 1) * sxh + (((m >> 1) & 1) - j) * sy + ((m & 1) - k);
-            ue[m][0] = hs * u[nm];
-            ue[m][1] = u[(size_t)N + nm];
-            ue[m][2] = u[(size_t)2 * N + nm];
-        }
-        const int fb = eidx(gf, 2 * ex, 2 * ey, 2 * ez);
-#pragma unroll
-        for (int g = 0; g < 8; ++g) {
-            const int fis = (g & 4) | ((e ^ g) & 3);  // the child index with its x bit taken from g
-            const T Efi = Ef[fb + ((g >> 2) & 1 ? fyzB : fyzA) + ((fis >> 1) & 1) * fz + (fis & 1)];
-            T t[3] = {0, 0, 0};
-#pragma unroll
-            for (int mp = 0; mp < 8; ++mp)
-#pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    const T uv = ((fis >> (2 - c)) & 1) ? -ue[mp ^ fis][c] : ue[mp ^ fis][c];
-#pragma unroll
-                    for (int a = 0; a < 3; ++a) t[a] += C0[(3 * g + a) * 24 + 3 * mp + c] * uv;
-                }
-#pragma unroll
-            for (int a = 0; a < 3; ++a) f[a] += (((fis >> (2 - a)) & 1) ? -Efi : Efi) * t[a];
-            if (WANT_M) {
-#pragma unroll
-                for (int a = 0; a < 3; ++a)
-#pragma unroll
-                    for (int c = 0; c < 3; ++c) {
-                        const bool neg = (bool)((fis >> (2 - a)) & 1) != (bool)((fis >> (2 - c)) & 1);
-                        M[3 * a + c] += (neg ? -Efi : Efi) * C0[(3 * g + a) * 24 + 3 * g + c];
-                    }
-            }
-        }
-    }
-    f[0] *= hs;
-    if (WANT_M) {
-        M[1] *= hs;
-        M[2] *= hs;
-        M[3] *= hs;
-        M[6] *= hs;
-    }
-#pragma unroll
-    for (int a = 0; a < 3; ++a) f[a] += __shfl_xor(f[a], 1, 64);
-    if (WANT_M)
-#pragma unroll
-        for (int q = 0; q < 9; ++q) M[q] += __shfl_xor(M[q], 1, 64);
-}
-
-template <typename T>
-__global__ void __launch_bounds__(TPB) k_l1_gs_r2(Grid gc, Grid gf, const T *__restrict__ C0,
-                                                  const T *__restrict__ Ef, T *__restrict__ u, const T *__restrict__ b,
-                                                  const uint8_t *__restrict__ dmask, int cx, int cy, int cz,
-                                                  int forward) {
-    const int mx = (gc.nn[0] - cx + 1) / 2, my = (gc.ydet - cy + 1) / 2, mz = (gc.nn[2] - cz + 1) / 2;
-    const int tt = blockIdx.x * TPB + threadIdx.x, t = tt >> 1, h = tt & 1;
-    if (t >= mx * my * mz) return;  // both work-items of a pair
-    const int jx = t / (my * mz), r = t - jx * my * mz, jy = r / mz, jz = r - jy * mz;
-    const int ix = 2 * jx + cx, iy = 2 * jy + cy, iz = 2 * jz + cz;
-    const int N = gc.nnodes, n = (ix * gc.nn[1] + iy) * gc.nn[2] + iz;
-    const uint8_t dm = dmask ? dmask[n] : uint8_t(0);
-    if (dm == 7) return;  // both work-items of a pair
-    T f[3] = {0, 0, 0};
-    T M[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    l1_row_refl_half<T, true>(gc, gf, C0, Ef, u, ix, iy, iz, h, f, M);
-    if (h) return;
-    const T bms[3] = {b[n] - f[0], b[N + n] - f[1], b[2 * N + n] - f[2]};
-    gs_update(u, N, n, bms, M, dm, forward);
-}
-
-// ------------------------------------------------------------------ assembled block rows
-// One node is worked on by the sixteen lanes of one DPP row: lane p holds neighbour slots p and p + 16 (27 in all), so
-// a node's 243 block entries and 81 neighbour values are requested at once, in one round of loads, and the row is
-// summed by four DPP exchanges without LDS. A colour pass over a small level is bound by that one memory round
-// instead of the three dependent rounds (and 81 loads per work-item) of four work-items per node; over a large level
-// it streams the interleaved rows (105 x 57 x 49 nodes in FP64: 20 us per colour, 3.6 TB/s). Time per colour, before
-// and after, averaged over the block levels of a hierarchy: 64 x 32 x 32 FP64 10.4 -> 4.3 us, 176 x 88 x 72 FP64
-// 13.6 -> 7.5 us, 208 x 112 x 96 FP64 16.2 -> 9.9 us, 384 x 192 x 192 FP32 9.5 -> 7.6 us.
 template <int CTRL>
 __device__ __forceinline__ float dpp_get(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
@@ -533,6 +284,257 @@ __device__ __forceinline__ double dpp_get(double v) {
     const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
     return __hiloint2double(hi, lo);
 }
+// Level-1 node row from the fine moduli of an isotropic box element, by sum factorisation. The element matrix is a sum of
+// products of 1D integrals over the axes, and so is its Galerkin coarsening: with I_pq(o) = sum over the 4 x 4 x 4 fine
+// elements around the node of E times the integral of d_p phi_0 d_q phi_o over the element (phi the coarse shape
+// functions of the node and of its neighbour at offset o), the 3 x 3 block of neighbour o is
+//   B_cc = mu (I_xx + I_yy + I_zz) + (lambda + mu) I_cc,   B_cd = lambda I_cd + mu I_dc,
+// and I_pq contracts E axis by axis with one of four functionals of the four fine cells along the axis: M (phi phi),
+// D (phi' phi'), G (phi_0' phi_o), T (phi_0 phi_o'). Up to constant factors (kept in L1Coef), for cells c0 c1 | c2 c3:
+//   o = -1: M = c0 + c1, D = -M, G = 3 c0 + c1, T = -(c0 + 3 c1);   o = +1: mirrored, G and T of opposite sign;
+//   o = 0: M = (c0 + 7 c1 + 7 c2 + c3) / 2, D = c0 + c1 + c2 + c3, G = T = c0 + 3 c1 - 3 c2 - c3.
+// That is about 840 operations per half row, in place of 2592 for the eight children's dense rows.
+// A node has two work-items, one per side along x (h = 0 low, h = 1 high): each contracts its side's 2 x 4 x 4 cells with
+// the neighbours of the outer and the centre plane, in x-mirrored order when h = 1 (which negates the x component of u and
+// of the row), and the two rows are added with a lane exchange. The halves of a wavefront take one side each, so that
+// neighbouring lanes read neighbouring nodes (interleaved lanes: residual 215 instead of 194 us in FP64).
+// Bound by the latency of three rounds of moduli and, on the largest level, by reading the moduli once per colour; the
+// nine sums and one layer's contractions fit three (FP64) and five (FP32) wavefronts per SIMD. Level 1 of 384 x 192 x 192:
+// a sweep of eight colours 665 -> 537 us in FP64 and 420 -> 253 us in FP32, the residual 326 -> 194 and 98 -> 103 us; of
+// 256 x 128 x 128: 303 -> 193 and 196 -> 100 us, 110 -> 58 and 38 -> 36 us (before: dense child rows with two work-items
+// per node, and the residual element by element in the Walsh basis).
+template <typename T>
+struct L1CoefT {
+    T mu[3], lm[3], cm[3], r;
+};
+template <typename T, int DL>
+struct Ax4 {  // functionals of four cells at offset DL
+    static __device__ __forceinline__ T M(T a, T b, T c, T d) {
+        return DL < 0 ? a + b : DL > 0 ? c + d : T(0.5) * (a + d) + T(3.5) * (b + c);
+    }
+    static __device__ __forceinline__ T D(T a, T b, T c, T d) { return DL < 0 ? -(a + b) : DL > 0 ? -(c + d) : (a + b) + (c + d); }
+    static __device__ __forceinline__ T G(T a, T b, T c, T d) {
+        return DL < 0 ? T(3) * a + b : DL > 0 ? -(c + T(3) * d) : (a + T(3) * b) - (T(3) * c + d);
+    }
+    static __device__ __forceinline__ T T_(T a, T b, T c, T d) {
+        return DL < 0 ? -(a + T(3) * b) : DL > 0 ? T(3) * c + d : (a + T(3) * b) - (T(3) * c + d);
+    }
+};
+// one offset's weights I, its neighbour's values u, and the sums they are added to: V[c] += B_cc u_c, and without the
+// scale of their pair of axes Q[xy, yx, xz, zx, yz, zy] += (I_dc + lambda / mu I_cd) u_d
+template <typename T>
+struct L1Sums {
+    T V[3], Q[6];
+};
+template <typename T>
+__device__ __forceinline__ void l1_offset(const L1CoefT<T> &k, T xx, T yy, T zz, T xy, T yx, T xz, T zx, T yz, T zy,
+                                          const T u[3], L1Sums<T> &s) {
+    const T S = k.mu[0] * xx + k.mu[1] * yy + k.mu[2] * zz;
+    s.V[0] += (S + k.lm[0] * xx) * u[0];
+    s.V[1] += (S + k.lm[1] * yy) * u[1];
+    s.V[2] += (S + k.lm[2] * zz) * u[2];
+    s.Q[0] += (yx + k.r * xy) * u[1];
+    s.Q[1] += (xy + k.r * yx) * u[0];
+    s.Q[2] += (zx + k.r * xz) * u[2];
+    s.Q[3] += (xz + k.r * zx) * u[0];
+    s.Q[4] += (zy + k.r * yz) * u[2];
+    s.Q[5] += (yz + k.r * zy) * u[1];
+}
+// the half row's part of the offsets (., DY, DZ): Z fields Z*[x][y] of the cells contracted along z
+template <typename T, int DY, int DZ, bool WANT_M>
+__device__ __forceinline__ void l1_line(const L1CoefT<T> &k, const T (&ZM)[2][4], const T (&ZD)[2][4], const T (&ZG)[2][4],
+                                        const T (&ZT)[2][4], const T uo[3], const T uc[3], L1Sums<T> &s, T M[6]) {
+    using Y = Ax4<T, DY>;
+    T mm[2], dm[2], gm[2], tm[2], md[2], mt[2], gt[2], mg[2], tg[2];
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+        mm[x] = Y::M(ZM[x][0], ZM[x][1], ZM[x][2], ZM[x][3]);
+        dm[x] = DY ? -mm[x] : Y::D(ZM[x][0], ZM[x][1], ZM[x][2], ZM[x][3]);
+        gm[x] = Y::G(ZM[x][0], ZM[x][1], ZM[x][2], ZM[x][3]);
+        tm[x] = DY ? Y::T_(ZM[x][0], ZM[x][1], ZM[x][2], ZM[x][3]) : gm[x];
+        md[x] = DZ ? -mm[x] : Y::M(ZD[x][0], ZD[x][1], ZD[x][2], ZD[x][3]);
+        mt[x] = Y::M(ZT[x][0], ZT[x][1], ZT[x][2], ZT[x][3]);
+        gt[x] = Y::G(ZT[x][0], ZT[x][1], ZT[x][2], ZT[x][3]);
+        mg[x] = DZ ? Y::M(ZG[x][0], ZG[x][1], ZG[x][2], ZG[x][3]) : mt[x];
+        tg[x] = Y::T_(ZG[x][0], ZG[x][1], ZG[x][2], ZG[x][3]);
+    }
+    // x: cells o (outer), i (inner)
+    auto mo = [](const T *w) { return w[0] + w[1]; };               // outer plane: M, -D
+    auto go = [](const T *w) { return T(3) * w[0] + w[1]; };        // G
+    auto t3 = [](const T *w) { return w[0] + T(3) * w[1]; };        // -T; centre plane: G, T
+    auto mc = [](const T *w) { return T(0.5) * w[0] + T(3.5) * w[1]; };  // centre plane: M (D as mo)
+    l1_offset(k, -mo(mm), mo(dm), mo(md), go(tm), -t3(gm), go(mt), -t3(mg), mo(gt), mo(tg), uo, s);
+    const T xx = mo(mm), yy = mc(dm), zz = mc(md), xy = t3(tm), yx = t3(gm), xz = t3(mt), zx = t3(mg), yz = mc(gt), zy = mc(tg);
+    l1_offset(k, xx, yy, zz, xy, yx, xz, zx, yz, zy, uc, s);
+    if (WANT_M && DY == 0 && DZ == 0) {
+        const T S = k.mu[0] * xx + k.mu[1] * yy + k.mu[2] * zz;
+        M[0] = S + k.lm[0] * xx;
+        M[1] = S + k.lm[1] * yy;
+        M[2] = S + k.lm[2] * zz;
+        M[3] = k.cm[0] * (T(1) + k.r) * xy;  // G = T at the node itself
+        M[4] = k.cm[1] * (T(1) + k.r) * xz;
+        M[5] = k.cm[2] * (T(1) + k.r) * yz;
+    }
+}
+// keeps what is derived from `at` behind the sums so far: the compiler would otherwise request every layer's operands
+// first and hold them all
+template <typename T>
+__device__ __forceinline__ void l1_pin(unsigned &at, L1Sums<T> &s) {
+    asm volatile("" : "+v"(at), "+v"(s.V[0]), "+v"(s.V[1]), "+v"(s.V[2]), "+v"(s.Q[0]), "+v"(s.Q[1]), "+v"(s.Q[2]),
+                 "+v"(s.Q[3]), "+v"(s.Q[4]), "+v"(s.Q[5]));
+}
+template <typename T>
+struct Vec2;
+template <>
+struct Vec2<float> { using t = float2; };
+template <>
+struct Vec2<double> { using t = double2; };
+
+template <typename T, bool WANT_M>
+__device__ __forceinline__ void l1_row_sep(const Grid &gc, const Grid &gf, const L1CoefT<T> &k, const T *__restrict__ Ef,
+                                           const T *__restrict__ u, int ix, int iy, int iz, int h, T f[3], T M[6]) {
+    const int N = gc.nnodes, sy = gc.nn[2], sx = gc.nn[1] * sy;
+    const int fz = gf.ne[2], fyz = gf.ne[1] * gf.ne[2];
+    const int n = ix * sx + iy * sy + iz;
+    const T hs = h ? T(-1) : T(1);
+    const bool xin = h ? ix < gc.ne[0] : ix > 0;
+    const int fx0 = h ? 2 * ix + 1 : 2 * ix - 2, fxs = h ? -fyz : fyz;
+    L1Sums<T> s;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) s.V[c] = s.Q[c] = s.Q[3 + c] = T(0);
+    const int ox = h ? sx : -sx;
+    const T *__restrict__ u1 = u + N, *__restrict__ u2 = u + (size_t)2 * N;
+    // the six values of a line (fixed offsets along y and z) of the two planes, requested one line ahead; a neighbour
+    // outside the grid has weight zero and reads the node itself
+    T nxt[6];
+    auto request = [&](unsigned nn, int dy, int dz) {
+        const bool in = (unsigned)(iy + dy) < (unsigned)gc.nn[1] && (unsigned)(iz + dz) < (unsigned)gc.nn[2];
+        const unsigned mc = in ? nn + dy * sy + dz : nn, mo = xin ? mc + ox : mc;
+        nxt[0] = u[mo];
+        nxt[1] = u1[mo];
+        nxt[2] = u2[mo];
+        nxt[3] = u[mc];
+        nxt[4] = u1[mc];
+        nxt[5] = u2[mc];
+    };
+    request(n, -1, -1);
+    auto line = [&](auto DYc, auto DZc, const T(&ZM)[2][4], const T(&ZD)[2][4], const T(&ZG)[2][4], const T(&ZT)[2][4]) {
+        constexpr int DY = decltype(DYc)::value, DZ = decltype(DZc)::value;
+        T uo[3] = {hs * nxt[0], nxt[1], nxt[2]}, uc[3] = {hs * nxt[3], nxt[4], nxt[5]};
+        if (DY < 1 || DZ < 1) {
+            unsigned nn = n;
+            l1_pin(nn, s);
+            request(nn, DY < 1 ? DY + 1 : -1, DY < 1 ? DZ : DZ + 1);
+        }
+        l1_line<T, DY, DZ, WANT_M>(k, ZM, ZD, ZG, ZT, uo, uc, s, M);
+    };
+    auto layer = [&](auto DZc) {
+        constexpr int DZ = decltype(DZc)::value;
+        using Z = Ax4<T, DZ>;
+        // cells E[x: outer, inner][y][z], zero outside the grid; read again for each layer, since holding
+        // them would cost the registers of a wavefront per SIMD
+        unsigned eb = (unsigned)(fx0 * fyz);
+        l1_pin(eb, s);
+        T E[2][4][4];
+#pragma unroll
+        for (int zz = 0; zz < 2; ++zz)
+#pragma unroll
+            for (int yy = 0; yy < 2; ++yy) {
+                const int ey = iy - 1 + yy, ez = iz - 1 + zz;
+                const bool ok = xin && (unsigned)ey < (unsigned)gc.ne[1] && (unsigned)ez < (unsigned)gc.ne[2];
+                const unsigned at = ok ? eb + (unsigned)(2 * ey * fz + 2 * ez) : 0u;  // element counts fit 31 bits
+                if ((DZ < 0 && zz == 1) || (DZ > 0 && zz == 0)) continue;  // only the cells shared with the neighbour
+#pragma unroll
+                for (int x = 0; x < 2; ++x)
+#pragma unroll
+                    for (int y = 0; y < 2; ++y) {
+                        // rows of fine elements are even in number and length, so a pair along z is aligned
+                        const auto v = *reinterpret_cast<const typename Vec2<T>::t *>(Ef + (at + (ok ? (unsigned)(x * fxs + y * fz) : 0u)));
+                        E[x][2 * yy + y][2 * zz] = ok ? v.x : T(0);
+                        E[x][2 * yy + y][2 * zz + 1] = ok ? v.y : T(0);
+                    }
+            }
+        T ZM[2][4], ZD[2][4], ZG[2][4], ZT[2][4];
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int y = 0; y < 4; ++y) {
+                T *e = E[x][y];
+                if (DZ > 0) e[0] = e[1] = T(0);
+                if (DZ < 0) e[2] = e[3] = T(0);
+                ZM[x][y] = Z::M(e[0], e[1], e[2], e[3]);
+                ZD[x][y] = Z::D(e[0], e[1], e[2], e[3]);
+                ZG[x][y] = Z::G(e[0], e[1], e[2], e[3]);
+                ZT[x][y] = DZ ? Z::T_(e[0], e[1], e[2], e[3]) : ZG[x][y];
+            }
+        line(std::integral_constant<int, -1>(), DZc, ZM, ZD, ZG, ZT);
+        __builtin_amdgcn_sched_barrier(0);
+        line(std::integral_constant<int, 0>(), DZc, ZM, ZD, ZG, ZT);
+        __builtin_amdgcn_sched_barrier(0);
+        line(std::integral_constant<int, 1>(), DZc, ZM, ZD, ZG, ZT);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    layer(std::integral_constant<int, -1>());
+    layer(std::integral_constant<int, 0>());
+    layer(std::integral_constant<int, 1>());
+    f[0] = hs * (s.V[0] + k.cm[0] * s.Q[0] + k.cm[1] * s.Q[2]);
+    f[1] = s.V[1] + k.cm[0] * s.Q[1] + k.cm[2] * s.Q[4];
+    f[2] = s.V[2] + k.cm[1] * s.Q[3] + k.cm[2] * s.Q[5];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) f[a] += __shfl_xor(f[a], 32, 64);  // the other work-item of the pair
+    if (WANT_M) {
+        M[3] *= hs;
+        M[4] *= hs;
+#pragma unroll
+        for (int q = 0; q < 6; ++q) M[q] += __shfl_xor(M[q], 32, 64);
+    }
+}
+
+template <typename T>
+__global__ void __launch_bounds__(TPB, sizeof(T) == 8 ? 2 : 4) k_l1_gs_sep(Grid gc, Grid gf, L1CoefT<T> k, const T *__restrict__ Ef,
+                                                   T *__restrict__ u, const T *__restrict__ b,
+                                                   const uint8_t *__restrict__ dmask, int cx, int cy, int cz, int forward) {
+    const int mx = (gc.nn[0] - cx + 1) / 2, my = (gc.ydet - cy + 1) / 2, mz = (gc.nn[2] - cz + 1) / 2;
+    const int t = xcd_remap(blockIdx.x, gridDim.x) * (TPB / 2) + threadIdx.x / 64 * 32 + threadIdx.x % 32,
+              h = threadIdx.x >> 5 & 1;
+    if (t >= mx * my * mz) return;  // both work-items of a pair
+    const int jx = t / (my * mz), r = t - jx * my * mz, jy = r / mz, jz = r - jy * mz;
+    const int ix = 2 * jx + cx, iy = 2 * jy + cy, iz = 2 * jz + cz;
+    const int N = gc.nnodes, n = (ix * gc.nn[1] + iy) * gc.nn[2] + iz;
+    const uint8_t dm = dmask ? dmask[n] : uint8_t(0);
+    if (dm == 7) return;  // both work-items of a pair
+    T f[3], S[6];
+    l1_row_sep<T, true>(gc, gf, k, Ef, u, ix, iy, iz, h, f, S);
+    if (h) return;
+    const T bms[3] = {b[n] - f[0], b[N + n] - f[1], b[2 * N + n] - f[2]};
+    const T M[9] = {S[0], S[3], S[4], S[3], S[1], S[5], S[4], S[5], S[2]};
+    gs_update(u, N, n, bms, M, dm, forward);
+}
+
+// y (mode) K u over the nodes of rows below ydet, two work-items per node
+template <typename T, int MODE>
+__global__ void __launch_bounds__(TPB, sizeof(T) == 8 ? 2 : 4) k_l1_apply_sep(Grid gc, Grid gf, L1CoefT<T> k, const T *__restrict__ Ef,
+                                                      const T *__restrict__ u, T *__restrict__ y, const T *__restrict__ b,
+                                                      const uint8_t *__restrict__ dmask) {
+    const int nz = gc.nn[2], slab = gc.ydet * nz;
+    const int t = xcd_remap(blockIdx.x, gridDim.x) * (TPB / 2) + threadIdx.x / 64 * 32 + threadIdx.x % 32,
+              h = threadIdx.x >> 5 & 1;
+    if (t >= gc.nn[0] * slab) return;
+    const int ix = t / slab, r = t - ix * slab, iy = r / nz, iz = r - iy * nz;
+    const int n = (ix * gc.nn[1] + iy) * nz + iz;
+    T f[3], M[6];
+    l1_row_sep<T, false>(gc, gf, k, Ef, u, ix, iy, iz, h, f, M);
+    if (!h) store_out(y, b, gc.nnodes, n, f, MODE, dmask ? dmask[n] : uint8_t(0));
+}
+
+// ------------------------------------------------------------------ assembled block rows
+// One node is worked on by the sixteen lanes of one DPP row: lane p holds neighbour slots p and p + 16 (27 in all), so
+// a node's 243 block entries and 81 neighbour values are requested at once, in one round of loads, and the row is
+// summed by four DPP exchanges without LDS. A colour pass over a small level is bound by that one memory round
+// instead of the three dependent rounds (and 81 loads per work-item) of four work-items per node; over a large level
+// it streams the interleaved rows (105 x 57 x 49 nodes in FP64: 20 us per colour, 3.6 TB/s). Time per colour, before
+// and after, averaged over the block levels of a hierarchy: 64 x 32 x 32 FP64 10.4 -> 4.3 us, 176 x 88 x 72 FP64
+// 13.6 -> 7.5 us, 208 x 112 x 96 FP64 16.2 -> 9.9 us, 384 x 192 x 192 FP32 9.5 -> 7.6 us.
 // sum over the sixteen lanes of a DPP row, the same in every lane
 template <typename T>
 __device__ __forceinline__ T row16_sum(T v) {
@@ -800,15 +802,23 @@ void launch_fine_apply(const Grid &g, const T *K0, const T *E, const T *u, T *y,
 }
 
 template <typename T>
-void launch_l1_apply(const Grid &gc, const Grid &gf, const T *Chat, const T *Cw, const T *Ef, const T *u, T *y,
+static L1CoefT<T> l1_coef(const L1Coef &c) {
+    L1CoefT<T> r;
+    for (int q = 0; q < 3; ++q) {
+        r.mu[q] = (T)c.mu[q];
+        r.lm[q] = (T)c.lm[q];
+        r.cm[q] = (T)c.cm[q];
+    }
+    r.r = (T)c.ratio;
+    return r;
+}
+
+template <typename T>
+void launch_l1_apply(const Grid &gc, const Grid &gf, const T *Chat, const L1Coef &sep, const T *Ef, const T *u, T *y,
                      const T *b, const uint8_t *dmask, int mode, bool reflect, hipStream_t s) {
     const long count = (long)gc.nn[0] * gc.ydet * gc.nn[2];
     if (count > 0 && reflect) {
-        if (!Cw) throw std::runtime_error("the Walsh-basis level-1 product needs its table");
-        const int ntX = (gc.nn[0] + WX - 1) / WX, ntY = (gc.ydet + WY - 1) / WY, ntZ = (gc.nn[2] + WZ - 1) / WZ;
-        const long tiles = (long)ntX * ntY * ntZ;
-        if (tiles > INT_MAX) throw std::runtime_error("grid too large for the level-1 product");
-        VF_DISPATCH_MODE(k_l1_apply_w, T, mode, dim3((unsigned)tiles), gc, gf, Cw, Ef, u, y, b, dmask, ntY, ntZ);
+        VF_DISPATCH_MODE(k_l1_apply_sep, T, mode, dim3(nblocks(2 * count)), gc, gf, l1_coef<T>(sep), Ef, u, y, b, dmask);
     } else if (count > 0) {
         VF_DISPATCH_MODE(k_l1_apply, T, mode, dim3(nblocks(count)), gc, gf, Chat, Ef, u, y, b, dmask);
     }
@@ -857,14 +867,14 @@ void launch_fine_gs(const Grid &g, const T *K0, const T *E, T *u, const T *b, co
 }
 
 template <typename T>
-void launch_l1_gs(const Grid &gc, const Grid &gf, const T *Chat, const T *Ef, T *u, const T *b, const uint8_t *dmask,
-                  int color, int forward, bool reflect, hipStream_t s) {
+void launch_l1_gs(const Grid &gc, const Grid &gf, const T *Chat, const L1Coef &sep, const T *Ef, T *u, const T *b,
+                  const uint8_t *dmask, int color, int forward, bool reflect, hipStream_t s) {
     const int cx = (color >> 2) & 1, cy = (color >> 1) & 1, cz = color & 1;
     const long count = color_count(gc, cx, cy, cz);
     if (!count) return;
     if (reflect)
-        hipLaunchKernelGGL(k_l1_gs_r2<T>, dim3(nblocks(2 * count)), dim3(TPB), 0, s, gc, gf, Chat, Ef, u, b, dmask, cx,
-                           cy, cz, forward);
+        hipLaunchKernelGGL(k_l1_gs_sep<T>, dim3(nblocks(2 * count)), dim3(TPB), 0, s, gc, gf, l1_coef<T>(sep), Ef, u, b,
+                           dmask, cx, cy, cz, forward);
     else
         hipLaunchKernelGGL(k_l1_gs<T>, dim3(nblocks(count)), dim3(TPB), 0, s, gc, gf, Chat, Ef, u, b, dmask, cx, cy,
                            cz, forward);
@@ -922,15 +932,15 @@ void launch_interpolate(const Grid &gf, const Grid &gc, const T *xc, T *xf, int 
     template void launch_zero_detached<T>(const Grid &, T *, hipStream_t);                                             \
     template void launch_fine_apply<T>(const Grid &, const T *, const T *, const T *, T *, const T *, const uint8_t *,  \
                                        int, hipStream_t);                                                              \
-    template void launch_l1_apply<T>(const Grid &, const Grid &, const T *, const T *, const T *, const T *, T *,      \
+    template void launch_l1_apply<T>(const Grid &, const Grid &, const T *, const L1Coef &, const T *, const T *, T *,    \
                                      const T *, const uint8_t *, int, bool, hipStream_t);                              \
     template void launch_block_apply<T>(const Grid &, const T *, const T *, T *, const T *, const uint8_t *, int,       \
                                         hipStream_t);                                                                  \
     template void launch_elem_apply<T>(const Grid &, const T *, const T *, T *, int, hipStream_t);                     \
     template void launch_fine_gs<T>(const Grid &, const T *, const T *, T *, const T *, const uint8_t *, int, int,      \
                                     hipStream_t);                                                                      \
-    template void launch_l1_gs<T>(const Grid &, const Grid &, const T *, const T *, T *, const T *, const uint8_t *,    \
-                                  int, int, bool, hipStream_t);                                                        \
+    template void launch_l1_gs<T>(const Grid &, const Grid &, const T *, const L1Coef &, const T *, T *, const T *,    \
+                                  const uint8_t *, int, int, bool, hipStream_t);                                                        \
     template void launch_block_gs<T>(const Grid &, const T *, T *, const T *, const uint8_t *, int, int, hipStream_t); \
     template void launch_restrict<T>(const Grid &, const Grid &, const T *, T *, hipStream_t, T *);                   \
     template void launch_interpolate<T>(const Grid &, const Grid &, const T *, T *, int, hipStream_t);
