@@ -38,8 +38,10 @@ def pair(ne, levels, layer=None, seed=0):
 
 
 # level 1 has (ne / 2 + 1) nodes per axis: colour classes of 1 to 45 nodes, with every remainder modulo the four nodes
-# that the block rows interleave and the sixteen that a workgroup holds; with layers masked, rows end inside a class
-@pytest.mark.parametrize("ne,levels,layer", [((4, 4, 4), 2, None), ((8, 4, 4), 2, None), ((8, 12, 4), 2, None),
+# that the block rows interleave and the sixteen that a workgroup holds; with layers masked, rows end inside a class.
+# Tiles of the two-launch sweep are 4 x 12 nodes of a plane: one and several, and a level (5 x 353 x 3) of too many for it
+@pytest.mark.parametrize("ne,levels,layer", [((4, 8, 52), 2, None), ((4, 20, 52), 2, 9), ((8, 704, 4), 2, None),
+                                             ((4, 4, 4), 2, None), ((8, 4, 4), 2, None), ((8, 12, 4), 2, None),
                                              ((16, 8, 12), 2, None), ((4, 12, 20), 2, 5), ((16, 16, 8), 3, 9)])
 def test_block_rows(ne, levels, layer):
     mg, om = pair(ne, levels, layer)

@@ -794,6 +794,11 @@ struct vf_mg {
             launch_fill<T>(n1, b1.data(), T(1), s);
             auto sweep = [&](int form) {
                 launch_fill<T>(n1, u1.data(), T(1e-3), s);
+                if (form == 0 && block_gs_planes(g1)) {
+                    launch_block_gs_plane<T>(g1, blocksp<T>(1), u1.data(), u1.data(), y.data(), b1.data(), dm(1), 0, 1, s);
+                    launch_block_gs_plane<T>(g1, blocksp<T>(1), u1.data(), y.data(), y.data(), b1.data(), dm(1), 1, 1, s);
+                    return;
+                }
                 for (int c = 0; c < 8; ++c) {
                     if (form == 0) launch_block_gs<T>(g1, blocksp<T>(1), u1.data(), b1.data(), dm(1), c, 1, s);
                     else if (form == 1)
@@ -862,13 +867,22 @@ struct vf_mg {
     template <typename T>
     void sweep_to(int l, const T *uin, T *uout, const T *b, bool forward, bool zeroIn = false) {
         const int p0 = forward ? 0 : 1;
+        if (l > 0) {
+            launch_block_gs_plane<T>(lv[l]->g, blocksp<T>(l), uin, uin, uout, b, dm(l), p0, forward, st(), zeroIn ? 3 : 0);
+            launch_block_gs_plane<T>(lv[l]->g, blocksp<T>(l), uin, uout, uout, b, dm(l), 1 - p0, forward, st(),
+                                     zeroIn ? 1 : 0);
+            return;
+        }
         launch_fine_gs_phase<T>(lv[0]->g, Fp<T>(), Ep<T>(), uin, uin, uout, b, dm(0), p0, forward, st(),
                                 zeroIn ? 3 : 0);
         launch_fine_gs_phase<T>(lv[0]->g, Fp<T>(), Ep<T>(), uin, uout, uout, b, dm(0), 1 - p0, forward, st(),
                                 zeroIn ? 1 : 0);
     }
     template <typename T>
-    bool paired(int l) const { return l == 0 && tiled_gs<T>(); }
+    bool paired(int l) const {
+        if (l == 0) return tiled_gs<T>();
+        return l < L && (l > 1 || l1_form(pidx<T>(), 1) == 0) && block_gs_planes(lv[l]->g);
+    }
     template <typename T>
     void smooth(int l, T *u, const T *b, bool forward) {
         if (paired<T>(l)) {

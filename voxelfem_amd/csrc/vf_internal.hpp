@@ -214,6 +214,13 @@ template <typename T>
 void launch_block_gs(const Grid &g, const T *blocks, T *u, const T *b, const uint8_t *dmask, int color, int forward,
                      hipStream_t s);
 
+// One x-parity of a block-row sweep, all four colours in one launch (arguments as launch_fine_gs_phase), and whether a
+// level is small enough for it to be the faster form
+bool block_gs_planes(const Grid &g);
+template <typename T>
+void launch_block_gs_plane(const Grid &g, const T *blocks, const T *uin, const T *unb, T *uout, const T *b,
+                           const uint8_t *dmask, int parity, int forward, hipStream_t s, int zin = 0);
+
 // transfers (MultigridSolver.hh:178-275)
 template <typename T>
 void launch_restrict(const Grid &gf, const Grid &gc, const T *rf, T *rc, hipStream_t s, T *xzero = nullptr);

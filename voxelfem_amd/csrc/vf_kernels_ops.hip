@@ -545,6 +545,9 @@ __device__ __forceinline__ T row16_sum(T v) {
     return v;
 }
 
+// tile and workgroup of the two-launch sweep: 28 of the 32 rows of lanes hold a node at the first colour
+constexpr int BP_TY = 4, BP_TZ = 12, BP_NT = 512, CUS = 256;
+
 constexpr int RL = 16;       // lanes per node
 constexpr int RN16 = TPB / RL;  // nodes per workgroup
 constexpr int DIAG_LANE = 13;   // the lane that holds the node's own slot
@@ -629,6 +632,125 @@ __global__ void __launch_bounds__(TPB) k_block_gs(Grid g, const T *__restrict__ 
     if (p == DIAG_LANE && dm != 7) {
         const T bms[3] = {bn[0] - f[0], bn[1] - f[1], bn[2] - f[2]};
         gs_update(u, N, n, bms, M, dm, forward);
+    }
+}
+
+// One x-parity of the colour sweep in one launch (a sweep is two): the four colours of a parity only see the other
+// parity's planes and each other, so a workgroup takes a (y, z) tile of one plane, holds its values in LDS and applies the
+// four in-plane colours in order, each on the tile grown by the halo that the later colours read ((1,3), (1,2), (0,1),
+// (0,0) nodes in (y, z); the neighbouring tiles recompute it from the same inputs). Sixteen lanes per node as in
+// block_row16, and a node for every row of lanes at each of the four positions: all block rows are requested before the
+// first colour, the off-plane part of the sums is taken as they arrive, and what a colour waits for is only three values
+// from LDS (a lane has at most one slot in the plane: s = 9 .. 17 are lanes 9 .. 15 and 0, 1). Bound by latency: about
+// 3.5 us of launch, one round of loads and four colours, 10 us against 15 for four colour launches. Requested one
+// colour ahead instead of all at once (tiles of 4 x 8): 12 us.
+// uin: the planes of this parity before the sweep, unb: the neighbour planes, uout (!= uin): receives this parity's
+// planes, every node. zin bit 0 / 1: uin / unb is zero.
+template <typename T, int TY, int TZ, int NT, bool FWD>
+__global__ void __launch_bounds__(NT) k_block_gs_plane(Grid g, const T *__restrict__ blocks, const T *__restrict__ uin,
+                                                       const T *__restrict__ unb, T *__restrict__ uout,
+                                                       const T *__restrict__ b, const uint8_t *__restrict__ dmask,
+                                                       int parity, int ntY, int ntZ, int zin) {
+    constexpr int HY = 2, HZ = 4, RY = TY + 2 * HY, RZ = TZ + 2 * HZ, CS = RY * RZ;
+    static_assert(TY % 2 == 0 && TZ % 2 == 0 && (TY / 2 + 1) * (TZ / 2 + 3) <= NT / RL, "one node per row of lanes");
+    __shared__ T su[3 * CS], sb[3 * CS];
+    const int N = g.nnodes, nx = g.nn[0], ny = g.nn[1], nz = g.nn[2];
+    const int ix = parity + 2 * blockIdx.y, tz = blockIdx.x % ntZ, ty = blockIdx.x / ntZ;
+    const int y0 = ty * ny / ntY, y1 = (ty + 1) * ny / ntY, z0 = tz * nz / ntZ, z1 = (tz + 1) * nz / ntZ;
+    const int t = threadIdx.x, p = t % RL, row = t / RL;
+    // this lane's two neighbour slots (see block_row16)
+    int off[2], dy[2], dz[2], slot[2];
+    bool okx[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const bool real = p + RL * h < 27;
+        const int s = real ? p + RL * h : 26, q = (s * 171) >> 9;
+        const int dx = ((s * 57) >> 9) - 1;
+        slot[h] = s;
+        dy[h] = q - 3 * (dx + 1) - 1;
+        dz[h] = s - 3 * q - 1;
+        okx[h] = real && dx != 0 && (unsigned)(ix + dx) < (unsigned)nx && !(zin & 2);
+        off[h] = (dx * ny + dy[h]) * nz + dz[h];
+    }
+    const int hp = p < 2 ? 1 : 0;  // the slot in the plane
+    const bool inplane = p < 2 || p >= 9;
+    T B[4][2][9], un[4][2][3];
+    int li[4];
+    bool act[4], okp[4];
+    uint8_t dm[4];
+#pragma unroll
+    for (int pos = 0; pos < 4; ++pos) {
+        const int sub = FWD ? pos : 3 - pos, cy = (sub >> 1) & 1, cz = sub & 1, hy = pos < 2 ? 1 : 0, hz = 3 - pos;
+        int ya = max(y0 - hy, 0), za = max(z0 - hz, 0);
+        const int yb = min(y1 + hy, g.ydet), zb = min(z1 + hz, nz);
+        ya += (ya & 1) != cy;
+        za += (za & 1) != cz;
+        const int nr = yb > ya ? (yb - ya + 1) / 2 : 0, nc = zb > za ? (zb - za + 1) / 2 : 0, ncs = max(nc, 1);
+        act[pos] = row < nr * nc;
+        const int wr = row / ncs;
+        const int iy = act[pos] ? ya + 2 * wr : cy, iz = act[pos] ? za + 2 * (row - wr * ncs) : cz;
+        const int n = (ix * ny + iy) * nz + iz;
+        const int my = (ny - cy + 1) / 2, mz = (nz - cz + 1) / 2;
+        const size_t bo = block_offset(block_class_base(g, 4 * parity + sub), ((ix >> 1) * my + (iy >> 1)) * mz + (iz >> 1));
+        li[pos] = act[pos] ? (iy - y0 + HY) * RZ + iz - z0 + HZ : HY * RZ + HZ;
+        dm[pos] = 7;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const bool ok = (unsigned)(iy + dy[h]) < (unsigned)ny && (unsigned)(iz + dz[h]) < (unsigned)nz;
+#pragma unroll
+            for (int k = 0; k < 9; ++k) B[pos][h][k] = act[pos] ? blocks[bo + (k * 27 + slot[h]) * BLOCK_GROUP] : T(0);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) un[pos][h][c] = act[pos] && okx[h] && ok ? unb[(size_t)c * N + n + off[h]] : T(0);
+            if (h == hp) okp[pos] = inplane && ok;
+        }
+        if (p == DIAG_LANE && act[pos]) dm[pos] = dmask ? dmask[n] : uint8_t(0);
+    }
+    for (int w = t; w < 3 * CS; w += NT) {
+        const int c = w / CS, q = w - c * CS, ly = q / RZ, lz = q - ly * RZ, gy = y0 - HY + ly, gz = z0 - HZ + lz;
+        const bool in = (unsigned)gy < (unsigned)ny && (unsigned)gz < (unsigned)nz;
+        const size_t m = (size_t)c * N + ((size_t)ix * ny + gy) * nz + gz;
+        sb[w] = in ? b[m] : T(0);
+        su[w] = in && !(zin & 1) ? uin[m] : T(0);
+    }
+    T acc[4][3];
+#pragma unroll
+    for (int pos = 0; pos < 4; ++pos)
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            T v = T(0);
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int c = 0; c < 3; ++c) v += B[pos][h][3 * a + c] * un[pos][h][c];
+            acc[pos][a] = v;
+        }
+    const int lo = (hp ? dy[1] : dy[0]) * RZ + (hp ? dz[1] : dz[0]);
+    __syncthreads();
+#pragma unroll
+    for (int pos = 0; pos < 4; ++pos) {
+        if (act[pos]) {  // whole rows of sixteen lanes
+            T v[3], f[3];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) v[c] = okp[pos] ? su[c * CS + li[pos] + lo] : T(0);
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                T s = acc[pos][a];
+#pragma unroll
+                for (int c = 0; c < 3; ++c) s += (hp ? B[pos][1][3 * a + c] : B[pos][0][3 * a + c]) * v[c];
+                f[a] = row16_sum(s);
+            }
+            if (p == DIAG_LANE && dm[pos] != 7) {
+                const T bms[3] = {sb[li[pos]] - f[0], sb[CS + li[pos]] - f[1], sb[2 * CS + li[pos]] - f[2]};
+                gs_update(su, CS, li[pos], bms, B[pos][0], dm[pos], FWD ? 1 : 0);
+            }
+        }
+        __syncthreads();
+    }
+    const int OY = y1 - y0, OZ = z1 - z0;
+    for (int w = t; w < 3 * TY * TZ; w += NT) {
+        const int c = w / (TY * TZ), q = w - c * TY * TZ, oy = q / TZ, oz = q - oy * TZ;
+        if (oy < OY && oz < OZ)
+            uout[(size_t)c * N + ((size_t)ix * ny + y0 + oy) * nz + z0 + oz] = su[c * CS + (oy + HY) * RZ + oz + HZ];
     }
 }
 
@@ -892,6 +1014,31 @@ void launch_block_gs(const Grid &g, const T *blocks, T *u, const T *b, const uin
     VF_HIP(hipGetLastError());
 }
 
+// A workgroup holds a compute unit with its registers, so a launch is one latency long while every workgroup has a unit of
+// its own, and the halo (27 + 24 + 14 + 12 nodes for a tile of 12 per colour) costs nothing; beyond that the eight colour
+// launches are faster. Sweeps in us, two launches / eight (FP64, FP32): 33x17x17 (170 workgroups) 21.7 / 29.6,
+// 19.7 / 30.6; 27x15x13 (112) 19.7 / 29.6, 18.6 / 29.5; 45x23x19 (276) 42.6 / 31.8, 31.1 / 30.7; 65x33x33 85 / 52, 58 / 53.
+bool block_gs_planes(const Grid &g) {
+    const int ntY = (g.nn[1] + BP_TY - 1) / BP_TY, ntZ = (g.nn[2] + BP_TZ - 1) / BP_TZ;
+    return (long)ntY * ntZ * ((g.nn[0] + 1) / 2) <= CUS;
+}
+
+template <typename T>
+void launch_block_gs_plane(const Grid &g, const T *blocks, const T *uin, const T *unb, T *uout, const T *b,
+                           const uint8_t *dmask, int parity, int forward, hipStream_t s, int zin) {
+    if (uin == uout) throw std::runtime_error("the two-launch sweep needs distinct input and output vectors");
+    const int planes = (g.nn[0] - parity + 1) / 2;
+    if (planes <= 0) return;
+    const int ntY = (g.nn[1] + BP_TY - 1) / BP_TY, ntZ = (g.nn[2] + BP_TZ - 1) / BP_TZ;
+    if (forward)
+        hipLaunchKernelGGL((k_block_gs_plane<T, BP_TY, BP_TZ, BP_NT, true>), dim3(ntY * ntZ, planes), dim3(BP_NT), 0, s, g,
+                           blocks, uin, unb, uout, b, dmask, parity, ntY, ntZ, zin);
+    else
+        hipLaunchKernelGGL((k_block_gs_plane<T, BP_TY, BP_TZ, BP_NT, false>), dim3(ntY * ntZ, planes), dim3(BP_NT), 0, s, g,
+                           blocks, uin, unb, uout, b, dmask, parity, ntY, ntZ, zin);
+    VF_HIP(hipGetLastError());
+}
+
 // x-chunks of a marching transfer: about TARGET workgroups in all, at least MINLEN planes per chunk; a
 // small level (fewer than TARGET workgroups even at one plane each), whose launch is latency-bound, gets
 // one plane per workgroup
@@ -941,6 +1088,8 @@ void launch_interpolate(const Grid &gf, const Grid &gc, const T *xc, T *xf, int 
                                     hipStream_t);                                                                      \
     template void launch_l1_gs<T>(const Grid &, const Grid &, const T *, const L1Coef &, const T *, T *, const T *,    \
                                   const uint8_t *, int, int, bool, hipStream_t);                                                        \
+    template void launch_block_gs_plane<T>(const Grid &, const T *, const T *, const T *, T *, const T *,               \
+                                           const uint8_t *, int, int, hipStream_t, int);                               \
     template void launch_block_gs<T>(const Grid &, const T *, T *, const T *, const uint8_t *, int, int, hipStream_t); \
     template void launch_restrict<T>(const Grid &, const Grid &, const T *, T *, hipStream_t, T *);                   \
     template void launch_interpolate<T>(const Grid &, const Grid &, const T *, T *, int, hipStream_t);
