@@ -152,3 +152,44 @@ def test_level1_on_the_fly(ne, levels, layer, size):
             assert rel(mg._precondition(r, 1, 1, False, "fp32"), mg._precondition(r, 1, 1, False, "fp64")) < 1e-5
     finally:
         capi.set_kernel_variant(0)
+
+
+# the planar sweep: tiles of 8 x 12 nodes (one, several, with remainders), both directions, layers masked so that rows end
+# inside a tile, one and two sweeps per visit (residual with the only sweep or the second, correction before the first);
+# an element row has 8 products, a node four elements: 1e-12 for a sweep, 1e-11 through a cycle's coarse solve
+@pytest.mark.parametrize("ne,levels,layer,fmg,nu,sym", [((4, 4), 1, None, False, 1, True), ((8, 12), 2, None, True, 2, True),
+                                                        ((36, 24), 2, 17, False, 2, True), ((20, 52), 2, 30, True, 1, True),
+                                                        ((64, 48), 3, 40, True, 2, False), ((40, 24), 1, None, False, 3, True),
+                                                        ((16, 32), 2, None, False, 0, True)])
+def test_planar_sweep(ne, levels, layer, fmg, nu, sym):
+    import voxelfem_amd
+    from oracle import oracle2d as o2
+
+    rho = wl.noise_density(ne, 3, base=0.5, amp=0.4)
+    mg = wl.configure2d(voxelfem_amd.pyVoxelFEM, ne, wl.MBB2D_BC, rho).multigridSolver(levels)
+    s = o2.Sim(ne)
+    s.set_etensor(1.0, 0.3)
+    s.set_law(0, 1.0, 1e-9, 3.0, 3.0)
+    s.set_densities(rho)
+    mask = wl.mbb2d_mask(ne)
+    s.set_dirichlet(mask)
+    om = o2.MG(s, levels)
+    if layer is not None:
+        mg.setFabricationMaskHeightByLayer(layer)
+        om.set_mask_layer(layer)
+    mg.setSymmetricGaussSeidel(sym)
+    om.set_symmetric(sym)
+    mg.updateStiffnessMatrices()
+    om.update_stiffness()
+    rng = np.random.default_rng(7)
+    for l in range(levels):
+        nn = om.num_nodes(l)
+        u, b = rng.normal(size=(nn, 2)), rng.normal(size=(nn, 2))
+        iy = np.arange(nn) % ((ne[1] >> l) + 1)
+        act = np.ones(nn, bool) if layer is None else iy < -(-layer >> l) + 1
+        u[~act] = 0
+        for fwd in (True, False):
+            assert rel(mg._smooth(l, u, b, fwd)[act], om.smooth(l, u, b, fwd)[act]) < 1e-12, (l, fwd)
+    r = rng.normal(size=(om.num_nodes(0), 2))
+    r[np.arange(len(r)) % (ne[1] + 1) >= (ne[1] if layer is None else layer) + 1] = 0
+    assert rel(mg._precondition(r, 2, nu, fmg), om.precondition(r, 2, nu, fmg)) < 1e-11

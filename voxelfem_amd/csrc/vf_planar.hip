@@ -101,7 +101,7 @@ __global__ void __launch_bounds__(TPB) k_zero_young_rows2(PGrid g, int y0, int y
 template <bool FINE>
 __device__ __forceinline__ void elem_rows(const PGrid &g, const double *__restrict__ K0, const double *__restrict__ E,
                                           const double *__restrict__ Ke, const double *__restrict__ u, int ex, int ey,
-                                          int ln, double out[2], double M[4]) {
+                                          int ln, double out[2]) {
     const int e = ex * g.ne[1] + ey;
     const double *K = FINE ? K0 : Ke + (size_t)e * 64;
     const double s = FINE ? E[e] : 1.0;
@@ -121,23 +121,19 @@ __device__ __forceinline__ void elem_rows(const PGrid &g, const double *__restri
         // two 64-byte lines), instead of one line per entry of a column
         for (int a = 0; a < 8; ++a) t += (FINE ? K[a * 8 + 2 * ln + c] : K[(2 * ln + c) * 8 + a]) * ue[a];
         out[c] += s * t;
-        if (M) {
-            M[2 * c] += s * K[(2 * ln + c) * 8 + 2 * ln];
-            M[2 * c + 1] += s * K[(2 * ln + c) * 8 + 2 * ln + 1];
-        }
     }
 }
 
 template <bool FINE>
 __device__ __forceinline__ void node_Ku(const PGrid &g, const double *K0, const double *E, const double *Ke,
-                                        const double *u, int ix, int iy, double f[2], double *M) {
+                                        const double *u, int ix, int iy, double f[2]) {
 #pragma unroll
     for (int i = 1; i >= 0; --i)
 #pragma unroll
         for (int j = 1; j >= 0; --j) {
             const int ex = ix - i, ey = iy - j;
             if (ex < 0 || ey < 0 || ex >= g.ne[0] || ey >= g.ne[1]) continue;
-            elem_rows<FINE>(g, K0, E, Ke, u, ex, ey, 2 * i + j, f, M);
+            elem_rows<FINE>(g, K0, E, Ke, u, ex, ey, 2 * i + j, f);
         }
 }
 
@@ -154,7 +150,7 @@ __global__ void __launch_bounds__(TPB) k_apply2(PGrid g, const double *__restric
         return;
     }
     double f[2] = {0, 0};
-    node_Ku<FINE>(g, K0, E, Ke, u, ix, iy, f, nullptr);
+    node_Ku<FINE>(g, K0, E, Ke, u, ix, iy, f);
     const double b0 = zeroInit ? 0.0 : y[n], b1 = zeroInit ? 0.0 : y[g.nnodes + n];
     y[n] = negate ? b0 - f[0] : b0 + f[0];
     y[g.nnodes + n] = negate ? b1 - f[1] : b1 + f[1];
@@ -173,7 +169,7 @@ __global__ void __launch_bounds__(TPB) k_residual2(PGrid g, const double *__rest
     const uint8_t dm = dmask[n];
     if (iy < g.ydet) {
         double f[2] = {0, 0};
-        node_Ku<FINE>(g, K0, E, Ke, u, ix, iy, f, nullptr);
+        node_Ku<FINE>(g, K0, E, Ke, u, ix, iy, f);
         r[n] = (dm & 1) ? 0.0 : b[n] - f[0];
         r[g.nnodes + n] = (dm & 2) ? 0.0 : b[g.nnodes + n] - f[1];
     } else if (iy < g.ydet + 4) {
@@ -186,7 +182,7 @@ __global__ void __launch_bounds__(TPB) k_residual2(PGrid g, const double *__rest
 }
 
 // computeResidual on a coarse level with four work-items per node (one per incident element, summed in
-// node_Ku's order by the first of the four, as in k_smooth2_x4): the same values as k_residual2<false>
+// node_Ku's order by the first of the four): the same values as k_residual2<false>
 __global__ void __launch_bounds__(TPB) k_residual2_x4(PGrid g, const double *__restrict__ Ke,
                                                      const uint8_t *__restrict__ dmask, const double *__restrict__ u,
                                                      const double *__restrict__ b, double *__restrict__ r) {
@@ -198,7 +194,7 @@ __global__ void __launch_bounds__(TPB) k_residual2_x4(PGrid g, const double *__r
         const int i = 1 - (p >> 1), j = 1 - (p & 1);
         const int ex = ix - i, ey = iy - j;
         if (ex >= 0 && ey >= 0 && ex < g.ne[0] && ey < g.ne[1])
-            elem_rows<false>(g, nullptr, nullptr, Ke, u, ex, ey, 2 * i + j, v, nullptr);
+            elem_rows<false>(g, nullptr, nullptr, Ke, u, ex, ey, 2 * i + j, v);
     }
     const int q0 = (int)(threadIdx.x & 63) & ~3;
     double f[2];
@@ -224,77 +220,211 @@ __global__ void __launch_bounds__(TPB) k_residual2_x4(PGrid g, const double *__r
     }
 }
 
-// one colour of the multicolour block Gauss-Seidel sweep (MultigridSolver.hh:347-379, 408-458): nodes
-// (ox + 2 i, oy + 2 j) of the non-detached rows; the 2 x 2 block solve for free nodes, the point sweep in
-// component order (reversed backwards) for partially constrained ones, fully constrained nodes kept
-__device__ __forceinline__ void gs_update2(const PGrid &g, uint8_t dm, const double f[2], const double M[4],
-                                           double *__restrict__ u, const double *__restrict__ b, int n, int forward) {
-    const double r0 = b[n] - f[0], r1 = b[g.nnodes + n] - f[1];
-    double d0, d1;
-    if (dm) {
-        const double fr0 = (dm & 1) ? 0.0 : 1.0, fr1 = (dm & 2) ? 0.0 : 1.0;
-        if (forward) {
-            d0 = r0 * (fr0 / M[0]);
-            d1 = (r1 - M[2] * d0) * (fr1 / M[3]);
-        } else {
-            d1 = r1 * (fr1 / M[3]);
-            d0 = (r0 - M[1] * d1) * (fr0 / M[0]);
-        }
-    } else {
-        const double id = 1.0 / (M[0] * M[3] - M[1] * M[2]);
-        d0 = (M[3] * r0 - M[1] * r1) * id;
-        d1 = (M[0] * r1 - M[2] * r0) * id;
-    }
-    u[n] += d0;
-    u[g.nnodes + n] += d1;
-}
-template <bool FINE>
-__global__ void __launch_bounds__(TPB) k_smooth2(PGrid g, const double *__restrict__ K0, const double *__restrict__ E,
-                                                 const double *__restrict__ Ke, const uint8_t *__restrict__ dmask,
-                                                 double *__restrict__ u, const double *__restrict__ b, int ox, int oy,
-                                                 int forward) {
-    const int mx = (g.nn[0] - ox + 1) / 2, my = (g.ydet - oy + 1) / 2;
-    const int t = blockIdx.x * TPB + threadIdx.x;
-    if (my <= 0 || t >= mx * my) return;
-    const int ix = ox + 2 * (t / my), iy = oy + 2 * (t % my);
-    const int n = ix * g.nn[1] + iy;
-    const uint8_t dm = dmask[n];
-    if (dm == 3) return;
-    double f[2] = {0, 0}, M[4] = {0, 0, 0, 0};
-    node_Ku<FINE>(g, K0, E, Ke, u, ix, iy, f, M);
-    gs_update2(g, dm, f, M, u, b, n, forward);
-}
-// The same colour step on a coarse level with four work-items per node, one per incident element in node_Ku's
-// order ((1,1), (1,0), (0,1), (0,0)): four times the work-items in flight and a quarter of the dependent gathers
-// each. The first of the four sums the contributions in that order (the coarse products carry no modulus, so
-// the sums equal node_Ku's bit for bit) and updates the node.
-__global__ void __launch_bounds__(TPB) k_smooth2_x4(PGrid g, const double *__restrict__ Ke,
-                                                    const uint8_t *__restrict__ dmask, double *__restrict__ u,
-                                                    const double *__restrict__ b, int ox, int oy, int forward) {
-    const int mx = (g.nn[0] - ox + 1) / 2, my = (g.ydet - oy + 1) / 2;
-    const int tt = blockIdx.x * TPB + threadIdx.x, t = tt >> 2, p = tt & 3;
-    if (my <= 0 || t >= mx * my) return;  // all four work-items of a node
-    const int ix = ox + 2 * (t / my), iy = oy + 2 * (t % my);
-    const int n = ix * g.nn[1] + iy;
-    const uint8_t dm = dmask[n];
-    if (dm == 3) return;  // all four work-items of a node
-    const int i = 1 - (p >> 1), j = 1 - (p & 1);
-    const int ex = ix - i, ey = iy - j;
-    double v[6] = {0, 0, 0, 0, 0, 0};  // f[2], M[4] of this element
-    if (ex >= 0 && ey >= 0 && ex < g.ne[0] && ey < g.ne[1])
-        elem_rows<false>(g, nullptr, nullptr, Ke, u, ex, ey, 2 * i + j, v, v + 2);
-    const int q0 = (int)(threadIdx.x & 63) & ~3;
-    double acc[6];
+// the value of interpolation at the fine node (ix, iy) (MultigridSolver.hh:178-214)
+__device__ __forceinline__ void prolong2(const PGrid &c, const double *__restrict__ xc, int ix, int iy, double v[2]) {
+    const int id[2] = {ix, iy};
+    int e[2];
+    double w[2][2];
 #pragma unroll
-    for (int k = 0; k < 6; ++k) {
-        double a = __shfl(v[k], q0, 64);
-        a += __shfl(v[k], q0 + 1, 64);
-        a += __shfl(v[k], q0 + 2, 64);
-        a += __shfl(v[k], q0 + 3, 64);
-        acc[k] = a;
+    for (int d = 0; d < 2; ++d) {
+        e[d] = min(id[d] / 2, c.ne[d]);
+        const int lf = id[d] - 2 * e[d];
+        w[d][0] = lf ? 0.5 : 1.0;
+        w[d][1] = lf ? 0.5 : 0.0;
     }
-    if (p) return;
-    gs_update2(g, dm, acc, acc + 2, u, b, n, forward);
+    v[0] = v[1] = 0;
+#pragma unroll
+    for (int lc = 0; lc < 4; ++lc) {
+        const int a = (lc >> 1) & 1, bb = lc & 1;
+        const double coeff = w[0][a] * w[1][bb];
+        if (coeff == 0) continue;
+        const int m = (e[0] + a) * c.nn[1] + e[1] + bb;
+        v[0] += coeff * xc[m];
+        v[1] += coeff * xc[c.nnodes + m];
+    }
+}
+
+// sum over the four lanes of a quad, in every lane (quad permutations: vector instructions)
+template <int CTRL>
+__device__ __forceinline__ double quad_perm(double v) {
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double quad_sum(double v) {
+    v += quad_perm<0xB1>(v);         // [1,0,3,2]
+    return v + quad_perm<0x4E>(v);  // [2,3,0,1]
+}
+
+// One multicolour block Gauss-Seidel sweep (MultigridSolver.hh:347-379, 408-458) in one launch: the four colours
+// (ox, oy), nodes (ox + 2 i, oy + 2 j) of the non-detached rows; the 2 x 2 block solve for free nodes, the point sweep in
+// component order (reversed backwards) for partially constrained ones, fully constrained nodes kept. A workgroup takes a
+// tile of SX x SY nodes, holds the values in LDS and applies each colour on the tile grown by the halo that the later
+// colours read ((1,3), (1,2), (0,1), (0,0) nodes in (x, y), one more with RES; neighbouring tiles recompute it from the
+// same inputs, so uout != uin). Four lanes per node, one per incident element, and a quad for every node of each of the
+// four colours: all element rows (coarse: of the products, fine: of K0, once, with the moduli) are requested before the
+// first colour. The rows in registers then give the residual as well: with RES, r = b - K u of the tile after the sweep
+// (computeResidual, MultigridSolver.hh:527-541; as k_residual2).
+// mode: 1: Dirichlet components of uin are taken as zero; 2: rows below ydet + 4 of uin are taken as zero and not read;
+// 4: the interpolation of xc is added to uin on the non-detached rows.
+// Bound by latency (launch, one round of loads, four colours through LDS): on the levels of a 384 x 192 grid a coarse sweep
+// takes 9.3 us, 12.7 with the residual, where four colour launches took 19 and the residual 5; the finest level 15.2 and
+// 19.4 us instead of 18.6 and 5. The larger saving is the host's, 5 launches per level of a cycle with two sweeps where
+// there were 21: the whole solve 9.8 -> 5.6 ms.
+constexpr int SX = 8, SY = 12, SNT = 256;
+template <bool FINE, bool FWD, bool RES>
+__global__ void __launch_bounds__(SNT) k_sweep2(PGrid g, PGrid c, const double *__restrict__ K0,
+                                                const double *__restrict__ E, const double *__restrict__ Ke,
+                                                const uint8_t *__restrict__ dmask, const double *__restrict__ uin,
+                                                const double *__restrict__ xc, const double *__restrict__ b,
+                                                double *__restrict__ uout, double *__restrict__ r, int mode, int ntX,
+                                                int ntY) {
+    constexpr int X = RES ? 1 : 0, HX = 2 + X, HY = 4 + X, RX = SX + 2 * HX, RY = SY + 2 * HY, CS = RX * RY;
+    static_assert(SX % 2 == 0 && SY % 2 == 0 && (SX / 2 + 1 + X) * (SY / 2 + 3 + X) <= SNT / 4, "a quad for every node");
+    __shared__ double su[2 * CS];
+    const int N = g.nnodes, nx = g.nn[0], ny = g.nn[1];
+    const int ty = blockIdx.x % ntY, tx = blockIdx.x / ntY;
+    const int x0 = (long)tx * nx / ntX, x1 = (long)(tx + 1) * nx / ntX;
+    const int y0 = (long)ty * ny / ntY, y1 = (long)(ty + 1) * ny / ntY;
+    const int t = threadIdx.x, quad = t >> 2, p = t & 3;
+    const int ei = 1 - (p >> 1), ej = 1 - (p & 1), ln = 2 * ei + ej;  // this lane's element (ix - ei, iy - ej)
+    double K[FINE ? 1 : 4][16], sc[4], bn[4][2], M[4][4], id[4];
+    int li[4], node[4];
+    bool act[4], own[4], val[4];
+    uint8_t dm[4];
+    if (FINE) {
+#pragma unroll
+        for (int k = 0; k < 16; ++k) K[0][k] = K0[2 * ln * 8 + k];
+    }
+#pragma unroll
+    for (int pos = 0; pos < 4; ++pos) {
+        const int sub = FWD ? pos : 3 - pos, ox = (sub >> 1) & 1, oy = sub & 1;
+        const int hx = (pos < 2 ? 1 : 0) + X, hy = 3 - pos + X;
+        int xa = max(x0 - hx, 0), ya = max(y0 - hy, 0);
+        const int xb = min(x1 + hx, nx), yb = min(y1 + hy, g.ydet);
+        xa += (xa & 1) != ox;
+        ya += (ya & 1) != oy;
+        const int nr = xb > xa ? (xb - xa + 1) / 2 : 0, nc = yb > ya ? (yb - ya + 1) / 2 : 0, ncs = max(nc, 1);
+        act[pos] = quad < nr * nc;
+        const int q = quad / ncs, ix = act[pos] ? xa + 2 * q : x0, iy = act[pos] ? ya + 2 * (quad - q * ncs) : y0;
+        const int ex = ix - ei, ey = iy - ej;
+        node[pos] = ix * ny + iy;
+        li[pos] = (ix - x0 + HX) * RY + iy - y0 + HY;
+        own[pos] = act[pos] && ix >= x0 && ix < x1 && iy >= y0 && iy < y1;
+        val[pos] = act[pos] && ex >= 0 && ey >= 0 && ex < g.ne[0] && ey < g.ne[1];
+        const size_t e = val[pos] ? (size_t)ex * g.ne[1] + ey : 0;
+        dm[pos] = act[pos] ? dmask[node[pos]] : uint8_t(3);
+        bn[pos][0] = act[pos] ? b[node[pos]] : 0.0;
+        bn[pos][1] = act[pos] ? b[N + node[pos]] : 0.0;
+        if (FINE) sc[pos] = val[pos] ? E[e] : 0.0;
+        else {
+#pragma unroll
+            for (int k = 0; k < 16; ++k) K[FINE ? 0 : pos][k] = val[pos] ? Ke[e * 64 + 2 * ln * 8 + k] : 0.0;
+        }
+    }
+    for (int w = t; w < CS; w += SNT) {
+        const int lx = w / RY, ly = w - lx * RY, gx = x0 - HX + lx, gy = y0 - HY + ly;
+        double v[2] = {0, 0};
+        if ((unsigned)gx < (unsigned)nx && (unsigned)gy < (unsigned)ny) {
+            const int m = gx * ny + gy;
+            if (!((mode & 2) && gy < g.ydet + 4)) {
+                v[0] = uin[m];
+                v[1] = uin[N + m];
+                if (mode & 1) {
+                    const uint8_t d = dmask[m];
+                    if (d & 1) v[0] = 0;
+                    if (d & 2) v[1] = 0;
+                }
+            }
+            if ((mode & 4) && gy < g.ydet) {
+                double q[2];
+                prolong2(c, xc, gx, gy, q);
+                v[0] += q[0];
+                v[1] += q[1];
+            }
+        }
+        su[w] = v[0];
+        su[CS + w] = v[1];
+    }
+#pragma unroll
+    for (int pos = 0; pos < 4; ++pos) {  // the diagonal blocks
+        const double s = FINE ? sc[pos] : 1.0;
+        const double *k = K[FINE ? 0 : pos];
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            const int o = (a >> 1) * 8 + (a & 1);
+            // entry 2 ln + (a & 1) of row a >> 1, by selects: registers have no index
+            const double d = ln == 0 ? k[o] : ln == 1 ? k[o + 2] : ln == 2 ? k[o + 4] : k[o + 6];
+            M[pos][a] = quad_sum(s * d);
+        }
+        id[pos] = dm[pos] == 0 ? 1.0 / (M[pos][0] * M[pos][3] - M[pos][1] * M[pos][2]) : 0.0;
+    }
+    auto Ku = [&](int pos, double f[2]) {
+        double ue[8];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            const int o = li[pos] + ((m >> 1) - ei) * RY + (m & 1) - ej;
+            ue[2 * m] = su[o];
+            ue[2 * m + 1] = su[CS + o];
+        }
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            double s = 0;
+#pragma unroll
+            for (int a = 0; a < 8; ++a) s += K[FINE ? 0 : pos][8 * q + a] * ue[a];
+            f[q] = quad_sum(val[pos] ? (FINE ? sc[pos] * s : s) : 0.0);
+        }
+    };
+    __syncthreads();
+#pragma unroll
+    for (int pos = 0; pos < 4; ++pos) {
+        if (dm[pos] != 3) {  // whole quads
+            double f[2], d0, d1;
+            Ku(pos, f);
+            const double r0 = bn[pos][0] - f[0], r1 = bn[pos][1] - f[1];
+            const double *m = M[pos];
+            if (dm[pos]) {
+                const double fr0 = (dm[pos] & 1) ? 0.0 : 1.0, fr1 = (dm[pos] & 2) ? 0.0 : 1.0;
+                if (FWD) {
+                    d0 = r0 * (fr0 / m[0]);
+                    d1 = (r1 - m[2] * d0) * (fr1 / m[3]);
+                } else {
+                    d1 = r1 * (fr1 / m[3]);
+                    d0 = (r0 - m[1] * d1) * (fr0 / m[0]);
+                }
+            } else {
+                d0 = (m[3] * r0 - m[1] * r1) * id[pos];
+                d1 = (m[0] * r1 - m[2] * r0) * id[pos];
+            }
+            if (p == 0) su[li[pos]] += d0;
+            if (p == 1) su[CS + li[pos]] += d1;
+        }
+        __syncthreads();
+    }
+    if (RES) {
+#pragma unroll
+        for (int pos = 0; pos < 4; ++pos)
+            if (own[pos]) {
+                double f[2];
+                Ku(pos, f);
+                if (p == 0) r[node[pos]] = (dm[pos] & 1) ? 0.0 : bn[pos][0] - f[0];
+                if (p == 1) r[N + node[pos]] = (dm[pos] & 2) ? 0.0 : bn[pos][1] - f[1];
+            }
+    }
+    const int OX = x1 - x0, OY = y1 - y0;
+    for (int w = t; w < SX * SY; w += SNT) {
+        const int lx = w / SY, ly = w - lx * SY, gy = y0 + ly, m = (x0 + lx) * ny + gy;
+        if (lx >= OX || ly >= OY) continue;
+        const int q = (lx + HX) * RY + ly + HY;
+        uout[m] = su[q];
+        uout[N + m] = su[CS + q];
+        if (RES && gy >= g.ydet) {
+            const uint8_t d = dmask[m];
+            const bool near = gy < g.ydet + 4;
+            if ((d & 1) || near) r[m] = (d & 1) ? 0.0 : b[m];
+            if ((d & 2) || near) r[N + m] = (d & 2) ? 0.0 : b[N + m];
+        }
+    }
 }
 
 // restriction (MultigridSolver.hh:216-275): the transpose of the bilinear interpolation over the fine
@@ -331,32 +461,14 @@ __global__ void __launch_bounds__(TPB) k_interp2(PGrid f, PGrid c, const double 
     if (n >= f.nnodes) return;
     const int ix = n / f.nn[1], iy = n % f.nn[1];
     if (iy >= (accumulate ? f.ydet : f.nn[1])) return;
-    const int id[2] = {ix, iy};
-    int e[2];
-    double w[2][2];
-#pragma unroll
-    for (int d = 0; d < 2; ++d) {
-        e[d] = min(id[d] / 2, c.ne[d]);
-        const int lf = id[d] - 2 * e[d];
-        w[d][0] = lf ? 0.5 : 1.0;
-        w[d][1] = lf ? 0.5 : 0.0;
-    }
-    double v0 = 0, v1 = 0;
-#pragma unroll
-    for (int lc = 0; lc < 4; ++lc) {
-        const int a = (lc >> 1) & 1, bb = lc & 1;
-        const double coeff = w[0][a] * w[1][bb];
-        if (coeff == 0) continue;
-        const int m = (e[0] + a) * c.nn[1] + e[1] + bb;
-        v0 += coeff * xc[m];
-        v1 += coeff * xc[c.nnodes + m];
-    }
+    double v[2];
+    prolong2(c, xc, ix, iy, v);
     if (accumulate) {
-        xf[n] += v0;
-        xf[f.nnodes + n] += v1;
+        xf[n] += v[0];
+        xf[f.nnodes + n] += v[1];
     } else {
-        xf[n] = v0;
-        xf[f.nnodes + n] = v1;
+        xf[n] = v[0];
+        xf[f.nnodes + n] = v[1];
     }
 }
 
@@ -912,9 +1024,11 @@ PMG::PMG(PSim *s, int levels) : sim(s), L(levels) {
         p->x.resize(n);
         p->b.resize(n);
         p->r.resize(n);
+        p->w.resize(n);
         launch_fill<double>(n, p->x.data(), 0.0, st());
         launch_fill<double>(n, p->b.data(), 0.0, st());
         launch_fill<double>(n, p->r.data(), 0.0, st());
+        launch_fill<double>(n, p->w.data(), 0.0, st());
     }
     // coarse shape functions at the nodes of child fi (MultigridSolver.hh:664-687), phi[fi][fine l][coarse l]
     for (int fi = 0; fi < 4; ++fi)
@@ -1083,22 +1197,30 @@ void PMG::residual(int l, const double *u, const double *b, double *r) {
                            lv[l]->Ke.data(), dm, u, b, r);
     check_launch();
 }
-void PMG::smooth(int l, double *u, const double *b, bool forward) {
+// one sweep from uin into uout (uout != uin); modes of k_sweep2; with r, the residual after the sweep as well
+void PMG::sweep(int l, const double *uin, double *uout, const double *b, bool forward, int mode, double *r,
+                const double *xc) {
     const PGrid &g = lv[l]->g;
     const uint8_t *dm = l == 0 ? sim->dmask.data() : lv[l]->dmask.data();
-    for (int t = 0; t < 4; ++t) {
-        const int color = forward ? t : 3 - t;
-        const int ox = (color >> 1) & 1, oy = color & 1;
-        const int cnt = ((g.nn[0] - ox + 1) / 2) * std::max(0, (g.ydet - oy + 1) / 2);
-        if (cnt <= 0) continue;
-        if (l == 0)
-            hipLaunchKernelGGL(k_smooth2<true>, dim3(nblk(cnt)), dim3(TPB), 0, st(), g, sim->K0.data(), sim->E.data(),
-                               nullptr, dm, u, b, ox, oy, forward ? 1 : 0);
-        else
-            hipLaunchKernelGGL(k_smooth2_x4, dim3(nblk(4 * (size_t)cnt)), dim3(TPB), 0, st(), g, lv[l]->Ke.data(), dm,
-                               u, b, ox, oy, forward ? 1 : 0);
-        check_launch();
+    const int ntX = (g.nn[0] + SX - 1) / SX, ntY = (g.nn[1] + SY - 1) / SY;
+    if (uin == uout || r == uin || r == uout) throw std::runtime_error("the sweep needs distinct vectors");
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(ntX * ntY), dim3(SNT), 0, st(), g, xc ? lv[l + 1]->g : g, sim->K0.data(),
+                           sim->E.data(), l ? lv[l]->Ke.data() : nullptr, dm, uin, xc, b, uout, r, mode | (xc ? 4 : 0),
+                           ntX, ntY);
+    };
+    if (l == 0) {
+        if (r) forward ? go(k_sweep2<true, true, true>) : go(k_sweep2<true, false, true>);
+        else forward ? go(k_sweep2<true, true, false>) : go(k_sweep2<true, false, false>);
+    } else {
+        if (r) forward ? go(k_sweep2<false, true, true>) : go(k_sweep2<false, false, true>);
+        else forward ? go(k_sweep2<false, true, false>) : go(k_sweep2<false, false, false>);
     }
+    check_launch();
+}
+void PMG::smooth(int l, double *u, const double *b, bool forward) {
+    sweep(l, u, lv[l]->w.data(), b, forward, 0, nullptr, nullptr);
+    d2d(u, lv[l]->w.data(), level_n(l), st());
 }
 void PMG::restrict_to(int l, const double *fine, double *coarse) {
     hipLaunchKernelGGL(k_restrict2, dim3(nblk(lv[l + 1]->g.nnodes)), dim3(TPB), 0, st(), lv[l]->g, lv[l + 1]->g, fine,
@@ -1122,24 +1244,41 @@ void PMG::zero_dirichlet(int l, double *u) {
 }
 
 // vcycle / fullMultigrid (MultigridSolver.hh:587-658)
-void PMG::vcycle(int l, int nu, bool residualSystem) {
+// xZero: the iterate starts at zero on the rows below ydet + 4, without having been written
+void PMG::vcycle(int l, int nu, bool residualSystem, bool xZero) {
     PLevel &p = *lv[l];
     if (l == L) {
         coarse_solve(p.b.data(), p.x.data());
         return;
     }
-    if (residualSystem || l > 0) zero_dirichlet(l, p.x.data());
-    else sim->enforce_dirichlet(p.x.data());
-    for (int i = 0; i < nu; ++i) smooth(l, p.x.data(), p.b.data(), true);
-    residual(l, p.x.data(), p.b.data(), p.r.data());
+    const bool zd = residualSystem || l > 0;
+    if (!zd) sim->enforce_dirichlet(p.x.data());
     PLevel &c = *lv[l + 1];
+    // sweeps alternate between x and w (2 nu of them bring the iterate back to x); the first clears the Dirichlet
+    // components as it reads x, the last before the coarse correction leaves the residual, the first after it adds the
+    // correction
+    double *cur = p.x.data(), *alt = p.w.data();
+    for (int i = 0; i < nu; ++i) {
+        sweep(l, cur, alt, p.b.data(), true, i ? 0 : (zd ? 1 : 0) | (xZero ? 2 : 0), i == nu - 1 ? p.r.data() : nullptr,
+              nullptr);
+        std::swap(cur, alt);
+    }
+    if (nu <= 0) {
+        if (xZero) {
+            hipLaunchKernelGGL(k_zero_rows2, dim3(nblk(p.g.nnodes)), dim3(TPB), 0, st(), p.g,
+                               std::min(p.g.ydet + 4, p.g.nn[1]), p.x.data());
+            check_launch();
+        }
+        if (zd) zero_dirichlet(l, p.x.data());
+        residual(l, p.x.data(), p.b.data(), p.r.data());
+    }
     restrict_to(l, p.r.data(), c.b.data());
-    hipLaunchKernelGGL(k_zero_rows2, dim3(nblk(c.g.nnodes)), dim3(TPB), 0, st(), c.g,
-                       std::min(c.g.ydet + 4, c.g.nn[1]), c.x.data());
-    check_launch();
-    vcycle(l + 1, nu, true);
-    interpolate(l, c.x.data(), p.x.data(), true);
-    for (int i = 0; i < nu; ++i) smooth(l, p.x.data(), p.b.data(), !symmetricGS);
+    vcycle(l + 1, nu, true, true);
+    if (nu <= 0) interpolate(l, c.x.data(), p.x.data(), true);
+    for (int i = 0; i < nu; ++i) {
+        sweep(l, cur, alt, p.b.data(), !symmetricGS, 0, nullptr, i ? nullptr : c.x.data());
+        std::swap(cur, alt);
+    }
 }
 void PMG::fmg(int l, int nu, bool residualSystem) {
     PLevel &p = *lv[l];

@@ -83,6 +83,7 @@ struct PLevel {
     DBuf<uint8_t> dmask;
     DBuf<double> Ke;  // levels >= 1: element matrices
     DBuf<double> x, b, r;
+    DBuf<double> w;  // the iterate between two sweeps
 };
 
 struct PMG {
@@ -115,12 +116,14 @@ struct PMG {
     // level operations on device arrays
     void apply_K(int l, const double *u, double *y, bool zeroInit, bool negate);
     void residual(int l, const double *u, const double *b, double *r);
+    void sweep(int l, const double *uin, double *uout, const double *b, bool forward, int mode, double *r,
+               const double *xc);
     void smooth(int l, double *u, const double *b, bool forward);
     void restrict_to(int l, const double *fine, double *coarse);
     void interpolate(int l, const double *coarse, double *fine, bool accumulate);
     void coarse_solve(const double *b, double *x);
     void zero_dirichlet(int l, double *u);
-    void vcycle(int l, int nu, bool residualSystem);
+    void vcycle(int l, int nu, bool residualSystem, bool xZero = false);
     void fmg(int l, int nu, bool residualSystem);
     void precondition(const double *r, double *s, int mgIter, int nu, bool fullMG);
     void solve(double *x, const double *f, int numSteps, int nu, bool stiffnessUpdated, bool zeroDirichlet,
