@@ -5,18 +5,28 @@
 // particular isotropic) elasticity tensor is K0 = (1/64) W^T Khat W where Khat = W K0 W^T has only 48
 // nonzero entries: Khat[(k,d),(k,d)] and Khat[(k,d),(k ^ e_d ^ e_c, c)] for c != d with k_d != k_c
 // (the monomials of the element's displacement basis are orthogonal under 2-point Gauss integration).
-// One element product y_e = E_e K0 u_e therefore costs two 3-stage butterflies per component (72 + 72
-// additions), 48 products with the Khat entries and 24 scalings by E_e, instead of the 576
-// multiply-adds of the dense 24 x 24 product (TPSStencils.hh:453-471). The host verifies the sparsity
+// One element product y_e = E_e K0 u_e therefore costs two 3-stage butterflies per component, 48 products with the
+// Khat entries and 24 scalings by E_e, instead of the 576 multiply-adds of the dense 24 x 24 product
+// (TPSStencils.hh:453-471); along the march below half of the butterflies are shared with the neighbouring
+// element, which leaves 72 + 48 additions. The host verifies the sparsity
 // on the actual K0 and selects this kernel only where it holds.
 //
-// Work layout: a workgroup owns a (y,z) tile of 16 x 16 element columns and marches along x. The node
-// plane ahead is staged in LDS; each work-item forms its element's 24 outputs, keeps the four of the
-// face ahead in registers (they belong to the next node plane), and publishes the four of the current
-// plane to LDS, where the owner of each node adds the four (y,z)-neighbouring elements' values in a
-// fixed order. The tile's outer element row/column only serves its neighbours: a tile owns 15 x 15
-// node columns. Every node value is summed in the same order whatever the tiling, so results are
-// deterministic.
+// Work layout: a workgroup owns a (y,z) tile of 16 x 16 element columns and marches along x. The node plane ahead
+// is staged in LDS; each work-item reads the four corners of its column's face, takes the y and z stages of the
+// butterflies on that face once (the plane's transformed values serve the element ahead and the one behind), forms the x
+// stage and the products, and adds the two elements' contributions to a plane while they are still transformed, so that
+// the y and z stages back are taken once per plane as well. The corner values of the four (y,z)-neighbouring columns
+// are then added along z between lanes and along y through LDS, with one barrier a step. The tile's outer element
+// row/column only serves its neighbours: a tile owns 15 x 15 node columns. Every node value is summed in the same order
+// whatever the tiling, so results are deterministic.
+//
+// Measured against one with both butterflies per element, all corners through LDS, two barriers a step and the addresses
+// formed in the loop (577 vector instructions a step, now 267), in us, K u / residual: 65x33x33 FP64 9.2 / 9.3 -> 7.1 /
+// 7.1; 209x113x97 FP64 54.3 / 55.9 -> 41.7 / 43.0, FP32 36.6 / 37.4 -> 28.1 / 27.3; 257x129x129 FP64 85.6 / 111.9 -> 64.9 /
+// 99.1, FP32 58.5 / 60.9 -> 45.1 / 45.0; 385x193x193 FP64 259 / 394 -> 259 / 332, FP32 173 / 227 -> 148 / 198. At the
+// largest, K u is bound by neither the vector units (about 45%) nor the bytes (3.1 TB/s): requesting the planes two steps
+// ahead costs registers that spill, and waiting for all of a step's loads before the next ones are requested changes
+// nothing.
 #include "vf_internal.hpp"
 
 #include <algorithm>
@@ -46,24 +56,26 @@ __device__ constexpr WalshGroup kWalshGroups[14] = {
     {3, {5, 7, 12}},  {2, {6, 13, 0}},  {3, {9, 16, 20}},  {2, {10, 15, 0}}, {2, {11, 18, 0}},
     {2, {17, 19, 0}}, {1, {21, 0, 0}},  {1, {22, 0, 0}},   {1, {23, 0, 0}}};
 
-// y = W^T diag/offdiag(Khat/64) W u for one element, u and y as [8 nodes][3 components], in place
-template <typename T>
-__device__ __forceinline__ void walsh_apply(const T *__restrict__ C, T Ee, T v[8][3]) {
-    // forward butterflies: v[m][d] -> z[k][d]
+// the y and z stages of the butterflies of one face (node 2j+k), forward (m -> index) and backward
+template <typename T, bool FWD>
+__device__ __forceinline__ void face_butterfly(T f[4][3]) {
 #pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        const int bb = bitof(a);
+    for (int bb = 2; bb > 0; bb >>= 1)
 #pragma unroll
-        for (int m = 0; m < 8; ++m) {
+        for (int m = 0; m < 4; ++m) {
             if (m & bb) continue;
 #pragma unroll
             for (int d = 0; d < 3; ++d) {
-                const T lo = v[m][d], hi = v[m | bb][d];
-                v[m][d] = lo + hi;
-                v[m | bb][d] = hi - lo;
+                const T lo = f[m][d], hi = f[m | bb][d];
+                f[m][d] = FWD ? lo + hi : lo - hi;
+                f[m | bb][d] = FWD ? hi - lo : lo + hi;
             }
         }
-    }
+}
+
+// z -> E Khat z / 64 of one element, [index][component], in place
+template <typename T>
+__device__ __forceinline__ void walsh_product(const T *__restrict__ C, T Ee, T v[8][3]) {
     // zh[k][d] = E (Khat[(k,d),(k,d)] z[k][d] + sum_{c != d, k_d != k_c} Khat[(k,d),(k^e_d^e_c,c)] z[..][c]) / 64,
     // group by group: a group's rows only read the group's own entries, so they are overwritten after the group
     // (the temporaries are one group, not a second 24-entry array)
@@ -96,21 +108,26 @@ __device__ __forceinline__ void walsh_apply(const T *__restrict__ C, T Ee, T v[8
             v[grp.r[q] / 3][grp.r[q] % 3] = out[q];
         }
     }
-    // backward butterflies: y[m][d] = sum_k W[k][m] zh[k][d]
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        const int bb = bitof(a);
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            if (k & bb) continue;
-#pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                const T z0 = v[k][d], z1 = v[k | bb][d];
-                v[k][d] = z0 - z1;
-                v[k | bb][d] = z0 + z1;
-            }
-        }
-    }
+}
+
+// base plus a byte offset: a scalar base and a 32-bit lane offset are one addressing mode of the global loads
+template <typename U>
+__device__ __forceinline__ const U *at(const U *base, unsigned off) {
+    return reinterpret_cast<const U *>(reinterpret_cast<const char *>(base) + off);
+}
+template <typename U>
+__device__ __forceinline__ U *at(U *base, unsigned off) {
+    return reinterpret_cast<U *>(reinterpret_cast<char *>(base) + off);
+}
+
+// v of the next lane of its sixteen (the last one: 0)
+__device__ __forceinline__ float next_lane(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x101, 0xf, 0xf, true));  // row_shl:1
+}
+__device__ __forceinline__ double next_lane(double v) {
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0x101, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0x101, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
 }
 
 // dotp (SET mode, optional): per-workgroup partial sums of <u, y> over the owned nodes, in a fixed order.
@@ -120,7 +137,7 @@ __global__ void __launch_bounds__(NTW, sizeof(T) == 8 ? 3 : 5) k_ku_walsh(Grid g
                                                   const uint8_t *__restrict__ dmask, int ntZ, int xchunk,
                                                   double *__restrict__ dotp) {
     __shared__ T su[2][3 * RN * RN];  // node planes, double-buffered
-    __shared__ T sp[4][3 * NTW];      // per element column: its values at the four corners of the plane
+    __shared__ T sp[2][3 * NTW];      // per element column: the plane's sums at its low-y edge, double-buffered
     __shared__ double sred[NTW / 64];
     const int N = g.nnodes, nx = g.nn[0], ny = g.nn[1], nz = g.nn[2];
     const int tiles = gridDim.x;
@@ -135,35 +152,48 @@ __global__ void __launch_bounds__(NTW, sizeof(T) == 8 ? 3 : 5) k_ku_walsh(Grid g
     const int Y = ey + 1, Z = ez + 1;  // node owned by this work-item
     const bool owner = ly < TN && lz < TN && Y < g.ydet && Z < nz;
 
-    // Node planes are fetched one step ahead into registers (PF values per work-item) and written to
-    // LDS at the start of the next step, so the global-load latency overlaps a whole step of compute.
-    constexpr int PLANE = 3 * RN * RN;
-    constexpr int PF = (PLANE + NTW - 1) / NTW;
-    T pf[PF];
+    // Node planes are fetched one step ahead into registers (per component PF values per work-item) and written to LDS at
+    // the start of the next step, so the global-load latency overlaps a whole step of compute. Every access is a plane's
+    // base in scalar registers and a byte offset inside the plane, found once: address arithmetic inside the march took
+    // more vector instructions (a third of them products, at a quarter of the rate) than the element's own.
+    constexpr int FACE = RN * RN, PF = (FACE + NTW - 1) / NTW;
+    const size_t nplane = (size_t)ny * nz, eplane = (size_t)g.ne[1] * g.ne[2];
+    unsigned po[PF];
+    bool pok[PF];
+#pragma unroll
+    for (int q = 0; q < PF; ++q) {
+        const int w = t + q * NTW, ry = w / RN, rz = w - ry * RN, gy = sy + ry, gz = sz + rz;
+        pok[q] = w < FACE && (unsigned)gy < (unsigned)ny && (unsigned)gz < (unsigned)nz;
+        po[q] = pok[q] ? (unsigned)(((size_t)gy * nz + gz) * sizeof(T)) : 0u;
+    }
+    const unsigned no = owner ? (unsigned)(((size_t)Y * nz + Z) * sizeof(T)) : 0u;
+    const unsigned eo = elemOk ? (unsigned)(((size_t)ey * g.ne[2] + ez) * sizeof(T)) : 0u;
+    T pf[PF][3];
     auto fetch_plane = [&](int ix) {
+        const bool in = (unsigned)ix < (unsigned)nx;  // uniform
+        const T *up = u + (in ? ix : 0) * nplane;
 #pragma unroll
         for (int q = 0; q < PF; ++q) {
-            const int w = t + q * NTW;
-            T v = T(0);
-            if (w < PLANE) {
-                const int c = w / (RN * RN), r = w - c * (RN * RN), ry = r / RN, rz = r - ry * RN;
-                const int gy = sy + ry, gz = sz + rz;
-                if ((unsigned)ix < (unsigned)nx && (unsigned)gy < (unsigned)ny && (unsigned)gz < (unsigned)nz)
-                    v = u[(size_t)c * N + ((size_t)ix * ny + gy) * nz + gz];
+            pf[q][0] = pf[q][1] = pf[q][2] = T(0);
+            if (in && pok[q]) {
+#pragma unroll
+                for (int c = 0; c < 3; ++c) pf[q][c] = *at(up + (size_t)c * N, po[q]);
             }
-            pf[q] = v;
         }
     };
     auto store_plane = [&](int buf) {
 #pragma unroll
         for (int q = 0; q < PF; ++q) {
             const int w = t + q * NTW;
-            if (w < PLANE) su[buf][w] = pf[q];
+            if ((q + 1) * NTW <= FACE || w < FACE) {
+#pragma unroll
+                for (int c = 0; c < 3; ++c) su[buf][c * FACE + w] = pf[q][c];
+            }
         }
     };
     auto fetch_E = [&](int ex) {
         T v = T(0);
-        if (elemOk && (unsigned)ex < (unsigned)g.ne[0]) v = E[((size_t)ex * g.ne[1] + ey) * g.ne[2] + ez];
+        if ((unsigned)ex < (unsigned)g.ne[0] && elemOk) v = *at(E + ex * eplane, eo);
         return v;
     };
     auto read_face = [&](int buf, T f[4][3]) {
@@ -175,69 +205,82 @@ __global__ void __launch_bounds__(NTW, sizeof(T) == 8 ? 3 : 5) k_ku_walsh(Grid g
         }
     };
 
-    T carry[4][3];    // contributions of the previous element to the current node plane
+    T zold[4][3], carry[4][3];  // of the node plane behind: transformed values, transformed contributions so far
+    T fin[3] = {0, 0, 0};       // plane being finished: its sums at the high-y edge
+    T bv[3] = {0, 0, 0};        // and the right-hand side, or u for the dot product, at the owned node
+    uint8_t dm = 0;
     double dacc = 0;  // <u, y> over the owned nodes (SET mode with dotp)
 #pragma unroll
     for (int q = 0; q < 4; ++q) carry[q][0] = carry[q][1] = carry[q][2] = T(0);
+    // node plane ix: corners (j,k) of the elements at (ly+1-j, lz+1-k) that hold node (Y, Z), summed along z, then y
+    auto finish = [&](int ix, int buf) {
+        T *yp = y + ix * nplane;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const T f = fin[c] + sp[buf][c * NTW + t + TE];
+            T out = MODE == AM_RESIDUAL ? bv[c] - f : f;
+            if (dm & (1 << c)) out = T(0);
+            *at(yp + (size_t)c * N, no) = out;
+            if (MODE == AM_SET && dotp) dacc += (double)out * (double)bv[c];
+        }
+    };
     fetch_plane(x0 - 1);
     store_plane((x0 + 1) & 1);
     fetch_plane(x0);
     T Enext = fetch_E(x0 - 1);
+    __syncthreads();
+    read_face((x0 + 1) & 1, zold);
+    face_butterfly<T, true>(zold);
     for (int ex = x0 - 1; ex < x1; ++ex) {
-        // element plane ex: node planes ex (face i = 0) and ex + 1 (face i = 1)
+        // element plane ex: node planes ex (face i = 0, transformed in zold) and ex + 1 (face i = 1)
         const int buf = (ex + 1) & 1;
         store_plane(buf);     // plane ex + 1, fetched during the previous step
         fetch_plane(ex + 2);  // consumed by the next step
         const T Ee = Enext;
         Enext = fetch_E(ex + 1);
-        // right-hand side and mask of the node finished in this step, requested early
-        const int ix = ex;
-        const size_t n = ((size_t)ix * ny + Y) * nz + Z;
-        uint8_t dm = 0;
-        T bv[3] = {0, 0, 0};
-        if (owner && ix >= x0) {
-            if (dmask) dm = dmask[n];
-            if (MODE == AM_RESIDUAL) {
-                bv[0] = b[n];
-                bv[1] = b[(size_t)N + n];
-                bv[2] = b[(size_t)2 * N + n];
+        // The only barrier of a step: plane ex + 1 and the edge sums of plane ex - 1 are in LDS. Both buffers alternate, so
+        // what is overwritten in this step was last read before this barrier's predecessor.
+        __syncthreads();
+        if (ex > x0 && owner) finish(ex - 1, buf ^ 1);
+        if (owner && ex >= x0) {  // right-hand side and mask of plane ex, which the next step finishes
+            if (dmask) dm = *at(dmask + ex * nplane, no / (unsigned)sizeof(T));
+            const T *src = (MODE == AM_RESIDUAL ? b : u) + ex * nplane;
+            if (MODE == AM_RESIDUAL || dotp) {
+#pragma unroll
+                for (int c = 0; c < 3; ++c) bv[c] = *at(src + (size_t)c * N, no);
             }
         }
-        __syncthreads();
-        // both node planes of the element are in LDS: plane ex (stored during the previous step) and plane
-        // ex + 1; the slot of plane ex is next overwritten after this step's second barrier
-        T v[8][3];
-        read_face(buf ^ 1, v);       // local nodes 0jk (face i = 0)
-        read_face(buf, v + 4);       // local nodes 1jk (face i = 1)
-        // u at the owned node (Y, Z) of plane ex: corner (1,1) of the element's face i = 0
-        const T un0 = v[3][0], un1 = v[3][1], un2 = v[3][2];
-        walsh_apply<T>(C, Ee, v);
-        if (ex >= x0) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-#pragma unroll
-                for (int c = 0; c < 3; ++c) sp[q][c * NTW + t] = carry[q][c] + v[q][c];
-        }
+        T f[4][3], v[8][3];
+        read_face(buf, f);
+        face_butterfly<T, true>(f);
 #pragma unroll
         for (int q = 0; q < 4; ++q)
 #pragma unroll
-            for (int c = 0; c < 3; ++c) carry[q][c] = v[4 + q][c];
-        __syncthreads();
-        if (ex >= x0 && owner) {
-            // corners (j,k) of the elements at (ly+1-j, lz+1-k) that hold node (Y, Z)
+            for (int c = 0; c < 3; ++c) {
+                v[q][c] = zold[q][c] + f[q][c];
+                v[4 + q][c] = f[q][c] - zold[q][c];
+                zold[q][c] = f[q][c];
+            }
+        walsh_product<T>(C, Ee, v);
+        T w[4][3];  // plane ex: this element and the one behind, transformed
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
-                T f = sp[3][c * NTW + ly * TE + lz];
-                f += sp[2][c * NTW + ly * TE + lz + 1];
-                f += sp[1][c * NTW + (ly + 1) * TE + lz];
-                f += sp[0][c * NTW + (ly + 1) * TE + lz + 1];
-                T out = MODE == AM_RESIDUAL ? bv[c] - f : f;
-                if (dm & (1 << c)) out = T(0);
-                y[(size_t)c * N + n] = out;
-                if (MODE == AM_SET && dotp) dacc += (double)out * (double)(c == 0 ? un0 : (c == 1 ? un1 : un2));
+                w[q][c] = carry[q][c] + (v[q][c] - v[4 + q][c]);
+                carry[q][c] = v[q][c] + v[4 + q][c];
+            }
+        if (ex >= x0) {  // uniform
+            face_butterfly<T, false>(w);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                fin[c] = w[3][c] + next_lane(w[2][c]);
+                sp[buf][c * NTW + t] = w[1][c] + next_lane(w[0][c]);
             }
         }
     }
+    __syncthreads();
+    if (owner) finish(x1 - 1, x1 & 1);
     if (MODE == AM_SET && dotp) {
         for (int o = 32; o > 0; o >>= 1) dacc += __shfl_xor(dacc, o, 64);
         if ((t & 63) == 0) sred[t >> 6] = dacc;
