@@ -106,6 +106,35 @@ def test_coarse_factor(ne, levels, graphs):
         assert rel(mg._coarseSolve(b), om.coarse_solve(b)) < 1e-9
 
 
+# stiff voxels floating in void: diagonal blocks of the coarsest matrix are nearly singular. Cholesky's error does not
+# exceed a modest multiple of u kappa, kappa the condition number of the matrix scaled to a unit diagonal (van der Sluis);
+# the stable orders of elimination reach a third of u kappa here, so u kappa itself is the bound. Reference: refined in long
+# double
+@pytest.mark.parametrize("ne,Emin", [((8, 4, 4), 1e-9), ((6, 5, 4), 1e-9), ((8, 4, 4), 1e-12)])
+def test_direct_solve_stiff_pieces(ne, Emin):
+    import scipy.linalg as sl
+
+    import voxelfem_amd
+    from tests import fem_reference as fr
+
+    K0 = np.asarray(orc.element_stiffness(1.0, 0.3, (1.0, 1.0, 1.0))).reshape(24, 24)
+    free = np.repeat(wl.cantilever_mask(ne) == 0, 3)
+    for seed in range(16):
+        rho = (np.random.default_rng(seed).uniform(size=int(np.prod(ne))) < 0.15).astype(float)
+        K = fr.assemble_K(ne, K0, Emin + (1 - Emin) * rho).toarray()[np.ix_(free, free)]
+        d = 1 / np.sqrt(np.diag(K))
+        w = np.linalg.eigvalsh(K * d[:, None] * d)
+        f = np.zeros(len(free))
+        f[free] = np.random.default_rng(seed + 100).normal(size=len(K))
+        c, KL = sl.cho_factor(K * d[:, None] * d), K.astype(np.longdouble)
+        x = np.zeros(len(K), np.longdouble)
+        for _ in range(20):
+            x += d * sl.cho_solve(c, d * (f[free] - KL @ x).astype(float))
+        tps = wl.configure(voxelfem_amd.pyVoxelFEM, ne, wl.CANTILEVER_BC, rho, Emin=Emin)
+        u = tps.solve(f.reshape(-1, 3)).reshape(-1)[free]
+        assert np.linalg.norm(u - x) <= 2.0 ** -53 * w[-1] / w[0] * np.linalg.norm(x), seed
+
+
 # level 1 on the fly: every side of the grid within reach of every node, sides of different length and element size,
 # masked layers, a partially filled workgroup; variant 1 keeps level 1 on the fly
 @pytest.mark.parametrize("ne,levels,layer", [((4, 4, 4), 2, None), ((8, 4, 12), 2, None), ((12, 20, 8), 2, None),

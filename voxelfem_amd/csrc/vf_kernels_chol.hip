@@ -112,44 +112,51 @@ __device__ __forceinline__ double even_lane(double v) {  // quad_perm [0, 0, 2, 
     const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0xA0, 0xf, 0xf, true);
     return __hiloint2double(hi, lo);
 }
-// One elimination step of the wavefront's 16 x 16 block (see chol16) by the 2 x 2 pivot at rows J, J + 1: the rows below
-// lose their combination of the two. The old columns and the pivot come from the lanes that hold them. One wavefront
+// One elimination step of the wavefront's 16 x 16 block (see chol16): rows J and J + 1 leave the rows below, one after the
+// other as far as rounding goes (row J with pivot p00, then row J + 1 less m = p01 / p00 times row J, with pivot
+// s = p11 - m p01), so the step is as stable as two of Cholesky's. (Through the adjugate of the 2 x 2 pivot, with one
+// reciprocal of its determinant, the combinations cancel when the pivot is nearly singular: stiff pieces in 1e-9 void
+// were solved to 8e-4 in place of 1e-5, or refused.) The old columns and the pivots come from the lanes that hold them. One wavefront
 // alone is bound by the instructions it issues one after the other, so two rows go per step, and A and Y share one array.
 template <int J>
-__device__ __forceinline__ void chol16_step(double (&a)[4], int r, int part, double (&piv)[3], bool &ok) {
+__device__ __forceinline__ void chol16_step(double (&a)[4], int r, int part, double (&piv)[2], bool &ok) {
     constexpr int h = J / 4, i0 = J % 4;
     const double p00 = lane_value(a[i0], J + 16 * h), p01 = lane_value(a[i0], J + 1 + 16 * h),
                  p11 = lane_value(a[i0 + 1], J + 1 + 16 * h);
     const double c0 = __shfl(a[i0], r + 16 * h, 64), c1 = __shfl(a[i0 + 1], r + 16 * h, 64);
-    // the combination of the two rows is formed without the determinant, so that only one product follows its reciprocal
-    const double g0 = r > J + 1 ? c0 * p11 - c1 * p01 : 0.0, g1 = r > J + 1 ? c1 * p00 - c0 * p01 : 0.0;
-    double u[4];
+    const double ip = recip(p00), m = p01 * ip, s = __builtin_fma(-m, p01, p11), is = -recip(s);
+    const bool below = r > J + 1;
+    const double g = below ? -(c0 * ip) : 0.0, w = below ? __builtin_fma(-m, c0, c1) : 0.0;
+    // only the last product waits for the second reciprocal
+    double u[4], v[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) u[i] = __builtin_fma(g1, row_bcast<J + 1>(a[i]), g0 * row_bcast<J>(a[i]));
+    for (int i = 0; i < 4; ++i) {
+        const double rj = row_bcast<J>(a[i]);
+        u[i] = __builtin_fma(g, rj, a[i]);
+        v[i] = w * __builtin_fma(-m, rj, row_bcast<J + 1>(a[i]));
+    }
     if (part == h) {  // columns J, J + 1 of Y start here: rows J, J + 1 of it are (1, 0), (0, 1)
-        u[i0] = g0;
-        u[i0 + 1] = g1;
-        a[i0] = 0.0;
-        a[i0 + 1] = 0.0;
+        u[i0] = g;
+        u[i0 + 1] = 0.0;
+        v[i0] = -(w * m);
+        v[i0 + 1] = w;
     }
-    const double det = __builtin_fma(p00, p11, -(p01 * p01)), id = -recip(det);
-    ok = ok && p00 > 0 && det > 0;
+    ok = ok && p00 > 0 && s > 0;
     if ((r >> 1) == J / 2) {
-        piv[0] = p00;
-        piv[1] = p01;
-        piv[2] = det;
+        piv[0] = r & 1 ? s : p00;
+        piv[1] = r & 1 ? -m : 0.0;
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) a[i] = __builtin_fma(id, u[i], a[i]);
+    for (int i = 0; i < 4; ++i) a[i] = __builtin_fma(is, v[i], u[i]);
 }
 // U = L^-1 of the 16 x 16 symmetric block whose lower triangle is at S (row stride LS), by one wavefront: lane l holds
-// columns 4 (l / 16) .. + 3 of row l % 16. Eliminating two rows at a time turns [A | I] into [.. | Y] with Y A Y^T = D
-// block diagonal with the 2 x 2 pivots P = [p00 p01; p01 p11]; after the step at J the columns up to J + 1 of A are not
-// used again and hold those of Y instead. U = M Y with M = chol(P)^-1 per pivot: M00 = p00^-1/2, M11 = (det / p00)^-1/2,
-// M10 = -p01 / p00 M11. Writes U (zero above its diagonal) to X (row stride LS).
+// columns 4 (l / 16) .. + 3 of row l % 16. Eliminating two rows at a time turns [A | I] into [.. | Y]; after the step at J
+// the columns up to J + 1 of A are not used again and hold those of Y instead. Row J + 1 of Y still lacks its part
+// -m of row J, which is added at the end; U = D^-1/2 Y with the pivots D. Writes U (zero above its diagonal) to X (row
+// stride LS).
 __device__ __forceinline__ bool chol16(const double *S, double *X, int l) {
     const int r = l & 15, part = l >> 4, c0 = 4 * part;
-    double a[4], piv[3] = {1.0, 0.0, 1.0};
+    double a[4], piv[2] = {1.0, 0.0};
     bool ok = true;
 #pragma unroll
     for (int i = 0; i < 4; ++i) a[i] = S[max(r, c0 + i) * LS + min(r, c0 + i)];
@@ -161,13 +168,12 @@ __device__ __forceinline__ bool chol16(const double *S, double *X, int l) {
     chol16_step<10>(a, r, part, piv, ok);
     chol16_step<12>(a, r, part, piv, ok);
     chol16_step<14>(a, r, part, piv, ok);
-    const bool odd = r & 1;
-    const double ip = recip(piv[0]), scale = rsqrt_full(odd ? piv[2] * ip : piv[0]), m = odd ? -piv[1] * ip : 0.0;
+    const double scale = rsqrt_full(piv[0]);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int c = c0 + i;
         const double y = c == r ? 1.0 : c < (r & ~1) ? a[i] : 0.0;  // row r of Y
-        X[r * LS + c] = scale * __builtin_fma(m, even_lane(y), y);
+        X[r * LS + c] = scale * __builtin_fma(piv[1], even_lane(y), y);
     }
     return ok;
 }
@@ -310,9 +316,9 @@ __device__ __forceinline__ void panel_rows(double *sP, const double *sL, double 
 //   the roles after them: strips of 16 CT columns of block row k of X, X_kJ = -Linv_k sum_q L_{k,k-q} X_{k-q,J}
 //     (J < k), X_kk = Linv_k, and their transposes into XT. They are off the chain and fill the chip beside it. CT = 1
 //     spreads a row over four times the workgroups; CT = 4 reads each band block a quarter as often.
-// 4131 unknowns, kb = 5: 61 launches of 16.0 us against 183 of 13.0 (panel), 13.1 (update) and 52.2 us (diagonal block)
-// and 61 of 14.8 us for the rows of X: 0.99 against 5.66 ms. Of the 16 us the loads take 1.7, the panel 1.7, the update
-// 1.9, the diagonal block 8.3 (four 16 x 16 factors of 1.3 us one after the other) and the launch the rest.
+// 4131 unknowns, kb = 5: 61 launches of 16.3 us against 183 of 13.0 (panel), 13.1 (update) and 52.2 us (diagonal block)
+// and 61 of 14.8 us for the rows of X: 1.01 against 5.66 ms. Of the 16 us the loads take 1.7, the panel 1.7, the update
+// 1.9, the diagonal block 8.6 (four 16 x 16 factors of 1.4 us one after the other) and the launch the rest.
 template <int CT>
 __global__ void __launch_bounds__(TPB) k_band_step(int k, int nb, int kb, double *__restrict__ B, double *__restrict__ Linv,
                                                    double *__restrict__ X, double *__restrict__ XT, int *__restrict__ flag,
