@@ -59,6 +59,28 @@ def test_block_rows(ne, levels, layer):
             assert rel(mg._smooth(l, u, b, fwd)[act], om.smooth(l, u, b, fwd)[act]) < 1e-11, (l, fwd)
 
 
+# single precision takes two nodes of a z-row at a time: rows of one to fourteen nodes per colour, even and odd, ending inside
+# a pair, with colour launches (5 x 353 nodes per plane) and with the two-launch sweep; the sums are the same, rounded to
+# single precision: 1e-5, as the V-cycles of test_gpu_tiled
+@pytest.mark.parametrize("ne,levels,layer", [((8, 704, 4), 2, None), ((8, 704, 12), 2, None), ((8, 704, 16), 2, 353),
+                                             ((4, 20, 52), 2, 9), ((4, 4, 4), 2, None), ((96, 48, 56), 3, None)])
+def test_block_rows_fp32(ne, levels, layer):
+    from voxelfem_amd import capi
+
+    capi.set_kernel_variant(3)  # block rows on level 1
+    try:
+        mg, om = pair(ne, levels, layer)
+        r = np.random.default_rng(5).normal(size=(om.num_nodes(0), 3))
+        n = np.arange(len(r))
+        r[n // ((ne[1] + 1) * (ne[2] + 1)) == 0] = 0
+        if layer is not None:
+            r[n // (ne[2] + 1) % (ne[1] + 1) > layer] = 0
+        for fmg, nu in ((False, 1), (True, 2)):
+            assert rel(mg._precondition(r, 1, nu, fmg, "fp32"), mg._precondition(r, 1, nu, fmg, "fp64")) < 1e-5
+    finally:
+        capi.set_kernel_variant(0)
+
+
 # the marching smoothing filter: tiles of 8 or 16 rows by 64 columns, reaches 1 to 4, sides below the reach (repeated
 # reflection), real radii, constant weights; sums of up to 729 positive terms in another order: 1e-13
 @pytest.mark.parametrize("dims", [(1, 1, 1), (2, 3, 1), (5, 8, 64), (7, 9, 65), (3, 17, 130), (40, 16, 63)])

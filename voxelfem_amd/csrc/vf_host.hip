@@ -1200,13 +1200,13 @@ struct vf_mg {
         if (L >= 2 && l1Blocks && !l1_blocks_unused(p)) {
             LevelData &c1 = *lv[1];
             DBuf<T> &buf = block_buf<T>(1);
-            buf.resize(block_storage(c1.g));
+            buf.resize(BlockRows<T>::storage(c1.g));
             launch_assemble_l1_blocks<T>(c1.g, lv[0]->g, dChat.data(), sim->E.data(), buf.data(), sim->structured, s);
         }
         for (int l = 2; l < L; ++l) {
             LevelData &c = *lv[l];
             DBuf<T> &buf = block_buf<T>(l);
-            buf.resize(block_storage(c.g));
+            buf.resize(BlockRows<T>::storage(c.g));
             launch_assemble_blocks<T>(c.g, c.Ke.data(), buf.data(), s);
         }
         blocksReady[p] = true;

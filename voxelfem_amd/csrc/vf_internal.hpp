@@ -94,28 +94,45 @@ struct DBuf {
 enum ApplyMode { AM_SET = 0, AM_ADD = 1, AM_SUB = 2, AM_RESIDUAL = 3 };
 
 // Assembled block rows (levels 1..L-1) are stored colour-major: the nodes of colour
-// c = 4(ix%2) + 2(iy%2) + (iz%2) form a class of cnt_c nodes numbered j = ((ix/2) my + iy/2) mz + iz/2
-// (m_ = nodes of that parity along each axis) and classes follow each other in colour order, each padded to a
-// multiple of BLOCK_GROUP nodes. Inside a class the rows of four consecutive nodes are interleaved: entry k = 3 a + c
-// of neighbour slot s of node j sits at ((j / 4 * 9 + k) * 27 + s) * 4 + j % 4. A wavefront that gives each of four
-// nodes sixteen lanes, one per neighbour slot, so reads contiguous memory, and a pass over one colour streams it.
-constexpr int BLOCK_GROUP = 4;
-__host__ __device__ inline size_t block_class_nodes(const Grid &g, int c) {  // padded node count of a class
-    const size_t mx = (g.nn[0] - ((c >> 2) & 1) + 1) / 2, my = (g.nn[1] - ((c >> 1) & 1) + 1) / 2,
-                 mz = (g.nn[2] - (c & 1) + 1) / 2;
-    return (mx * my * mz + BLOCK_GROUP - 1) / BLOCK_GROUP * BLOCK_GROUP;
-}
-__host__ __device__ inline size_t block_class_base(const Grid &g, int c) {  // padded nodes of the classes before c
-    size_t before = 0;
-    for (int q = 0; q < c; ++q) before += block_class_nodes(g, q);
-    return before;
-}
-inline size_t block_storage(const Grid &g) { return block_class_base(g, 8) * 243; }  // values of a whole level
-// offset of entry 0 of slot 0 of node j inside a level whose class starts at padded node `base`; entry k of slot s
-// is (k * 27 + s) * BLOCK_GROUP further on
-__host__ __device__ inline size_t block_offset(size_t base, int j) {
-    return (base + (size_t)(j / BLOCK_GROUP) * BLOCK_GROUP) * 243 + j % BLOCK_GROUP;
-}
+// c = 4(ix%2) + 2(iy%2) + (iz%2) form a class of nodes numbered j = ((ix/2) my + iy/2) mz + iz/2 (m_ = nodes of that
+// parity along each axis; mz rounded up to a multiple of LANE) and classes follow each other in colour order, each padded
+// to a multiple of GROUP nodes. Inside a class the rows of four consecutive nodes are interleaved: entry k = 3 a + c of
+// neighbour slot s of node j sits at ((j / GROUP * 9 + k) * 27 + s) * GROUP + j % GROUP. A wavefront that gives sixteen
+// lanes, one per neighbour slot, to each LANE nodes so reads contiguous memory, eight bytes a lane (LANE neighbouring
+// nodes of one z-row), and a pass over one colour streams it.
+template <typename T>
+struct BlockRows {
+    static constexpr int LANE = 8 / sizeof(T), GROUP = 4;
+    __host__ __device__ static int row_nodes(const Grid &g, int cz) {  // mz
+        return ((g.nn[2] - cz + 1) / 2 + LANE - 1) / LANE * LANE;
+    }
+    __host__ __device__ static size_t class_nodes(const Grid &g, int c) {  // padded node count of a class
+        const size_t mx = (g.nn[0] - ((c >> 2) & 1) + 1) / 2, my = (g.nn[1] - ((c >> 1) & 1) + 1) / 2;
+        return (mx * my * row_nodes(g, c & 1) + GROUP - 1) / GROUP * GROUP;
+    }
+    __host__ __device__ static size_t class_base(const Grid &g, int c) {  // padded nodes of the classes before c
+        size_t before = 0;
+        for (int q = 0; q < c; ++q) before += class_nodes(g, q);
+        return before;
+    }
+    static size_t storage(const Grid &g) { return class_base(g, 8) * 243; }  // values of a whole level
+    struct Bases {
+        size_t at[8];
+    };
+    static Bases bases(const Grid &g) {  // of all classes
+        Bases b;
+        for (int c = 0; c < 8; ++c) b.at[c] = class_base(g, c);
+        return b;
+    }
+    // offset of entry 0 of slot 0 of node (2 jx + cx, 2 jy + cy, 2 jz + cz) of colour c, whose class starts at padded
+    // node `base`
+    __host__ __device__ static size_t offset(const Grid &g, size_t base, int c, int jx, int jy, int jz) {
+        const size_t j = ((size_t)jx * ((g.nn[1] - ((c >> 1) & 1) + 1) / 2) + jy) * row_nodes(g, c & 1) + jz;
+        return (base + j / GROUP * GROUP) * 243 + j % GROUP;
+    }
+    // of entry k of slot s, from there
+    __host__ __device__ static constexpr int entry(int k, int s) { return (k * 27 + s) * GROUP; }
+};
 
 // fine level (TPSStencils.hh:431-728).  AM_SET: y = K u (detached rows zeroed);
 // AM_RESIDUAL: y = b - K u on active rows; dmask != nullptr zeroes constrained output components.

@@ -80,10 +80,19 @@ __device__ __forceinline__ void gs_update(T *u, int N, int n, const T bms[3], co
     T ud[3];
     if (dm) {
         ud[0] = ud[1] = ud[2] = T(0);
-        for (int t = 0; t < 3; ++t) {
-            const int i = forward ? t : 2 - t;
+        auto point = [&](int i) {
             const T fr = (dm & (1 << i)) ? T(0) : T(1);
             ud[i] = (bms[i] - (M[3 * i] * ud[0] + M[3 * i + 1] * ud[1] + M[3 * i + 2] * ud[2])) * (fr / M[4 * i]);
+        };
+        // no index that is only known at run time: the arrays stay in registers
+        if (forward) {
+            point(0);
+            point(1);
+            point(2);
+        } else {
+            point(2);
+            point(1);
+            point(0);
         }
     } else {
         inv3_apply(M, bms, ud);
@@ -528,13 +537,16 @@ __global__ void __launch_bounds__(TPB, sizeof(T) == 8 ? 2 : 4) k_l1_apply_sep(Gr
 }
 
 // ------------------------------------------------------------------ assembled block rows
-// One node is worked on by the sixteen lanes of one DPP row: lane p holds neighbour slots p and p + 16 (27 in all), so
-// a node's 243 block entries and 81 neighbour values are requested at once, in one round of loads, and the row is
-// summed by four DPP exchanges without LDS. A colour pass over a small level is bound by that one memory round
-// instead of the three dependent rounds (and 81 loads per work-item) of four work-items per node; over a large level
-// it streams the interleaved rows (105 x 57 x 49 nodes in FP64: 20 us per colour, 3.6 TB/s). Time per colour, before
-// and after, averaged over the block levels of a hierarchy: 64 x 32 x 32 FP64 10.4 -> 4.3 us, 176 x 88 x 72 FP64
-// 13.6 -> 7.5 us, 208 x 112 x 96 FP64 16.2 -> 9.9 us, 384 x 192 x 192 FP32 9.5 -> 7.6 us.
+// LANE nodes (one in FP64, two neighbours of a z-row in FP32: eight bytes of every block entry) are worked on by the
+// sixteen lanes of one DPP row: lane p holds neighbour slots p and p + 16 (27 in all), so the nodes' 243 block entries
+// and 81 neighbour values each are requested at once, in one round of loads, and the rows are summed by four DPP
+// exchanges without LDS. A colour pass over a small level is bound by that one memory round; over a large level it
+// streams the interleaved rows.
+// Time per colour, averaged over the block levels of a hierarchy: 64 x 32 x 32 FP64 10.4 -> 4.3 us, 176 x 88 x 72 FP64
+// 13.6 -> 7.5 us, 208 x 112 x 96 FP64 16.2 -> 9.9 us (before: four work-items per node). In FP32 one node per row of lanes
+// reads four bytes a lane, which no level of 100,000 nodes or more can be streamed with: sweeps and residuals of
+// 97 x 49 x 49 nodes 105 and 77 us with one node, 71 and 44 with two, of 193 x 97 x 97 nodes 655 and 610, 454 and 429 (FP64
+// 839 and 820 us, 4.2 TB/s).
 // sum over the sixteen lanes of a DPP row, the same in every lane
 template <typename T>
 __device__ __forceinline__ T row16_sum(T v) {
@@ -548,45 +560,96 @@ __device__ __forceinline__ T row16_sum(T v) {
 // tile and workgroup of the two-launch sweep: 28 of the 32 rows of lanes hold a node at the first colour
 constexpr int BP_TY = 4, BP_TZ = 12, BP_NT = 512, CUS = 256;
 
-constexpr int RL = 16;       // lanes per node
-constexpr int RN16 = TPB / RL;  // nodes per workgroup
-constexpr int DIAG_LANE = 13;   // the lane that holds the node's own slot
+constexpr int RL = 16;          // lanes per node
+constexpr int RN16 = TPB / RL;  // rows of lanes per workgroup
+constexpr int DIAG_LANE = 13;   // the lane that holds the nodes' own slot
 
-// this lane's part of row f = sum_s B_s u_s of the node (ix, iy, iz) whose rows start at bp; M: the entries of slot p
+// A row's results are written by lane 13 (its first node) and lane 12 (its second): which node is this lane's, if any
 template <typename T>
-__device__ __forceinline__ void block_row16(const Grid &g, const T *__restrict__ bp, int p, int ix, int iy, int iz,
+__device__ __forceinline__ int lane_node(int p) {
+    return p == DIAG_LANE ? 0 : BlockRows<T>::LANE == 2 && p == DIAG_LANE - 1 ? 1 : BlockRows<T>::LANE;
+}
+
+// LANE neighbouring nodes of a z-row of one colour: the first one's coordinates and index, how many there are
+struct LaneNodes {
+    int ix, iy, iz, n, count;
+    size_t at;  // entry 0 of slot 0 of their block rows
+};
+template <typename T>
+__device__ __forceinline__ bool lane_nodes(const Grid &g, size_t base, int c, int row, LaneNodes &r) {
+    constexpr int LANE = BlockRows<T>::LANE;
+    const int cx = (c >> 2) & 1, cy = (c >> 1) & 1, cz = c & 1;
+    const int mx = (g.nn[0] - cx + 1) / 2, my = (g.ydet - cy + 1) / 2, mz = (g.nn[2] - cz + 1) / 2;
+    const int mq = BlockRows<T>::row_nodes(g, cz) / LANE;
+    if (row >= mx * my * mq) return false;
+    const int jx = row / (my * mq), q = row - jx * my * mq, jy = q / mq, jz = (q - jy * mq) * LANE;
+    r.ix = 2 * jx + cx;
+    r.iy = 2 * jy + cy;
+    r.iz = 2 * jz + cz;
+    r.n = (r.ix * g.nn[1] + r.iy) * g.nn[2] + r.iz;
+    r.count = min(LANE, mz - jz);
+    r.at = BlockRows<T>::offset(g, base, c, jx, jy, jz);
+    return true;
+}
+
+// row f = sum_s B_s u_s and, with WANT_M, diagonal block M of node lane_node(p) of the nodes r
+template <typename T, bool WANT_M>
+__device__ __forceinline__ void block_row16(const Grid &g, const T *__restrict__ blocks, int p, const LaneNodes &r,
                                             const T *__restrict__ u, T f[3], T M[9]) {
+    using R = BlockRows<T>;
     const int N = g.nnodes, sy = g.nn[2], sx = g.nn[1] * sy;
-    const int n = ix * sx + iy * sy + iz;
-    T B[2][9], un[2][3];
+    T B[2][9][R::LANE], un[2][R::LANE][3];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
         const bool real = p + RL * h < 27;
         const int s = real ? p + RL * h : 26;  // the idle lanes of the second half repeat slot 26 with u = 0
         const int q = (s * 171) >> 9;          // s / 3
         const int dx = ((s * 57) >> 9) - 1, dy = q - 3 * (dx + 1) - 1, dz = s - 3 * q - 1;
-        const bool ok = real && (unsigned)(ix + dx) < (unsigned)g.nn[0] && (unsigned)(iy + dy) < (unsigned)g.nn[1] &&
-                        (unsigned)(iz + dz) < (unsigned)g.nn[2];
-        const int m = ok ? n + dx * sx + dy * sy + dz : n;
+        const bool okxy = real && (unsigned)(r.ix + dx) < (unsigned)g.nn[0] && (unsigned)(r.iy + dy) < (unsigned)g.nn[1];
 #pragma unroll
-        for (int k = 0; k < 9; ++k) B[h][k] = bp[(k * 27 + s) * BLOCK_GROUP];
+        for (int k = 0; k < 9; ++k) {
+            const T *e = blocks + (r.at + R::entry(k, s));
+            if constexpr (R::LANE == 2) {
+                const float2 v = *reinterpret_cast<const float2 *>(e);
+                B[h][k][0] = v.x;
+                B[h][k][1] = v.y;
+            } else {
+                B[h][k][0] = *e;
+            }
+        }
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            const T v = u[(size_t)c * N + m];
-            un[h][c] = ok ? v : T(0);
+        for (int e = 0; e < R::LANE; ++e) {
+            const bool ok = okxy && (unsigned)(r.iz + 2 * e + dz) < (unsigned)g.nn[2];
+            const int m = ok ? r.n + dx * sx + dy * sy + dz + 2 * e : r.n;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                const T v = u[(size_t)c * N + m];
+                un[h][e][c] = ok ? v : T(0);
+            }
         }
     }
+    const bool second = lane_node<T>(p) == 1;
 #pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        T acc = B[0][3 * a] * un[0][0];
-        acc += B[0][3 * a + 1] * un[0][1];
-        acc += B[0][3 * a + 2] * un[0][2];
+    for (int e = 0; e < R::LANE; ++e)
 #pragma unroll
-        for (int c = 0; c < 3; ++c) acc += B[1][3 * a + c] * un[1][c];
-        f[a] = row16_sum(acc);
-    }
+        for (int a = 0; a < 3; ++a) {
+            T acc = B[0][3 * a][e] * un[0][e][0];
+            acc += B[0][3 * a + 1][e] * un[0][e][1];
+            acc += B[0][3 * a + 2][e] * un[0][e][2];
 #pragma unroll
-    for (int k = 0; k < 9; ++k) M[k] = B[0][k];
+            for (int c = 0; c < 3; ++c) acc += B[1][3 * a + c][e] * un[1][e][c];
+            acc = row16_sum(acc);
+            f[a] = e == 0 || second ? acc : f[a];
+        }
+    if (WANT_M)
+#pragma unroll
+        for (int k = 0; k < 9; ++k) {
+            M[k] = B[0][k][0];
+            if constexpr (R::LANE == 2) {
+                const T v = dpp_get<0xE5>(B[0][k][1]);  // quad_perm [1, 1, 2, 3]: lane 12 takes lane 13's
+                M[k] = second ? v : M[k];
+            }
+        }
 }
 
 // grid.y = colour class (the rows are stored by class)
@@ -594,42 +657,36 @@ template <typename T, int MODE>
 __global__ void __launch_bounds__(TPB) k_block_apply(Grid g, const T *__restrict__ blocks, const T *__restrict__ u,
                                                      T *__restrict__ y, const T *__restrict__ b,
                                                      const uint8_t *__restrict__ dmask) {
-    const int col = blockIdx.y, cx = (col >> 2) & 1, cy = (col >> 1) & 1, cz = col & 1;
-    const int mx = (g.nn[0] - cx + 1) / 2, my = (g.ydet - cy + 1) / 2, mz = (g.nn[2] - cz + 1) / 2;
-    const int node = blockIdx.x * RN16 + threadIdx.x / RL, p = threadIdx.x % RL;
-    if (node >= mx * my * mz) return;
-    const int jx = node / (my * mz), r = node - jx * my * mz, jy = r / mz, jz = r - jy * mz;
-    const int ix = 2 * jx + cx, iy = 2 * jy + cy, iz = 2 * jz + cz;
-    const int n = (ix * g.nn[1] + iy) * g.nn[2] + iz;
-    const int j = (jx * ((g.nn[1] - cy + 1) / 2) + jy) * mz + jz;
-    T f[3], M[9];
-    block_row16<T>(g, blocks + block_offset(block_class_base(g, col), j), p, ix, iy, iz, u, f, M);
-    if (p == DIAG_LANE) store_out(y, b, g.nnodes, n, f, MODE, dmask ? dmask[n] : uint8_t(0));
+    const int p = threadIdx.x % RL, e = lane_node<T>(p);
+    LaneNodes r;
+    if (!lane_nodes<T>(g, BlockRows<T>::class_base(g, blockIdx.y), blockIdx.y, blockIdx.x * RN16 + threadIdx.x / RL, r))
+        return;
+    T f[3];
+    block_row16<T, false>(g, blocks, p, r, u, f, nullptr);
+    const int n = r.n + 2 * e;
+    if (e < r.count) store_out(y, b, g.nnodes, n, f, MODE, dmask ? dmask[n] : uint8_t(0));
 }
 
-// One colour of the block Gauss-Seidel sweep; lane 13 of a node's sixteen, which holds the diagonal block, updates it.
+// One colour of the block Gauss-Seidel sweep; the lanes that hold the diagonal blocks update the nodes.
 template <typename T>
 __global__ void __launch_bounds__(TPB) k_block_gs(Grid g, const T *__restrict__ blocks, T *__restrict__ u,
                                                   const T *__restrict__ b, const uint8_t *__restrict__ dmask,
-                                                  size_t base, int cx, int cy, int cz, int forward) {
-    const int mx = (g.nn[0] - cx + 1) / 2, my = (g.ydet - cy + 1) / 2, mz = (g.nn[2] - cz + 1) / 2;
-    const int node = blockIdx.x * RN16 + threadIdx.x / RL, p = threadIdx.x % RL;
-    if (node >= mx * my * mz) return;
-    const int jx = node / (my * mz), r = node - jx * my * mz, jy = r / mz, jz = r - jy * mz;
-    const int ix = 2 * jx + cx, iy = 2 * jy + cy, iz = 2 * jz + cz;
-    const int N = g.nnodes, n = (ix * g.nn[1] + iy) * g.nn[2] + iz;
-    const int j = (jx * ((g.nn[1] - cy + 1) / 2) + jy) * mz + jz;
-    // requested with the row, so that the update waits for no second round
-    uint8_t dm = 0;
+                                                  size_t base, int colour, int forward) {
+    const int p = threadIdx.x % RL, e = lane_node<T>(p), N = g.nnodes;
+    LaneNodes r;
+    if (!lane_nodes<T>(g, base, colour, blockIdx.x * RN16 + threadIdx.x / RL, r)) return;
+    // requested with the rows, so that the update waits for no second round
+    const int n = r.n + 2 * e;
+    uint8_t dm = 7;
     T bn[3] = {0, 0, 0};
-    if (p == DIAG_LANE) {
-        if (dmask) dm = dmask[n];
+    if (e < r.count) {
+        dm = dmask ? dmask[n] : uint8_t(0);
 #pragma unroll
         for (int c = 0; c < 3; ++c) bn[c] = b[(size_t)c * N + n];
     }
     T f[3], M[9];
-    block_row16<T>(g, blocks + block_offset(base, j), p, ix, iy, iz, u, f, M);
-    if (p == DIAG_LANE && dm != 7) {
+    block_row16<T, true>(g, blocks, p, r, u, f, M);
+    if (dm != 7) {
         const T bms[3] = {bn[0] - f[0], bn[1] - f[1], bn[2] - f[2]};
         gs_update(u, N, n, bms, M, dm, forward);
     }
@@ -647,7 +704,8 @@ __global__ void __launch_bounds__(TPB) k_block_gs(Grid g, const T *__restrict__ 
 // uin: the planes of this parity before the sweep, unb: the neighbour planes, uout (!= uin): receives this parity's
 // planes, every node. zin bit 0 / 1: uin / unb is zero.
 template <typename T, int TY, int TZ, int NT, bool FWD>
-__global__ void __launch_bounds__(NT) k_block_gs_plane(Grid g, const T *__restrict__ blocks, const T *__restrict__ uin,
+__global__ void __launch_bounds__(NT) k_block_gs_plane(Grid g, typename BlockRows<T>::Bases bases,
+                                                       const T *__restrict__ blocks, const T *__restrict__ uin,
                                                        const T *__restrict__ unb, T *__restrict__ uout,
                                                        const T *__restrict__ b, const uint8_t *__restrict__ dmask,
                                                        int parity, int ntY, int ntZ, int zin) {
@@ -690,15 +748,15 @@ __global__ void __launch_bounds__(NT) k_block_gs_plane(Grid g, const T *__restri
         const int wr = row / ncs;
         const int iy = act[pos] ? ya + 2 * wr : cy, iz = act[pos] ? za + 2 * (row - wr * ncs) : cz;
         const int n = (ix * ny + iy) * nz + iz;
-        const int my = (ny - cy + 1) / 2, mz = (nz - cz + 1) / 2;
-        const size_t bo = block_offset(block_class_base(g, 4 * parity + sub), ((ix >> 1) * my + (iy >> 1)) * mz + (iz >> 1));
+        const int col = 4 * parity + sub;
+        const size_t bo = BlockRows<T>::offset(g, bases.at[col], col, ix >> 1, iy >> 1, iz >> 1);
         li[pos] = act[pos] ? (iy - y0 + HY) * RZ + iz - z0 + HZ : HY * RZ + HZ;
         dm[pos] = 7;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const bool ok = (unsigned)(iy + dy[h]) < (unsigned)ny && (unsigned)(iz + dz[h]) < (unsigned)nz;
 #pragma unroll
-            for (int k = 0; k < 9; ++k) B[pos][h][k] = act[pos] ? blocks[bo + (k * 27 + slot[h]) * BLOCK_GROUP] : T(0);
+            for (int k = 0; k < 9; ++k) B[pos][h][k] = act[pos] ? blocks[bo + BlockRows<T>::entry(k, slot[h])] : T(0);
 #pragma unroll
             for (int c = 0; c < 3; ++c) un[pos][h][c] = act[pos] && okx[h] && ok ? unb[(size_t)c * N + n + off[h]] : T(0);
             if (h == hp) okp[pos] = inplane && ok;
@@ -951,10 +1009,17 @@ void launch_l1_apply(const Grid &gc, const Grid &gf, const T *Chat, const L1Coef
     VF_HIP(hipGetLastError());
 }
 
+// rows of lanes that a colour's active nodes take
+template <typename T>
+static long block_lane_rows(const Grid &g, int color) {
+    const long mx = (g.nn[0] - ((color >> 2) & 1) + 1) / 2, my = (g.ydet - ((color >> 1) & 1) + 1) / 2;
+    return mx * my * (BlockRows<T>::row_nodes(g, color & 1) / BlockRows<T>::LANE);
+}
+
 template <typename T>
 void launch_block_apply(const Grid &g, const T *blocks, const T *u, T *y, const T *b, const uint8_t *dmask, int mode,
                         hipStream_t s) {
-    const long most = (long)((g.nn[0] + 1) / 2) * ((g.ydet + 1) / 2) * ((g.nn[2] + 1) / 2);
+    const long most = block_lane_rows<T>(g, 0);
     if (most > 0)
         VF_DISPATCH_MODE(k_block_apply, T, mode, dim3((unsigned)((most + RN16 - 1) / RN16), 8), g, blocks, u, y, b, dmask);
     if (mode == AM_SET && g.ydet < g.nn[1]) {
@@ -1006,11 +1071,10 @@ void launch_l1_gs(const Grid &gc, const Grid &gf, const T *Chat, const L1Coef &s
 template <typename T>
 void launch_block_gs(const Grid &g, const T *blocks, T *u, const T *b, const uint8_t *dmask, int color, int forward,
                      hipStream_t s) {
-    const int cx = (color >> 2) & 1, cy = (color >> 1) & 1, cz = color & 1;
-    const long count = color_count(g, cx, cy, cz);
-    if (!count) return;
-    hipLaunchKernelGGL(k_block_gs<T>, dim3((unsigned)((count + RN16 - 1) / RN16)), dim3(TPB), 0, s, g, blocks, u, b, dmask,
-                       block_class_base(g, color), cx, cy, cz, forward);
+    const long rows = block_lane_rows<T>(g, color);
+    if (rows <= 0) return;
+    hipLaunchKernelGGL(k_block_gs<T>, dim3((unsigned)((rows + RN16 - 1) / RN16)), dim3(TPB), 0, s, g, blocks, u, b, dmask,
+                       BlockRows<T>::class_base(g, color), color, forward);
     VF_HIP(hipGetLastError());
 }
 
@@ -1032,10 +1096,10 @@ void launch_block_gs_plane(const Grid &g, const T *blocks, const T *uin, const T
     const int ntY = (g.nn[1] + BP_TY - 1) / BP_TY, ntZ = (g.nn[2] + BP_TZ - 1) / BP_TZ;
     if (forward)
         hipLaunchKernelGGL((k_block_gs_plane<T, BP_TY, BP_TZ, BP_NT, true>), dim3(ntY * ntZ, planes), dim3(BP_NT), 0, s, g,
-                           blocks, uin, unb, uout, b, dmask, parity, ntY, ntZ, zin);
+                           BlockRows<T>::bases(g), blocks, uin, unb, uout, b, dmask, parity, ntY, ntZ, zin);
     else
         hipLaunchKernelGGL((k_block_gs_plane<T, BP_TY, BP_TZ, BP_NT, false>), dim3(ntY * ntZ, planes), dim3(BP_NT), 0, s, g,
-                           blocks, uin, unb, uout, b, dmask, parity, ntY, ntZ, zin);
+                           BlockRows<T>::bases(g), blocks, uin, unb, uout, b, dmask, parity, ntY, ntZ, zin);
     VF_HIP(hipGetLastError());
 }
 

@@ -133,12 +133,13 @@ __global__ void __launch_bounds__(576) k_galerkin_recurse(Grid gc, Grid gf, cons
 // lm = 4 (i + ox) + 2 (jj + oy) + (k + oz). The 27 slots split into three groups of nine by ox; in group ox
 // only the elements with lx = i + ox in {0, 1} contribute, and for one element and one matrix row 3 ln + a
 // the twelve entries 3 lm + c of that group (lx fixed) are contiguous. A work-item holds one group's 81
-// FP64 sums in registers, so every element datum it needs is read once per group; four neighbouring
-// work-items' rows are interleaved in the block layout (block_offset).
+// FP64 sums in registers, so every element datum it needs is read once per group; neighbouring work-items'
+// rows are interleaved in the block layout (BlockRows).
 struct ClassNode {
     int ix, iy, iz;
     size_t at;  // entry 0 of slot 0 of the node's block rows
 };
+template <typename OutT>
 __device__ inline bool class_node(const Grid &g, int colour, ClassNode &r) {
     const int cx = (colour >> 2) & 1, cy = (colour >> 1) & 1, cz = colour & 1;
     const int mx = (g.nn[0] - cx + 1) / 2, my = (g.nn[1] - cy + 1) / 2, mz = (g.nn[2] - cz + 1) / 2;
@@ -148,7 +149,7 @@ __device__ inline bool class_node(const Grid &g, int colour, ClassNode &r) {
     r.ix = 2 * jx + cx;
     r.iy = 2 * jy + cy;
     r.iz = 2 * jz + cz;
-    r.at = block_offset(block_class_base(g, colour), j);
+    r.at = BlockRows<OutT>::offset(g, BlockRows<OutT>::class_base(g, colour), colour, jx, jy, jz);
     return true;
 }
 
@@ -158,7 +159,7 @@ template <typename OutT>
 __global__ void __launch_bounds__(TPB) k_assemble_blocks(Grid g, const double *__restrict__ Ke,
                                                          OutT *__restrict__ blocks, int nylo, int nyhi) {
     ClassNode n;
-    if (!class_node(g, blockIdx.y, n)) return;
+    if (!class_node<OutT>(g, blockIdx.y, n)) return;
     if (n.iy < nylo || n.iy > nyhi) return;
     OutT *out = blocks + n.at;
     for (int gx = 0; gx < 3; ++gx) {
@@ -201,7 +202,7 @@ __global__ void __launch_bounds__(TPB) k_assemble_blocks(Grid g, const double *_
                 }
         }
 #pragma unroll
-        for (int q = 0; q < 81; ++q) out[((q % 9) * 27 + gx * 9 + q / 9) * BLOCK_GROUP] = (OutT)acc[q];
+        for (int q = 0; q < 81; ++q) out[BlockRows<OutT>::entry(q % 9, gx * 9 + q / 9)] = (OutT)acc[q];
     }
 }
 
@@ -221,7 +222,7 @@ __global__ void __launch_bounds__(TPB) k_assemble_l1_blocks(Grid gc, Grid gf, co
                                                             const double *__restrict__ Ef,
                                                             OutT *__restrict__ blocks, int nylo, int nyhi) {
     ClassNode n;
-    if (!class_node(gc, blockIdx.y, n)) return;
+    if (!class_node<OutT>(gc, blockIdx.y, n)) return;
     if (n.iy < nylo || n.iy > nyhi) return;
     const int eyEnd = min(gc.ne[1], gc.ymask);
     const int fz = gf.ne[2], fyz = gf.ne[1] * gf.ne[2];
@@ -306,7 +307,7 @@ __global__ void __launch_bounds__(TPB) k_assemble_l1_blocks(Grid gc, Grid gf, co
             }
         }
 #pragma unroll
-        for (int q = 0; q < 27; ++q) out[((q % 9) * 27 + gxy * 3 + q / 9) * BLOCK_GROUP] = (OutT)acc[q];
+        for (int q = 0; q < 27; ++q) out[BlockRows<OutT>::entry(q % 9, gxy * 3 + q / 9)] = (OutT)acc[q];
     }
 }
 
