@@ -82,8 +82,10 @@ def test_block_rows_fp32(ne, levels, layer):
 
 
 # the marching smoothing filter: tiles of 8 or 16 rows by 64 columns, reaches 1 to 4, sides below the reach (repeated
-# reflection), real radii, constant weights; sums of up to 729 positive terms in another order: 1e-13
-@pytest.mark.parametrize("dims", [(1, 1, 1), (2, 3, 1), (5, 8, 64), (7, 9, 65), (3, 17, 130), (40, 16, 63)])
+# reflection), real radii, constant weights; thin grids (the last two) sum tap by tap; sums of up to 729 positive terms in
+# another order: 1e-13
+@pytest.mark.parametrize("dims", [(1, 1, 1), (2, 3, 1), (5, 8, 64), (7, 9, 65), (3, 17, 130), (40, 16, 63), (700, 300, 1),
+                                  (60000, 1, 1)])
 @pytest.mark.parametrize("rmin,linear", [(2.0, True), (3.0, True), (4.0, True), (5.0, True), (2.5, True), (3.7, True),
                                          (3.0, False), (4.0, False), (6.0, True)])
 def test_smoothing_march(dims, rmin, linear):

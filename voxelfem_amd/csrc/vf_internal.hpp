@@ -390,9 +390,10 @@ void launch_self_weight(const Grid &g, const double *rho, const double *grav, do
 // filters / optimiser
 // y += a x
 void launch_axpy_plain(size_t n, double a, const double *x, double *y, hipStream_t s);
-// the folded marching form for kernels reaching 1 <= R <= 4 voxels (W: sum of the weights); false: not launched
-bool launch_smoothing_filter_march(const int dims[3], int R, double rmin, int type, double W, const double *in, double *out,
-                                   hipStream_t s);
+// the folded marching form for kernels reaching 1 <= R <= 4 voxels (W: sum of the weights, taps: how many); false: not
+// launched
+bool launch_smoothing_filter_march(const int dims[3], int R, double rmin, int type, double W, long taps, const double *in,
+                                   double *out, hipStream_t s);
 void launch_smoothing_filter(const int dims[3], double rmin, int type, const double *in, double *out, hipStream_t s);
 // UpsampleFilter / VertexToCellFilter on an nd-dimensional grid of inDims values (adjoint: in holds the output
 // grid's gradient, out the input grid's); LangelaarFilter on a planar nx x ny grid (lam: nx ny scratch)

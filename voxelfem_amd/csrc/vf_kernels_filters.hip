@@ -432,7 +432,8 @@ __global__ void __launch_bounds__(ST) k_smoothing_march(int d0, int d1, int d2, 
 #pragma unroll
     for (int q = 0; q < NL; ++q) {
         const int e = min(t + q * ST, PLANE - 1);
-        off[q] = reflect_cell(y0 - R + e / RZ, d1) * d2 + reflect_cell(z0 - R + e % RZ, d2);
+        // cells further out than the reach are read by no output: on a thin grid they would reflect many times over
+        off[q] = reflect_cell(min(y0 - R + e / RZ, d1 + R - 1), d1) * d2 + reflect_cell(min(z0 - R + e % RZ, d2 + R - 1), d2);
     }
     double pf[NL];
     auto fetch = [&](int p) {
@@ -514,20 +515,32 @@ __global__ void __launch_bounds__(ST) k_smoothing_march(int d0, int d1, int d2, 
 
 }  // namespace
 
+// The marching kernel unless tap by tap is faster: a tile holds 64 columns along z and 4 YB rows, so a grid thin along z
+// or y (or long along x and thin in both) is marched mostly through empty lanes. A workgroup's step through one plane
+// costs as much as `cost` taps of the other kernel (half of them when the weights are constant and need no square root),
+// whose voxels each take their taps one after the other, which costs a small grid as much as 260,000 (200,000) voxels more;
+// a launch of the march costs 1000 steps. Measured, march / tap by tap in us: reach 1 (hat) 2000x1000x1 232 / 71,
+// 1000x1000x4 116 / 123, 500x500x16 31 / 124, 300000x1x1 283 / 15; reach 2 (hat) 2000x1000x1 317 / 256, 2000x1000x2 314 /
+// 457; reach 3 (hat) 2000x1000x1 542 / 658, 100000x3x3 367 / 309; 16x12x12, reach 1 to 4: 4.6 / 8.7, 6.9 / 28, 11 / 72,
+// 15 / 145.
 template <int R, int YB, bool HAT>
-static void launch_smoothing_march(const int d[3], const SmoothWeights &sw, double W, const double *in, double *out,
-                                   hipStream_t s) {
+static bool launch_smoothing_march(const int d[3], const SmoothWeights &sw, double W, long taps, bool constant,
+                                   const double *in, double *out, hipStream_t s) {
     constexpr int TY = ST / STZ * YB;
+    constexpr double cost = HAT ? (R == 1 ? 1570 : R == 2 ? 2300 : R == 3 ? 4200 : 2400) : (R == 1 ? 1250 : R == 2 ? 2900 : 6800);
     const int ntY = (d[1] + TY - 1) / TY, ntZ = (d[2] + STZ - 1) / STZ, tiles = ntY * ntZ;
     const int chunks = plane_chunks(tiles, d[0], 1024, resident_workgroups((const void *)k_smoothing_march<R, YB, HAT>, ST));
-    const int xchunk = (d[0] + chunks - 1) / chunks;
-    hipLaunchKernelGGL((k_smoothing_march<R, YB, HAT>), dim3(tiles, (d[0] + xchunk - 1) / xchunk), dim3(ST), 0, s, d[0],
-                       d[1], d[2], sw, W, in, out, ntZ, xchunk);
+    const int xchunk = (d[0] + chunks - 1) / chunks, nch = (d[0] + xchunk - 1) / xchunk;
+    const double n = (double)d[0] * d[1] * d[2];
+    if (((double)tiles * nch * (xchunk + 2 * R) + 1000) * cost > (constant ? 0.5 * n + 200000 : n + 260000) * taps) return false;
+    hipLaunchKernelGGL((k_smoothing_march<R, YB, HAT>), dim3(tiles, nch), dim3(ST), 0, s, d[0], d[1], d[2], sw, W, in, out,
+                       ntZ, xchunk);
     VF_HIP(hipGetLastError());
+    return true;
 }
 
-bool launch_smoothing_filter_march(const int dims[3], int R, double rmin, int type, double W, const double *in, double *out,
-                                   hipStream_t s) {
+bool launch_smoothing_filter_march(const int dims[3], int R, double rmin, int type, double W, long taps, const double *in,
+                                   double *out, hipStream_t s) {
     const long n = (long)dims[0] * dims[1] * dims[2];
     if (R < 1 || R > 4 || n <= 0) return false;
     const int NC = (R + 1) * (R + 2) / 2;
@@ -546,15 +559,15 @@ bool launch_smoothing_filter_march(const int dims[3], int R, double rmin, int ty
                 hat = hat && inside == (a * a + b * b + c * c < (R + 1) * (R + 1));
             }
     auto go = [&](auto r, auto yb) {
-        if (hat) launch_smoothing_march<decltype(r)::value, decltype(yb)::value, true>(dims, sw, W, in, out, s);
-        else launch_smoothing_march<decltype(r)::value, decltype(yb)::value, false>(dims, sw, W, in, out, s);
+        constexpr int RR = decltype(r)::value, YB = decltype(yb)::value;
+        return hat ? launch_smoothing_march<RR, YB, true>(dims, sw, W, taps, type != 1, in, out, s)
+                   : launch_smoothing_march<RR, YB, false>(dims, sw, W, taps, type != 1, in, out, s);
     };
     // four outputs per work-item along y; two for R = 4, whose folded rows would not fit the registers
-    if (R == 1) go(std::integral_constant<int, 1>(), std::integral_constant<int, 4>());
-    else if (R == 2) go(std::integral_constant<int, 2>(), std::integral_constant<int, 4>());
-    else if (R == 3) go(std::integral_constant<int, 3>(), std::integral_constant<int, 4>());
-    else go(std::integral_constant<int, 4>(), std::integral_constant<int, 2>());
-    return true;
+    if (R == 1) return go(std::integral_constant<int, 1>(), std::integral_constant<int, 4>());
+    if (R == 2) return go(std::integral_constant<int, 2>(), std::integral_constant<int, 4>());
+    if (R == 3) return go(std::integral_constant<int, 3>(), std::integral_constant<int, 4>());
+    return go(std::integral_constant<int, 4>(), std::integral_constant<int, 2>());
 }
 
 void upsample_dims(int nd, const int64_t *in, int factor, int64_t *out) {

@@ -950,14 +950,18 @@ void launch_axpy_plain(size_t n, double a, const double *x, double *y, hipStream
 void launch_smoothing_filter(const int dims[3], double rmin, int type, const double *in, double *out, hipStream_t s) {
     const int R = (int)ceil(rmin) - 1;
     double W = 0;
+    long taps = 0;
     for (int a = -R; a <= R; ++a)
         for (int b = -R; b <= R; ++b)
             for (int c = -R; c <= R; ++c) {
                 const double w = type == 1 ? rmin - sqrt((double)(a * a + b * b + c * c)) : 1.0;
-                if (w > 0) W += w;
+                if (w > 0) {
+                    W += w;
+                    ++taps;
+                }
             }
-    // reaches of one to four voxels march with the folded kernel; wider ones (and R = 0) sum tap by tap
-    if (launch_smoothing_filter_march(dims, R, rmin, type, W, in, out, s)) return;
+    // reaches of one to four voxels march with the folded kernel; wider ones, R = 0 and thin grids sum tap by tap
+    if (launch_smoothing_filter_march(dims, R, rmin, type, W, taps, in, out, s)) return;
     const long n = (long)dims[0] * dims[1] * dims[2];
     hipLaunchKernelGGL(k_smoothing, dim3(nblocks(n)), dim3(TPB), 0, s, dims[0], dims[1], dims[2], R, rmin, type, W, in,
                        out);
