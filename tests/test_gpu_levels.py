@@ -246,3 +246,48 @@ def test_planar_sweep(ne, levels, layer, fmg, nu, sym):
     r = rng.normal(size=(om.num_nodes(0), 2))
     r[np.arange(len(r)) % (ne[1] + 1) >= (ne[1] if layer is None else layer) + 1] = 0
     assert rel(mg._precondition(r, 2, nu, fmg), om.precondition(r, 2, nu, fmg)) < 1e-11
+
+
+# one and two levels of more than six workgroups per compute unit, whose colours are launches of their own. The second
+# cycle's residual is rounded at u |K| |x|, which the inverse amplifies to u kappa of x: kappa of the finest level is
+# taken as 4^levels times that of the coarsest
+@pytest.mark.parametrize("ne,levels,layer,fmg,nu,sym", [((640, 320), 4, None, False, 2, False),
+                                                        ((1536, 384), 5, 201, True, 1, True)])
+def test_planar_colour_launches(ne, levels, layer, fmg, nu, sym):
+    import voxelfem_amd
+    from oracle import oracle2d as o2
+
+    rho = wl.noise_density(ne, 3, base=0.5, amp=0.4)
+    mg = wl.configure2d(voxelfem_amd.pyVoxelFEM, ne, wl.MBB2D_BC, rho).multigridSolver(levels)
+    s = o2.Sim(ne)
+    s.set_etensor(1.0, 0.3)
+    s.set_law(0, 1.0, 1e-9, 3.0, 3.0)
+    s.set_densities(rho)
+    s.set_dirichlet(wl.mbb2d_mask(ne))
+    om = o2.MG(s, levels)
+    if layer is not None:
+        mg.setFabricationMaskHeightByLayer(layer)
+        om.set_mask_layer(layer)
+    mg.setSymmetricGaussSeidel(sym)
+    om.set_symmetric(sym)
+    mg.updateStiffnessMatrices()
+    om.update_stiffness()
+    rng = np.random.default_rng(7)
+    for l in range(levels):
+        nn = om.num_nodes(l)
+        u, b = rng.normal(size=(nn, 2)), rng.normal(size=(nn, 2))
+        iy = np.arange(nn) % ((ne[1] >> l) + 1)
+        act = np.ones(nn, bool) if layer is None else iy < -(-layer >> l) + 1
+        u[~act] = 0
+        for fwd in (True, False):
+            assert rel(mg._smooth(l, u, b, fwd)[act], om.smooth(l, u, b, fwd)[act]) < 1e-12, (l, fwd)
+    nn = om.num_nodes(levels)
+    A = np.stack([om.apply_K(levels, e.reshape(nn, 2)).ravel() for e in np.eye(2 * nn)])
+    free = (np.diag(A) > 0) & ((np.repeat(om.dirichlet_mask(levels), 2) >> np.tile([0, 1], nn)) & 1 == 0)
+    A = A[np.ix_(free, free)]
+    d = 1 / np.sqrt(np.diag(A))
+    w = np.linalg.eigvalsh(A * d[:, None] * d)
+    r = rng.normal(size=(om.num_nodes(0), 2))
+    r[np.arange(len(r)) % (ne[1] + 1) >= (ne[1] if layer is None else layer) + 1] = 0
+    tol = 2.0 ** -53 * 4 ** levels * w[-1] / w[0]
+    assert rel(mg._precondition(r, 2, nu, fmg), om.precondition(r, 2, nu, fmg)) < tol

@@ -146,6 +146,7 @@ void launch_fine_apply_tiled(const Grid &g, const T *K0, const T *E, const T *u,
                              const uint8_t *dmask, int mode, hipStream_t s);
 // Workgroups of `threads` work-items of `kernel` (static LDS only) that the current device holds at once.
 int resident_workgroups(const void *kernel, int threads);
+int cu_count();  // compute units of the device
 // Chunk count along x for a launch of `tiles` x chunks workgroups that march over `n` planes: about
 // `want` workgroups, never more than `resident` (a workgroup left waiting for a free slot would run its
 // whole chunk after the others finish).

@@ -1017,19 +1017,6 @@ __global__ void __launch_bounds__(256) k_gs_gather_f(Grid g, const T *__restrict
 
 inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
-int cu_count() {
-    static int n = 0;
-    if (!n) {
-        int dev = 0, v = 0;
-        if (hipGetDevice(&dev) == hipSuccess &&
-            hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0)
-            n = v;
-        else
-            n = 256;
-    }
-    return n;
-}
-
 // fine K u tile: 16 x 16 outputs, 256 work-items
 constexpr int KU_TY = 16, KU_TZ = 16, KU_NT = 256;
 // GS tile: up to 16 x GS_TZ outputs, 256 work-items (the four colour positions cover at most 171/162/136/128
@@ -1042,6 +1029,18 @@ template <typename T>
 constexpr int GS_TZ = sizeof(T) == 4 ? 28 : 32;
 
 }  // namespace
+
+int cu_count() {
+    static const int n = [] {
+        int dev = 0, v = 0;
+        if (hipGetDevice(&dev) == hipSuccess &&
+            hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0)
+            return v;
+        (void)hipGetLastError();
+        return 256;
+    }();
+    return n;
+}
 
 int resident_workgroups(const void *kernel, int threads) {
     static std::mutex m;

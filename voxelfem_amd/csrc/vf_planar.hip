@@ -2,9 +2,10 @@
 //
 // The reference instantiates its whole stack for N = 2 (python_bindings/VoxelFEM.cc:301-308): bilinear
 // quads, 2^2 = 4 colours, 3^2 = 9 neighbour blocks per node row. Planar grids are small (the reference's 2D
-// demos use 384 x 192 and 256 x 128 elements, 0.15 M DoF), so the kernels here are one work-item per node
-// or per element entry, FP64 throughout: a planar V-cycle is bound by launch latency, not by HBM or the
-// vector units, and the full fine operator (E_e K0 with 64 doubles of K0) stays in L2.
+// demos use 384 x 192 and 256 x 128 elements, 0.15 M DoF), so a planar V-cycle is bound by launch latency, not by
+// HBM or the vector units, and the full fine operator (E_e K0 with 64 doubles of K0) stays in L2: a sweep is one
+// launch with four lanes per node (k_sweep2), on levels that fill the chip one per colour; the other kernels are one
+// work-item per node or per element entry. FP64 throughout.
 //
 // Levels >= 1 hold element matrices (the Galerkin products of the level below, MultigridSolver.hh:704-819),
 // which the operator, residual and smoother gather per node: the same operators as the reference's
@@ -101,7 +102,7 @@ __global__ void __launch_bounds__(TPB) k_zero_young_rows2(PGrid g, int y0, int y
 template <bool FINE>
 __device__ __forceinline__ void elem_rows(const PGrid &g, const double *__restrict__ K0, const double *__restrict__ E,
                                           const double *__restrict__ Ke, const double *__restrict__ u, int ex, int ey,
-                                          int ln, double out[2]) {
+                                          int ln, double out[2], double M[4]) {
     const int e = ex * g.ne[1] + ey;
     const double *K = FINE ? K0 : Ke + (size_t)e * 64;
     const double s = FINE ? E[e] : 1.0;
@@ -121,19 +122,23 @@ __device__ __forceinline__ void elem_rows(const PGrid &g, const double *__restri
         // two 64-byte lines), instead of one line per entry of a column
         for (int a = 0; a < 8; ++a) t += (FINE ? K[a * 8 + 2 * ln + c] : K[(2 * ln + c) * 8 + a]) * ue[a];
         out[c] += s * t;
+        if (M) {
+            M[2 * c] += s * K[(2 * ln + c) * 8 + 2 * ln];
+            M[2 * c + 1] += s * K[(2 * ln + c) * 8 + 2 * ln + 1];
+        }
     }
 }
 
 template <bool FINE>
 __device__ __forceinline__ void node_Ku(const PGrid &g, const double *K0, const double *E, const double *Ke,
-                                        const double *u, int ix, int iy, double f[2]) {
+                                        const double *u, int ix, int iy, double f[2], double *M) {
 #pragma unroll
     for (int i = 1; i >= 0; --i)
 #pragma unroll
         for (int j = 1; j >= 0; --j) {
             const int ex = ix - i, ey = iy - j;
             if (ex < 0 || ey < 0 || ex >= g.ne[0] || ey >= g.ne[1]) continue;
-            elem_rows<FINE>(g, K0, E, Ke, u, ex, ey, 2 * i + j, f);
+            elem_rows<FINE>(g, K0, E, Ke, u, ex, ey, 2 * i + j, f, M);
         }
 }
 
@@ -150,7 +155,7 @@ __global__ void __launch_bounds__(TPB) k_apply2(PGrid g, const double *__restric
         return;
     }
     double f[2] = {0, 0};
-    node_Ku<FINE>(g, K0, E, Ke, u, ix, iy, f);
+    node_Ku<FINE>(g, K0, E, Ke, u, ix, iy, f, nullptr);
     const double b0 = zeroInit ? 0.0 : y[n], b1 = zeroInit ? 0.0 : y[g.nnodes + n];
     y[n] = negate ? b0 - f[0] : b0 + f[0];
     y[g.nnodes + n] = negate ? b1 - f[1] : b1 + f[1];
@@ -169,7 +174,7 @@ __global__ void __launch_bounds__(TPB) k_residual2(PGrid g, const double *__rest
     const uint8_t dm = dmask[n];
     if (iy < g.ydet) {
         double f[2] = {0, 0};
-        node_Ku<FINE>(g, K0, E, Ke, u, ix, iy, f);
+        node_Ku<FINE>(g, K0, E, Ke, u, ix, iy, f, nullptr);
         r[n] = (dm & 1) ? 0.0 : b[n] - f[0];
         r[g.nnodes + n] = (dm & 2) ? 0.0 : b[g.nnodes + n] - f[1];
     } else if (iy < g.ydet + 4) {
@@ -182,7 +187,7 @@ __global__ void __launch_bounds__(TPB) k_residual2(PGrid g, const double *__rest
 }
 
 // computeResidual on a coarse level with four work-items per node (one per incident element, summed in
-// node_Ku's order by the first of the four): the same values as k_residual2<false>
+// node_Ku's order by the first of the four, as in k_smooth2_x4): the same values as k_residual2<false>
 __global__ void __launch_bounds__(TPB) k_residual2_x4(PGrid g, const double *__restrict__ Ke,
                                                      const uint8_t *__restrict__ dmask, const double *__restrict__ u,
                                                      const double *__restrict__ b, double *__restrict__ r) {
@@ -194,7 +199,7 @@ __global__ void __launch_bounds__(TPB) k_residual2_x4(PGrid g, const double *__r
         const int i = 1 - (p >> 1), j = 1 - (p & 1);
         const int ex = ix - i, ey = iy - j;
         if (ex >= 0 && ey >= 0 && ex < g.ne[0] && ey < g.ne[1])
-            elem_rows<false>(g, nullptr, nullptr, Ke, u, ex, ey, 2 * i + j, v);
+            elem_rows<false>(g, nullptr, nullptr, Ke, u, ex, ey, 2 * i + j, v, nullptr);
     }
     const int q0 = (int)(threadIdx.x & 63) & ~3;
     double f[2];
@@ -218,6 +223,78 @@ __global__ void __launch_bounds__(TPB) k_residual2_x4(PGrid g, const double *__r
         if (dm & 1) r[n] = 0.0;
         if (dm & 2) r[g.nnodes + n] = 0.0;
     }
+}
+
+// one colour of the multicolour block Gauss-Seidel sweep (MultigridSolver.hh:347-379, 408-458): nodes
+// (ox + 2 i, oy + 2 j) of the non-detached rows; the 2 x 2 block solve for free nodes, the point sweep in
+// component order (reversed backwards) for partially constrained ones, fully constrained nodes kept
+__device__ __forceinline__ void gs_update2(const PGrid &g, uint8_t dm, const double f[2], const double M[4],
+                                           double *__restrict__ u, const double *__restrict__ b, int n, int forward) {
+    const double r0 = b[n] - f[0], r1 = b[g.nnodes + n] - f[1];
+    double d0, d1;
+    if (dm) {
+        const double fr0 = (dm & 1) ? 0.0 : 1.0, fr1 = (dm & 2) ? 0.0 : 1.0;
+        if (forward) {
+            d0 = r0 * (fr0 / M[0]);
+            d1 = (r1 - M[2] * d0) * (fr1 / M[3]);
+        } else {
+            d1 = r1 * (fr1 / M[3]);
+            d0 = (r0 - M[1] * d1) * (fr0 / M[0]);
+        }
+    } else {
+        const double id = 1.0 / (M[0] * M[3] - M[1] * M[2]);
+        d0 = (M[3] * r0 - M[1] * r1) * id;
+        d1 = (M[0] * r1 - M[2] * r0) * id;
+    }
+    u[n] += d0;
+    u[g.nnodes + n] += d1;
+}
+__global__ void __launch_bounds__(TPB) k_smooth2(PGrid g, const double *__restrict__ K0, const double *__restrict__ E,
+                                                 const uint8_t *__restrict__ dmask,
+                                                 double *__restrict__ u, const double *__restrict__ b, int ox, int oy,
+                                                 int forward) {
+    const int mx = (g.nn[0] - ox + 1) / 2, my = (g.ydet - oy + 1) / 2;
+    const int t = blockIdx.x * TPB + threadIdx.x;
+    if (my <= 0 || t >= mx * my) return;
+    const int ix = ox + 2 * (t / my), iy = oy + 2 * (t % my);
+    const int n = ix * g.nn[1] + iy;
+    const uint8_t dm = dmask[n];
+    if (dm == 3) return;
+    double f[2] = {0, 0}, M[4] = {0, 0, 0, 0};
+    node_Ku<true>(g, K0, E, nullptr, u, ix, iy, f, M);
+    gs_update2(g, dm, f, M, u, b, n, forward);
+}
+// The same colour step on a coarse level with four work-items per node, one per incident element in node_Ku's
+// order ((1,1), (1,0), (0,1), (0,0)): four times the work-items in flight and a quarter of the dependent gathers
+// each. The first of the four sums the contributions in that order (the coarse products carry no modulus, so
+// the sums equal node_Ku's bit for bit) and updates the node.
+__global__ void __launch_bounds__(TPB) k_smooth2_x4(PGrid g, const double *__restrict__ Ke,
+                                                    const uint8_t *__restrict__ dmask, double *__restrict__ u,
+                                                    const double *__restrict__ b, int ox, int oy, int forward) {
+    const int mx = (g.nn[0] - ox + 1) / 2, my = (g.ydet - oy + 1) / 2;
+    const int tt = blockIdx.x * TPB + threadIdx.x, t = tt >> 2, p = tt & 3;
+    if (my <= 0 || t >= mx * my) return;  // all four work-items of a node
+    const int ix = ox + 2 * (t / my), iy = oy + 2 * (t % my);
+    const int n = ix * g.nn[1] + iy;
+    const uint8_t dm = dmask[n];
+    if (dm == 3) return;  // all four work-items of a node
+    const int i = 1 - (p >> 1), j = 1 - (p & 1);
+    const int ex = ix - i, ey = iy - j;
+    double v[6] = {0, 0, 0, 0, 0, 0};  // f[2], M[4] of this element
+    if (ex >= 0 && ey >= 0 && ex < g.ne[0] && ey < g.ne[1])
+        elem_rows<false>(g, nullptr, nullptr, Ke, u, ex, ey, 2 * i + j, v, v + 2);
+    const int q0 = (int)(threadIdx.x & 63) & ~3;
+    double acc[6];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+        double a = __shfl(v[k], q0, 64);
+        a += __shfl(v[k], q0 + 1, 64);
+        a += __shfl(v[k], q0 + 2, 64);
+        a += __shfl(v[k], q0 + 3, 64);
+        acc[k] = a;
+    }
+    if (p) return;
+    gs_update2(g, dm, acc, acc + 2, u, b, n, forward);
 }
 
 // the value of interpolation at the fine node (ix, iy) (MultigridSolver.hh:178-214)
@@ -1218,9 +1295,35 @@ void PMG::sweep(int l, const double *uin, double *uout, const double *b, bool fo
     }
     check_launch();
 }
+// Tiles recompute their halo (1.4 times the nodes of a sweep, twice with the residual). While a launch is bound by latency
+// that costs nothing, on a full chip more than the launches saved: one launch up to six workgroups per compute unit.
+// V-cycles with one sweep each way in us, one launch per sweep / one per colour on the finest level: 385x193 nodes (833
+// workgroups) 148 / 171, 577x289 (1825) 188 / 193, 769x385 (3201) 266 / 250, 1537x769 (12545) 699 / 568; on the first
+// coarse level: 385x193 269 / 290, 577x289 426 / 429, 769x385 700 / 673.
+bool PMG::one_launch(int l) const {
+    const PGrid &g = lv[l]->g;
+    return (long)((g.nn[0] + SX - 1) / SX) * ((g.nn[1] + SY - 1) / SY) <= 6 * cu_count();
+}
 void PMG::smooth(int l, double *u, const double *b, bool forward) {
-    sweep(l, u, lv[l]->w.data(), b, forward, 0, nullptr, nullptr);
-    d2d(u, lv[l]->w.data(), level_n(l), st());
+    const PGrid &g = lv[l]->g;
+    if (one_launch(l)) {
+        sweep(l, u, lv[l]->w.data(), b, forward, 0, nullptr, nullptr);
+        d2d(u, lv[l]->w.data(), level_n(l), st());
+        return;
+    }
+    const uint8_t *dm = l == 0 ? sim->dmask.data() : lv[l]->dmask.data();
+    for (int t = 0; t < 4; ++t) {
+        const int color = forward ? t : 3 - t, ox = (color >> 1) & 1, oy = color & 1;
+        const size_t cnt = (size_t)((g.nn[0] - ox + 1) / 2) * std::max(0, (g.ydet - oy + 1) / 2);
+        if (!cnt) continue;
+        if (l == 0)
+            hipLaunchKernelGGL(k_smooth2, dim3(nblk(cnt)), dim3(TPB), 0, st(), g, sim->K0.data(), sim->E.data(), dm, u, b,
+                               ox, oy, forward ? 1 : 0);
+        else
+            hipLaunchKernelGGL(k_smooth2_x4, dim3(nblk(4 * cnt)), dim3(TPB), 0, st(), g, lv[l]->Ke.data(), dm, u, b, ox, oy,
+                               forward ? 1 : 0);
+        check_launch();
+    }
 }
 void PMG::restrict_to(int l, const double *fine, double *coarse) {
     hipLaunchKernelGGL(k_restrict2, dim3(nblk(lv[l + 1]->g.nnodes)), dim3(TPB), 0, st(), lv[l]->g, lv[l + 1]->g, fine,
@@ -1258,23 +1361,29 @@ void PMG::vcycle(int l, int nu, bool residualSystem, bool xZero) {
     // components as it reads x, the last before the coarse correction leaves the residual, the first after it adds the
     // correction
     double *cur = p.x.data(), *alt = p.w.data();
-    for (int i = 0; i < nu; ++i) {
+    const bool fused = nu > 0 && one_launch(l);
+    for (int i = 0; fused && i < nu; ++i) {
         sweep(l, cur, alt, p.b.data(), true, i ? 0 : (zd ? 1 : 0) | (xZero ? 2 : 0), i == nu - 1 ? p.r.data() : nullptr,
               nullptr);
         std::swap(cur, alt);
     }
-    if (nu <= 0) {
+    if (!fused) {
         if (xZero) {
             hipLaunchKernelGGL(k_zero_rows2, dim3(nblk(p.g.nnodes)), dim3(TPB), 0, st(), p.g,
                                std::min(p.g.ydet + 4, p.g.nn[1]), p.x.data());
             check_launch();
         }
         if (zd) zero_dirichlet(l, p.x.data());
+        for (int i = 0; i < nu; ++i) smooth(l, p.x.data(), p.b.data(), true);
         residual(l, p.x.data(), p.b.data(), p.r.data());
     }
     restrict_to(l, p.r.data(), c.b.data());
     vcycle(l + 1, nu, true, true);
-    if (nu <= 0) interpolate(l, c.x.data(), p.x.data(), true);
+    if (!fused) {
+        interpolate(l, c.x.data(), p.x.data(), true);
+        for (int i = 0; i < nu; ++i) smooth(l, p.x.data(), p.b.data(), !symmetricGS);
+        return;
+    }
     for (int i = 0; i < nu; ++i) {
         sweep(l, cur, alt, p.b.data(), !symmetricGS, 0, nullptr, i ? nullptr : c.x.data());
         std::swap(cur, alt);

@@ -118,6 +118,7 @@ struct PMG {
     void residual(int l, const double *u, const double *b, double *r);
     void sweep(int l, const double *uin, double *uout, const double *b, bool forward, int mode, double *r,
                const double *xc);
+    bool one_launch(int l) const;  // whether sweeps of the level take the one-launch form
     void smooth(int l, double *u, const double *b, bool forward);
     void restrict_to(int l, const double *fine, double *coarse);
     void interpolate(int l, const double *coarse, double *fine, bool accumulate);
