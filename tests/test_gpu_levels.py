@@ -130,6 +130,25 @@ def test_coarse_factor(ne, levels, graphs):
         assert rel(mg._coarseSolve(b), om.coarse_solve(b)) < 1e-9
 
 
+# wide bands (more than 512 pairs of panel blocks: the panel gets a launch of its own), long ones (more than 128 block
+# columns: wide strips of the inverse) and both, against the operator itself: the solution's error, u kappa at most, is seen
+# through A as u kappa of b, with the 1e-9 of test_coarse_factor
+@pytest.mark.parametrize("ne", [(4, 52, 52), (40, 24, 24), (12, 60, 60)])
+def test_coarse_factor_wide(ne):
+    import voxelfem_amd
+
+    tps = wl.configure(voxelfem_amd.pyVoxelFEM, ne, wl.CANTILEVER_BC, wl.noise_density(ne, 0))
+    mg = tps.multigridSolver(1)
+    mg.updateStiffnessMatrices()
+    n = [e // 2 + 1 for e in ne]
+    free = np.arange(int(np.prod(n))) >= n[1] * n[2]  # x = 0 is clamped
+    b = np.random.default_rng(6).normal(size=(len(free), 3))
+    b[~free] = 0
+    x = mg._coarseSolve(b)
+    assert not x[~free].any()
+    assert rel(mg.applyK(1, x)[free], b[free]) < 1e-9
+
+
 # stiff voxels floating in void: diagonal blocks of the coarsest matrix are nearly singular. Cholesky's error does not
 # exceed a modest multiple of u kappa, kappa the condition number of the matrix scaled to a unit diagonal (van der Sluis);
 # the stable orders of elimination reach a third of u kappa here, so u kappa itself is the bound. Reference: refined in long

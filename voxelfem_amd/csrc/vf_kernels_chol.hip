@@ -307,10 +307,32 @@ __device__ __forceinline__ void panel_rows(double *sP, const double *sL, double 
     for (int j = 0; j < 4; ++j) panel_put(v[j], j, sP, Lp, ld, w, li, lk);
 }
 
+// ---- L_{k+a,k} of the whole panel, for wide bands (grid: systems x m)
+__global__ void __launch_bounds__(TPB) k_band_panel(int k, int nb, int kb, const double *__restrict__ B,
+                                                    const double *__restrict__ Linv, double *__restrict__ XT, size_t zB,
+                                                    size_t zL, size_t zX, const int *__restrict__ nbz) {
+    const size_t ld = (size_t)nb * NB;
+    const int z = blockIdx.x, a = blockIdx.y + 1, I = k + a;
+    if (nbz) nb = min(nb, nbz[z]);
+    if (I >= nb) return;
+    __shared__ double sL[NB * LS];
+    const int t = threadIdx.x, w = t >> 6, l = t & 63;
+    panel_block(bandblk(B + z * zB, kb, I, a), Linv + z * zL + (size_t)k * BB, sL,
+                XT + z * zX + (size_t)I * NB * ld + (size_t)k * NB, ld, w, l & 15, l >> 4);
+}
+// a 64 x 64 block of the panel from there into LDS
+__device__ __forceinline__ void load_panel(const double *__restrict__ Lp, size_t ld, double *sL, int t) {
+    double v[BB / TPB];
+#pragma unroll
+    for (int q = 0; q < BB / TPB; ++q) v[q] = Lp[(size_t)((q * TPB + t) / NB) * ld + t % NB];
+#pragma unroll
+    for (int q = 0; q < BB / TPB; ++q) sL[(q * TPB + t) / NB * LS + t % NB] = v[q];
+}
+
 // ---- everything that block column k allows once Linv_k is known (grid: systems x roles):
 //   roles 0 .. m (m + 1) / 2 - 1, m = min(kb, nb - 1 - k): the pair (a, b), 1 <= b <= a <= m, forms L_{k+a,k} and
-//     L_{k+b,k} from the panel (each pair for itself: the products cost less than a launch between panel and update)
-//     and subtracts their product from A_{k+a,k+b}. Pairs with b = 1 store L_{k+a,k} in the lower block triangle of XT,
+//     L_{k+b,k} from the panel (each pair for itself: the products cost less than a launch between panel and update;
+//     PANEL: k_band_panel has formed them, see band_steps) and subtracts their product from A_{k+a,k+b}. Pairs with b = 1 store L_{k+a,k} in the lower block triangle of XT,
 //     which nothing else uses. Role 0 is the pair (1, 1), which goes on to invert the factor of diagonal block k + 1:
 //     that is the chain from launch to launch;
 //   the roles after them: strips of 16 CT columns of block row k of X, X_kJ = -Linv_k sum_q L_{k,k-q} X_{k-q,J}
@@ -319,7 +341,7 @@ __device__ __forceinline__ void panel_rows(double *sP, const double *sL, double 
 // 4131 unknowns, kb = 5: 61 launches of 16.3 us against 183 of 13.0 (panel), 13.1 (update) and 52.2 us (diagonal block)
 // and 61 of 14.8 us for the rows of X: 1.01 against 5.66 ms. Of the 16 us the loads take 1.7, the panel 1.7, the update
 // 1.9, the diagonal block 8.6 (four 16 x 16 factors of 1.4 us one after the other) and the launch the rest.
-template <int CT>
+template <int CT, bool PANEL>
 __global__ void __launch_bounds__(TPB) k_band_step(int k, int nb, int kb, double *__restrict__ B, double *__restrict__ Linv,
                                                    double *__restrict__ X, double *__restrict__ XT, int *__restrict__ flag,
                                                    size_t zB, size_t zL, size_t zX, const int *__restrict__ nbz) {
@@ -349,10 +371,12 @@ __global__ void __launch_bounds__(TPB) k_band_step(int k, int nb, int kb, double
             constexpr uint64_t tr = 0x3323213210, tc = 0x3221110000;  // row and column of tile q, a nibble each
             const double *A = bandblk(B, kb, I, a);
             double va[16], vl[16], old[3][4];
+            if (!PANEL) {
 #pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                va[q] = A[q * TPB + t];
-                vl[q] = Lk[q * TPB + t];
+                for (int q = 0; q < 16; ++q) {
+                    va[q] = A[q * TPB + t];
+                    vl[q] = Lk[q * TPB + t];
+                }
             }
             const int wu = __builtin_amdgcn_readfirstlane(w);
             int ti[3], tj[3];
@@ -364,13 +388,17 @@ __global__ void __launch_bounds__(TPB) k_band_step(int k, int nb, int kb, double
 #pragma unroll
                 for (int v = 0; v < 4; ++v) old[q][v] = Aij[(16 * ti[q] + 4 * v + lk) * NB + 16 * tj[q] + li];
             }
+            if (PANEL) {
+                load_panel(Lp, ld, sP, t);
+            } else {
 #pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                sP[(q * TPB + t) / NB * LS + t % NB] = va[q];
-                sQ[(q * TPB + t) / NB * LS + t % NB] = vl[q];
+                for (int q = 0; q < 16; ++q) {
+                    sP[(q * TPB + t) / NB * LS + t % NB] = va[q];
+                    sQ[(q * TPB + t) / NB * LS + t % NB] = vl[q];
+                }
+                __syncthreads();
+                panel_rows(sP, sQ, a == 1 ? Lp : nullptr, ld, w, li, lk);
             }
-            __syncthreads();
-            panel_rows(sP, sQ, a == 1 ? Lp : nullptr, ld, w, li, lk);
             __syncthreads();
             dx4 v[3];
 #pragma unroll
@@ -406,8 +434,13 @@ __global__ void __launch_bounds__(TPB) k_band_step(int k, int nb, int kb, double
         for (int j = 0; j < 4; ++j)
 #pragma unroll
             for (int q = 0; q < 4; ++q) old[j][q] = Aij[(16 * w + 4 * q + lk) * NB + 16 * j + li];
-        panel_block(bandblk(B, kb, I, a), Lk, sP, b == 1 ? Lp : nullptr, ld, w, li, lk);
-        panel_block(bandblk(B, kb, J, b), Lk, sQ, nullptr, ld, w, li, lk);
+        if (PANEL) {
+            load_panel(Lp, ld, sP, t);
+            load_panel(XT + (size_t)J * NB * ld + (size_t)k * NB, ld, sQ, t);
+        } else {
+            panel_block(bandblk(B, kb, I, a), Lk, sP, b == 1 ? Lp : nullptr, ld, w, li, lk);
+            panel_block(bandblk(B, kb, J, b), Lk, sQ, nullptr, ld, w, li, lk);
+        }
         __syncthreads();
         dx4 v[4];
 #pragma unroll
@@ -596,21 +629,28 @@ void band_cholesky_inverse(const Grid &g, const double *Ke, const int *red, int 
     band_factor_inverse(n, kb, B, Linv, X, XT, flag, s);
 }
 
-// the launches of the factorization and the inverse for nsys systems (see k_band_step). Rows of X with many strips in
-// flight take the wide ones, which read each band block a quarter as often: above 512 narrow strips (two workgroups on
-// every CU, as many as the LDS holds at once). Whole runs with narrow strips only / wide only / this rule, in ms: a
-// 64 x 32 x 32 solve 4.20 / 5.18 / 4.22, forty layers of 160 x 80 x 80 in batches 257.2 / 250.1 / 249.9.
+// the launches of the factorization and the inverse for nsys systems (see k_band_step). Both rules compare with the
+// workgroups that run at once, two on every CU (as many as the LDS holds). Rows of X with more narrow strips than that take
+// the wide ones, which read each band block a quarter as often: whole runs with narrow strips only / wide only / this rule,
+// in ms: a 64 x 32 x 32 solve 4.20 / 5.18 / 4.22, forty layers of 160 x 80 x 80 in batches 257.2 / 250.1 / 249.9. With more
+// pairs than that, the panel gets a launch of its own instead of being formed again by every pair: 14739 unknowns, kb = 14
+// 15.4 either way (16.8 with the panel launch always), 24843, kb = 93 104 -> 88 ms, 23409, kb = 122 187 -> 142 ms (the
+// separate launches and vector-unit products before k_band_step: 162).
 static void band_steps(int nsys, const int *nbz, int nb, int kb, double *B, double *Linv, double *X, double *XT, int *flags,
                        size_t zB, size_t zL, size_t zX, hipStream_t s) {
+    const long room = 2L * cu_count();
     hipLaunchKernelGGL(k_band_first, dim3(nsys), dim3(TPB), 0, s, kb, B, Linv, flags, zB, zL);
     for (int k = 0; k < nb; ++k) {
         const int m = std::min(kb, nb - 1 - k), pairs = m * (m + 1) / 2;
-        if ((long)nsys * (k + 1) * 4 <= 512)
-            hipLaunchKernelGGL(k_band_step<1>, dim3(nsys, pairs + (k + 1) * 4), dim3(TPB), 0, s, k, nb, kb, B, Linv, X, XT,
-                               flags, zB, zL, zX, nbz);
-        else
-            hipLaunchKernelGGL(k_band_step<4>, dim3(nsys, pairs + k + 1), dim3(TPB), 0, s, k, nb, kb, B, Linv, X, XT, flags,
-                               zB, zL, zX, nbz);
+        const bool panel = (long)nsys * pairs > room;
+        if (panel) hipLaunchKernelGGL(k_band_panel, dim3(nsys, m), dim3(TPB), 0, s, k, nb, kb, B, Linv, XT, zB, zL, zX, nbz);
+        const bool narrow = (long)nsys * (k + 1) * 4 <= room;
+        const dim3 grid(nsys, pairs + (narrow ? 4 : 1) * (k + 1));
+        auto step = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, dim3(TPB), 0, s, k, nb, kb, B, Linv, X, XT, flags, zB, zL, zX, nbz);
+        };
+        if (narrow) panel ? step(k_band_step<1, true>) : step(k_band_step<1, false>);
+        else panel ? step(k_band_step<4, true>) : step(k_band_step<4, false>);
     }
     VF_HIP(hipGetLastError());
 }
