@@ -75,6 +75,15 @@ def test_stacked_levels_and_short_last_layer(pv, levels, inc):
     _check(seq, _run(pv, sim, levels, inc, "fp64", True, 2), f"L={levels} increment {inc}")
 
 
+def test_stacked_wide_strips(pv):
+    """Eight structures of up to fifty block columns: their rows of the inverse take the wide strips from the
+    seventeenth on (more than 512 narrow ones), those of the sequential evaluator the narrow ones."""
+    ne = (16, 24, 16)
+    sim = _lbl_sim(pv, ne, 13)
+    seq = _run(pv, sim, 1, 3, "fp64", False)
+    _check(seq, _run(pv, sim, 1, 3, "fp64", True, 8), "wide strips")
+
+
 def test_stacked_full_multigrid_and_ramp(pv):
     ne = (16, 8, 8)
     sim = _lbl_sim(pv, ne, 5, pv.InterpolationLaw.RAMP)
