@@ -410,7 +410,7 @@ struct vf_mg {
     double Chat[8 * 576];
     L1Coef l1c;  // constants of the level-1 rows formed from the fine moduli
     DBuf<double> dChat, dphi, dM2, dKe0;
-    DBuf<float> dChat32;
+    DBuf<float> dChat32, dCw32;
     bool symmetricGS = true;
     bool useGraphs = false;  // replay the steady-state PCG iteration from a captured HIP graph
     // the last solve's iteration graph, destroyed during the next solve's capture (while the device is busy)
@@ -507,7 +507,7 @@ struct vf_mg {
     // hierarchy buffers and work vectors are reused by the next evaluation with the same layers and
     // constraints (the moduli, hierarchy and factors are recomputed every time)
     std::vector<std::shared_ptr<StackedBatch>> stackCache;
-    // the coarsened element matrices (Chat and the level-2 path matrices) of
+    // the coarsened element matrices (Chat, the level-2 path matrices and the Walsh form of Chat_0) of
     // another solver, so that both build identical level operators from the same moduli
     void copy_coarsening(const vf_mg &o) {
         std::copy(o.Chat, o.Chat + 8 * 576, Chat);
@@ -517,7 +517,7 @@ struct vf_mg {
             dst.resize(src.size());
             d2d(dst.data(), src.data(), src.size(), st());
         };
-        dup(dChat, o.dChat); dup(dChat32, o.dChat32); dup(dphi, o.dphi); dup(dM2, o.dM2);
+        dup(dChat, o.dChat); dup(dChat32, o.dChat32); dup(dphi, o.dphi); dup(dM2, o.dM2); dup(dCw32, o.dCw32);
     }
     // level-0 views used by the cycles (set per preconditioner call)
     double *x0v = nullptr, *b0v = nullptr;
@@ -624,6 +624,28 @@ struct vf_mg {
         std::vector<float> c32(Chat, Chat + 8 * 576);
         h2d(dChat.data(), Chat, 8 * 576, st());
         h2d(dChat32.data(), c32.data(), 8 * 576, st());
+        // child 0's matrix in the Walsh basis for the element-wise level-1 product: Cw = W^T Chat_0 W / 64
+        std::vector<float> cw32(576, 0.0f);
+        {
+            auto wal = [](int l, int k) {
+                int v = 1;
+                for (int a = 0; a < 3; ++a)
+                    if ((k >> (2 - a)) & 1) v *= ((l >> (2 - a)) & 1) ? 1 : -1;
+                return v;
+            };
+            for (int k = 0; k < 8; ++k)
+                for (int a = 0; a < 3; ++a)
+                    for (int kp = 0; kp < 8; ++kp)
+                        for (int c = 0; c < 3; ++c) {
+                            double acc = 0;
+                            for (int l = 0; l < 8; ++l)
+                                for (int m = 0; m < 8; ++m)
+                                    acc += wal(l, k) * Chat[(3 * l + a) * 24 + 3 * m + c] * wal(m, kp);
+                            cw32[(3 * k + a) * 24 + 3 * kp + c] = (float)(acc / 64.0);
+                        }
+        }
+        dCw32.resize(576);
+        h2d(dCw32.data(), cw32.data(), 576, st());
         h2d(dphi.data(), phi, 512, st());
         if (L >= 2) {
             std::vector<double> M2(64 * 576, 0.0);
@@ -784,8 +806,16 @@ struct vf_mg {
             float tr[3], ts[3];
             tr[0] = best([&] { launch_block_apply<T>(g1, blocksp<T>(1), u.data(), y.data(), rhs.data(), dm(1),
                                                      AM_RESIDUAL, s); });
-            tr[1] = best([&] { launch_l1_apply<T>(g1, g, Chatp<T>(), l1c, Ep<T>(), u.data(), y.data(), rhs.data(), dm(1),
-                                                  AM_RESIDUAL, sim->structured, s); });
+            auto vec = [&](const float *cw) {
+                return best([&] { launch_l1_apply<T>(g1, g, Chatp<T>(), l1c, cw, Ep<T>(), u.data(), y.data(), rhs.data(),
+                                                     dm(1), AM_RESIDUAL, sim->structured, s); });
+            };
+            tr[1] = vec(nullptr);
+            if (p == 1) {
+                const float w = vec(dCw32.data());
+                l1Walsh32 = w < tr[1];
+                tr[1] = std::min(tr[1], w);
+            }
             tr[2] = best([&] { launch_l1_apply_mfma<T>(g1, g, Chatp<T>(), Ep<T>(), u.data(), y.data(), rhs.data(),
                                                        dm(1), AM_RESIDUAL, s); });
             // one forward sweep, from the same start each time
@@ -825,6 +855,7 @@ struct vf_mg {
     // level-1 form of the residual ([p][0]) and of the smoother ([p][1]) the tuner chose: 0 assembled block
     // rows, 1 on the fly on the vector units, 2 on the fly on the matrix cores; -1 not tuned
     int l1Tuned[2][2] = {{-1, -1}, {-1, -1}};
+    bool l1Walsh32 = true;  // form 1 of the FP32 residual: element by element in the Walsh basis, or the factorised rows
     int l1_form(int p, int op) const {
         if (!(l1Blocks && L >= 2)) return g_kernel_variant == 5 ? 2 : 1;  // no block rows: on the fly
         return l1Tuned[p][op] >= 0 ? l1Tuned[p][op] : 0;
@@ -843,8 +874,8 @@ struct vf_mg {
         else if (l == 0 && fam == 1) launch_fine_apply_tiled<T>(lv[0]->g, Fp<T>(), Ep<T>(), u, y, b, mask, mode, st());
         else if (l == 0) launch_fine_apply<T>(lv[0]->g, K0p<T>(), Ep<T>(), u, y, b, mask, mode, st());
         else if (l == 1 && l1_form(pidx<T>(), 0) == 1)
-            launch_l1_apply<T>(lv[1]->g, lv[0]->g, Chatp<T>(), l1c, Ep<T>(), u, y, b, mask, mode, sim->structured,
-                               st());
+            launch_l1_apply<T>(lv[1]->g, lv[0]->g, Chatp<T>(), l1c, pidx<T>() == 1 && l1Walsh32 ? dCw32.data() : nullptr,
+                               Ep<T>(), u, y, b, mask, mode, sim->structured, st());
         else if (l == 1 && l1_form(pidx<T>(), 0) == 2)
             launch_l1_apply_mfma<T>(lv[1]->g, lv[0]->g, Chatp<T>(), Ep<T>(), u, y, b, mask, mode, st());
         else if (l < L) launch_block_apply<T>(lv[l]->g, blocksp<T>(l), u, y, b, mask, mode, st());

@@ -199,10 +199,12 @@ inline L1Coef l1_coef_of(double young, double nu, const double h[3]) {
     return c;
 }
 // level-1 operator on the fly from the fine moduli (reflect: the element matrix is that of an isotropic box element,
-// whose rows are formed by sum factorisation from `sep`; otherwise from Chat)
+// whose rows are formed by sum factorisation from `sep` or, in FP32 and with Cw = W^T Chat_0 W / 64 (rows (3 k + a),
+// columns (3 k' + c), W[l][k] = prod over the axes a in k of the side of node l along a), element by element in the Walsh
+// basis; otherwise from Chat)
 template <typename T>
-void launch_l1_apply(const Grid &gc, const Grid &gf, const T *Chat, const L1Coef &sep, const T *Ef, const T *u, T *y,
-                     const T *b, const uint8_t *dmask, int mode, bool reflect, hipStream_t s);
+void launch_l1_apply(const Grid &gc, const Grid &gf, const T *Chat, const L1Coef &sep, const float *Cw, const T *Ef,
+                     const T *u, T *y, const T *b, const uint8_t *dmask, int mode, bool reflect, hipStream_t s);
 // level-1 operator on the fly with the matrix cores (full Chat, any element matrix)
 template <typename T>
 void launch_l1_apply_mfma(const Grid &gc, const Grid &gf, const T *Chat, const T *Ef, const T *u, T *y, const T *b,
