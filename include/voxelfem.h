@@ -329,6 +329,10 @@ int vf_mg_tuning(vf_mg *mg, int precision, int choice[2], double ms[6]);
  * Implementation detail of this library: the reference always applies level 1 on the fly
  * (MultigridSolver.hh:483-491). */
 int vf_mg_tuning_level1(vf_mg *mg, int precision, int choice[2], double ms[6]);
+/* Whether the sum-factorised level-1 rows of an isotropic material on fine elements of size h reproduce the
+ * coarsened element matrices chat (8 x 24 x 24, host memory; the children's order and DoF order of the solver):
+ * the condition under which the on-the-fly level-1 forms use them. No device work. */
+int vf_level1_factorised(double young, double poisson, const double h[3], const double *chat, int *factorised);
 /* Replay the steady-state PCG iteration of vf_mg_pcg from a HIP graph captured on its second iteration
  * (enable = 1) instead of launching its kernels one by one (0, the default). Needs the solver's stream
  * to be a created stream, not the null stream; otherwise the iterations run eagerly. Same results. */

@@ -90,3 +90,30 @@ def test_grid_changing_filter_dimensions():
         lg.setOutputDimensions([4, 4, 4])
     with pytest.raises(RuntimeError, match="not set"):
         pv.VertexToCellFilter().apply(np.zeros(4))
+
+
+@pytest.mark.parametrize("h", [(1.0, 1.0, 1.0), (0.5, 1.5, 2.0)])
+@pytest.mark.parametrize("young,nu", [(1.0, 0.3), (210.0, 0.0), (3.0, 0.45)])
+def test_level1_rows_taken_for_isotropic_matrices_only(h, young, nu):
+    """The sum-factorised level-1 rows stand for an isotropic box element; any other matrix, an orthotropic one with the
+    same reflection symmetry among them, keeps the rows formed from the coarsened matrices."""
+    import voxelfem_amd
+    from oracle import oracle as orc
+
+    lib = ctypes.CDLL(voxelfem_amd.LIBRARY_PATH)
+
+    def factorised(chat):
+        hh, c, ok = (ctypes.c_double * 3)(*h), np.ascontiguousarray(chat), ctypes.c_int(-1)
+        assert lib.vf_level1_factorised(ctypes.c_double(young), ctypes.c_double(nu), hh, c.ctypes.data_as(ctypes.c_void_p),
+                                        ctypes.byref(ok)) == 0
+        return ok.value
+
+    s = orc.Sim((4, 4, 4), [0.0, 0.0, 0.0], [4 * v for v in h])
+    s.set_etensor(young, nu)
+    s.set_densities(np.ones(64))
+    chat = orc.MG(s, 1).chat()
+    assert factorised(chat) == 1
+    # components scaled by d_a d_c, as a congruence of the tensor: orthotropic, no longer isotropic
+    d = np.tile([1.0, 1.0 + 1e-6, 1.0], 8)
+    assert factorised(chat * d[:, None] * d) == 0
+    assert factorised(np.full_like(chat, np.nan)) == 0

@@ -409,6 +409,7 @@ struct vf_mg {
     double phi[512];
     double Chat[8 * 576];
     L1Coef l1c;  // constants of the level-1 rows formed from the fine moduli
+    bool l1Sep = false;  // whether they give this element matrix (structured, and of an isotropic material)
     DBuf<double> dChat, dphi, dM2, dKe0;
     DBuf<float> dChat32, dCw32;
     bool symmetricGS = true;
@@ -512,6 +513,7 @@ struct vf_mg {
     void copy_coarsening(const vf_mg &o) {
         std::copy(o.Chat, o.Chat + 8 * 576, Chat);
         l1c = o.l1c;
+        l1Sep = o.l1Sep;
         std::copy(o.phi, o.phi + 512, phi);
         auto dup = [&](auto &dst, const auto &src) {
             dst.resize(src.size());
@@ -618,6 +620,7 @@ struct vf_mg {
         std::fill(Chat, Chat + 8 * 576, 0.0);
         for (int fi = 0; fi < 8; ++fi) coarsen_into(phi, fi, sim->K0h, Chat + fi * 576);
         l1c = l1_coef_of(sim->young, sim->poisson, sim->h);
+        l1Sep = sim->structured && l1_rows_factorise(l1c, Chat);
         dChat.resize(8 * 576);
         dChat32.resize(8 * 576);
         dphi.resize(512);
@@ -808,7 +811,7 @@ struct vf_mg {
                                                      AM_RESIDUAL, s); });
             auto vec = [&](const float *cw) {
                 return best([&] { launch_l1_apply<T>(g1, g, Chatp<T>(), l1c, cw, Ep<T>(), u.data(), y.data(), rhs.data(),
-                                                     dm(1), AM_RESIDUAL, sim->structured, s); });
+                                                     dm(1), AM_RESIDUAL, l1Sep, s); });
             };
             tr[1] = vec(nullptr);
             if (p == 1) {
@@ -832,7 +835,7 @@ struct vf_mg {
                 for (int c = 0; c < 8; ++c) {
                     if (form == 0) launch_block_gs<T>(g1, blocksp<T>(1), u1.data(), b1.data(), dm(1), c, 1, s);
                     else if (form == 1)
-                        launch_l1_gs<T>(g1, g, Chatp<T>(), l1c, Ep<T>(), u1.data(), b1.data(), dm(1), c, 1, sim->structured, s);
+                        launch_l1_gs<T>(g1, g, Chatp<T>(), l1c, Ep<T>(), u1.data(), b1.data(), dm(1), c, 1, l1Sep, s);
                     else launch_l1_gs_mfma<T>(g1, g, Chatp<T>(), Ep<T>(), u1.data(), b1.data(), dm(1), c, 1, s);
                 }
             };
@@ -875,7 +878,7 @@ struct vf_mg {
         else if (l == 0) launch_fine_apply<T>(lv[0]->g, K0p<T>(), Ep<T>(), u, y, b, mask, mode, st());
         else if (l == 1 && l1_form(pidx<T>(), 0) == 1)
             launch_l1_apply<T>(lv[1]->g, lv[0]->g, Chatp<T>(), l1c, pidx<T>() == 1 && l1Walsh32 ? dCw32.data() : nullptr,
-                               Ep<T>(), u, y, b, mask, mode, sim->structured, st());
+                               Ep<T>(), u, y, b, mask, mode, l1Sep, st());
         else if (l == 1 && l1_form(pidx<T>(), 0) == 2)
             launch_l1_apply_mfma<T>(lv[1]->g, lv[0]->g, Chatp<T>(), Ep<T>(), u, y, b, mask, mode, st());
         else if (l < L) launch_block_apply<T>(lv[l]->g, blocksp<T>(l), u, y, b, mask, mode, st());
@@ -928,8 +931,7 @@ struct vf_mg {
                 launch_fine_gs_gather_f<T>(lv[0]->g, Fp<T>(), Ep<T>(), u, b, dm(0), color, forward, st());
             else if (l == 0) launch_fine_gs<T>(lv[0]->g, K0p<T>(), Ep<T>(), u, b, dm(0), color, forward, st());
             else if (l == 1 && l1_form(pidx<T>(), 1) == 1)
-                launch_l1_gs<T>(lv[1]->g, lv[0]->g, Chatp<T>(), l1c, Ep<T>(), u, b, dm(1), color, forward, sim->structured,
-                                st());
+                launch_l1_gs<T>(lv[1]->g, lv[0]->g, Chatp<T>(), l1c, Ep<T>(), u, b, dm(1), color, forward, l1Sep, st());
             else if (l == 1 && l1_form(pidx<T>(), 1) == 2)
                 launch_l1_gs_mfma<T>(lv[1]->g, lv[0]->g, Chatp<T>(), Ep<T>(), u, b, dm(1), color, forward, st());
             else launch_block_gs<T>(lv[l]->g, blocksp<T>(l), u, b, dm(l), color, forward, st());
@@ -3835,6 +3837,13 @@ int vf_mg_tuning_level1(vf_mg *mg, int precision, int choice[2], double ms[6]) {
     choice[0] = mg->l1_form(p, 0);
     choice[1] = mg->l1_form(p, 1);
     for (int i = 0; i < 6; ++i) ms[i] = mg->tuneMs[p][6 + i];
+    VF_API_END
+}
+
+int vf_level1_factorised(double young, double poisson, const double h[3], const double *chat, int *factorised) {
+    VF_API_BEGIN
+    need(h && chat && factorised, "invalid argument");
+    *factorised = l1_rows_factorise(l1_coef_of(young, poisson, h), chat) ? 1 : 0;
     VF_API_END
 }
 

@@ -198,6 +198,8 @@ inline L1Coef l1_coef_of(double young, double nu, const double h[3]) {
     c.ratio = lam / mu;
     return c;
 }
+// whether those rows reproduce the coarsened element matrices Chat (8 x 24 x 24)
+bool l1_rows_factorise(const L1Coef &c, const double *Chat);
 // level-1 operator on the fly from the fine moduli (reflect: the element matrix is that of an isotropic box element,
 // whose rows are formed by sum factorisation from `sep` or, in FP32 and with Cw = W^T Chat_0 W / 64 (rows (3 k + a),
 // columns (3 k' + c), W[l][k] = prod over the axes a in k of the side of node l along a), element by element in the Walsh

@@ -8,7 +8,9 @@
 // which the compiler turns into scalar loads shared by the whole wavefront.
 #include "vf_internal.hpp"
 
+#include <algorithm>
 #include <climits>
+#include <cmath>
 #include <type_traits>
 
 namespace vf {
@@ -460,14 +462,14 @@ struct L1CoefT {
 };
 template <typename T, int DL>
 struct Ax4 {  // functionals of four cells at offset DL
-    static __device__ __forceinline__ T M(T a, T b, T c, T d) {
+    static __host__ __device__ __forceinline__ T M(T a, T b, T c, T d) {
         return DL < 0 ? a + b : DL > 0 ? c + d : T(0.5) * (a + d) + T(3.5) * (b + c);
     }
-    static __device__ __forceinline__ T D(T a, T b, T c, T d) { return DL < 0 ? -(a + b) : DL > 0 ? -(c + d) : (a + b) + (c + d); }
-    static __device__ __forceinline__ T G(T a, T b, T c, T d) {
+    static __host__ __device__ __forceinline__ T D(T a, T b, T c, T d) { return DL < 0 ? -(a + b) : DL > 0 ? -(c + d) : (a + b) + (c + d); }
+    static __host__ __device__ __forceinline__ T G(T a, T b, T c, T d) {
         return DL < 0 ? T(3) * a + b : DL > 0 ? -(c + T(3) * d) : (a + T(3) * b) - (T(3) * c + d);
     }
-    static __device__ __forceinline__ T T_(T a, T b, T c, T d) {
+    static __host__ __device__ __forceinline__ T T_(T a, T b, T c, T d) {
         return DL < 0 ? -(a + T(3) * b) : DL > 0 ? T(3) * c + d : (a + T(3) * b) - (T(3) * c + d);
     }
 };
@@ -1121,6 +1123,43 @@ void launch_fine_apply(const Grid &g, const T *K0, const T *E, const T *u, T *y,
         hipLaunchKernelGGL(k_zero_detached<T>, dim3(nblocks(cz)), dim3(TPB), 0, s, g, y);
     }
     VF_HIP(hipGetLastError());
+}
+
+// Every block of every child's matrix against the rows' formulas (see l1_row_sep) with that child's modulus alone
+bool l1_rows_factorise(const L1Coef &k, const double *Chat) {
+    // functional q (M, D, G, T) at offset o of one of the four cells along an axis
+    auto axis = [](int q, int o, int cell) {
+        double c[4] = {0, 0, 0, 0};
+        c[cell] = 1;
+        auto at = [&](auto A) {
+            using Ax = decltype(A);
+            return q == 0 ? Ax::M(c[0], c[1], c[2], c[3]) : q == 1 ? Ax::D(c[0], c[1], c[2], c[3])
+                   : q == 2 ? Ax::G(c[0], c[1], c[2], c[3]) : Ax::T_(c[0], c[1], c[2], c[3]);
+        };
+        return o < 0 ? at(Ax4<double, -1>()) : o > 0 ? at(Ax4<double, 1>()) : at(Ax4<double, 0>());
+    };
+    double most = 0;
+    for (int i = 0; i < 8 * 576; ++i) most = std::max(most, std::fabs(Chat[i]));
+    for (int fi = 0; fi < 8; ++fi)
+        for (int l = 0; l < 8; ++l)
+            for (int m = 0; m < 8; ++m) {
+                double W[3][3];
+                for (int p = 0; p < 3; ++p)
+                    for (int q = 0; q < 3; ++q) {
+                        W[p][q] = 1;
+                        for (int a = 0; a < 3; ++a) {
+                            const int bl = (l >> (2 - a)) & 1, bm = (m >> (2 - a)) & 1, bf = (fi >> (2 - a)) & 1;
+                            W[p][q] *= axis(p == q ? (a == p ? 1 : 0) : a == p ? 2 : a == q ? 3 : 0, bm - bl, bl ? bf : 2 + bf);
+                        }
+                    }
+                const double S = k.mu[0] * W[0][0] + k.mu[1] * W[1][1] + k.mu[2] * W[2][2];
+                for (int c = 0; c < 3; ++c)
+                    for (int d = 0; d < 3; ++d) {
+                        const double v = c == d ? S + k.lm[c] * W[c][c] : k.cm[c + d - 1] * (W[d][c] + k.ratio * W[c][d]);
+                        if (!(std::fabs(v - Chat[fi * 576 + (3 * l + c) * 24 + 3 * m + d]) <= 1e-13 * most)) return false;
+                    }
+            }
+    return true;
 }
 
 template <typename T>
