@@ -701,8 +701,8 @@ __device__ __forceinline__ T row16_sum(T v) {
     return v;
 }
 
-// tile and workgroup of the two-launch sweep: 28 of the 32 rows of lanes hold a node at the first colour
-constexpr int BP_TY = 4, BP_TZ = 12, BP_NT = 512, CUS = 256;
+// tile and workgroup of the two-launch sweep: 27 of the 32 rows of lanes hold a node at the first colour
+constexpr int BP_TY = 4, BP_TZ = 12, BP_NT = 512;
 
 constexpr int RL = 16;          // lanes per node
 constexpr int RN16 = TPB / RL;  // rows of lanes per workgroup
@@ -843,8 +843,8 @@ __global__ void __launch_bounds__(TPB) k_block_gs(Grid g, const T *__restrict__ 
 // block_row16, and a node for every row of lanes at each of the four positions: all block rows are requested before the
 // first colour, the off-plane part of the sums is taken as they arrive, and what a colour waits for is only three values
 // from LDS (a lane has at most one slot in the plane: s = 9 .. 17 are lanes 9 .. 15 and 0, 1). Bound by latency: about
-// 3.5 us of launch, one round of loads and four colours, 10 us against 15 for four colour launches. Requested one
-// colour ahead instead of all at once (tiles of 4 x 8): 12 us.
+// 3.5 us of launch, one round of loads and four colours, 9 us against 15 for four colour launches. Requested one colour
+// ahead instead of all at once (tiles of 4 x 8): 12 us, where all at once took 10.
 // uin: the planes of this parity before the sweep, unb: the neighbour planes, uout (!= uin): receives this parity's
 // planes, every node. zin bit 0 / 1: uin / unb is zero.
 template <typename T, int TY, int TZ, int NT, bool FWD>
@@ -1270,11 +1270,12 @@ void launch_block_gs(const Grid &g, const T *blocks, T *u, const T *b, const uin
 
 // A workgroup holds a compute unit with its registers, so a launch is one latency long while every workgroup has a unit of
 // its own, and the halo (27 + 24 + 14 + 12 nodes for a tile of 12 per colour) costs nothing; beyond that the eight colour
-// launches are faster. Sweeps in us, two launches / eight (FP64, FP32): 33x17x17 (170 workgroups) 21.7 / 29.6,
-// 19.7 / 30.6; 27x15x13 (112) 19.7 / 29.6, 18.6 / 29.5; 45x23x19 (276) 42.6 / 31.8, 31.1 / 30.7; 65x33x33 85 / 52, 58 / 53.
+// launches are faster. Sweeps in us, two launches / eight (FP64, FP32): 27x15x13 (112 workgroups) 16.7 / 28.3, 16.0 / 30.4;
+// 33x17x17 (170) 18.7 / 28.6, 17.4 / 32.3; 41x21x21 (252) 23.6 / 29.2, 19.0 / 31.6; 45x23x19 (276) 37.7 / 29.6, 28.5 / 31.8;
+// 65x33x33 (891) 76 / 50, 57 / 44.
 bool block_gs_planes(const Grid &g) {
     const int ntY = (g.nn[1] + BP_TY - 1) / BP_TY, ntZ = (g.nn[2] + BP_TZ - 1) / BP_TZ;
-    return (long)ntY * ntZ * ((g.nn[0] + 1) / 2) <= CUS;
+    return (long)ntY * ntZ * ((g.nn[0] + 1) / 2) <= cu_count();
 }
 
 template <typename T>

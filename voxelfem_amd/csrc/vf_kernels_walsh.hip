@@ -305,26 +305,13 @@ __global__ void __launch_bounds__(256) k_zero_rows_w(Grid g, T *__restrict__ y) 
     y[(size_t)2 * g.nnodes + n] = T(0);
 }
 
-int cu_count_w() {
-    static int n = 0;
-    if (!n) {
-        int dev = 0, v = 0;
-        if (hipGetDevice(&dev) == hipSuccess &&
-            hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0)
-            n = v;
-        else
-            n = 256;
-    }
-    return n;
-}
-
 inline int cdiv(int a, int b) { return (a + b - 1) / b; }
 
 }  // namespace
 
 static int walsh_xchunk_of(const Grid &g, const void *kern, int alignX) {
     const int tiles = cdiv(g.ydet, TN) * cdiv(g.nn[2], TN);
-    const int chunks0 = plane_chunks(tiles, g.nn[0], 4 * cu_count_w(), resident_workgroups(kern, NTW));
+    const int chunks0 = plane_chunks(tiles, g.nn[0], 4 * cu_count(), resident_workgroups(kern, NTW));
     int xchunk = cdiv(g.nn[0], chunks0);
     if (alignX > 0) {  // the largest divisor of alignX not above xchunk: no x-chunk straddles a multiple of alignX
         int best = 1;
