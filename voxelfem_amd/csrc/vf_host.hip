@@ -630,22 +630,23 @@ struct vf_mg {
         // child 0's matrix in the Walsh basis for the element-wise level-1 product: Cw = W^T Chat_0 W / 64
         std::vector<float> cw32(576, 0.0f);
         {
-            auto wal = [](int l, int k) {
-                int v = 1;
-                for (int a = 0; a < 3; ++a)
-                    if ((k >> (2 - a)) & 1) v *= ((l >> (2 - a)) & 1) ? 1 : -1;
-                return v;
-            };
-            for (int k = 0; k < 8; ++k)
-                for (int a = 0; a < 3; ++a)
-                    for (int kp = 0; kp < 8; ++kp)
-                        for (int c = 0; c < 3; ++c) {
+            // W^T (M W), W[l][k] = prod over the axes a in k of the side of l along a
+            double W[8][8];
+            for (int l = 0; l < 8; ++l)
+                for (int k = 0; k < 8; ++k) W[l][k] = __builtin_popcount(k & ~l & 7) & 1 ? -1.0 : 1.0;
+            for (int a = 0; a < 3; ++a)
+                for (int c = 0; c < 3; ++c) {
+                    double MW[8][8] = {};
+                    for (int l = 0; l < 8; ++l)
+                        for (int m = 0; m < 8; ++m)
+                            for (int kp = 0; kp < 8; ++kp) MW[l][kp] += Chat[(3 * l + a) * 24 + 3 * m + c] * W[m][kp];
+                    for (int k = 0; k < 8; ++k)
+                        for (int kp = 0; kp < 8; ++kp) {
                             double acc = 0;
-                            for (int l = 0; l < 8; ++l)
-                                for (int m = 0; m < 8; ++m)
-                                    acc += wal(l, k) * Chat[(3 * l + a) * 24 + 3 * m + c] * wal(m, kp);
+                            for (int l = 0; l < 8; ++l) acc += W[l][k] * MW[l][kp];
                             cw32[(3 * k + a) * 24 + 3 * kp + c] = (float)(acc / 64.0);
                         }
+                }
         }
         dCw32.resize(576);
         h2d(dCw32.data(), cw32.data(), 576, st());

@@ -1127,17 +1127,21 @@ void launch_fine_apply(const Grid &g, const T *K0, const T *E, const T *u, T *y,
 
 // Every block of every child's matrix against the rows' formulas (see l1_row_sep) with that child's modulus alone
 bool l1_rows_factorise(const L1Coef &k, const double *Chat) {
-    // functional q (M, D, G, T) at offset o of one of the four cells along an axis
-    auto axis = [](int q, int o, int cell) {
-        double c[4] = {0, 0, 0, 0};
-        c[cell] = 1;
-        auto at = [&](auto A) {
-            using Ax = decltype(A);
-            return q == 0 ? Ax::M(c[0], c[1], c[2], c[3]) : q == 1 ? Ax::D(c[0], c[1], c[2], c[3])
-                   : q == 2 ? Ax::G(c[0], c[1], c[2], c[3]) : Ax::T_(c[0], c[1], c[2], c[3]);
-        };
-        return o < 0 ? at(Ax4<double, -1>()) : o > 0 ? at(Ax4<double, 1>()) : at(Ax4<double, 0>());
+    // F[q][o + 1][cell]: functional q (M, D, G, T) at offset o of one of the four cells along an axis
+    double F[4][3][4];
+    auto fill = [&](auto A, int o) {
+        using Ax = decltype(A);
+        for (int cell = 0; cell < 4; ++cell) {
+            const double c0 = cell == 0, c1 = cell == 1, c2 = cell == 2, c3 = cell == 3;
+            F[0][o + 1][cell] = Ax::M(c0, c1, c2, c3);
+            F[1][o + 1][cell] = Ax::D(c0, c1, c2, c3);
+            F[2][o + 1][cell] = Ax::G(c0, c1, c2, c3);
+            F[3][o + 1][cell] = Ax::T_(c0, c1, c2, c3);
+        }
     };
+    fill(Ax4<double, -1>(), -1);
+    fill(Ax4<double, 0>(), 0);
+    fill(Ax4<double, 1>(), 1);
     double most = 0;
     for (int i = 0; i < 8 * 576; ++i) most = std::max(most, std::fabs(Chat[i]));
     for (int fi = 0; fi < 8; ++fi)
@@ -1149,7 +1153,7 @@ bool l1_rows_factorise(const L1Coef &k, const double *Chat) {
                         W[p][q] = 1;
                         for (int a = 0; a < 3; ++a) {
                             const int bl = (l >> (2 - a)) & 1, bm = (m >> (2 - a)) & 1, bf = (fi >> (2 - a)) & 1;
-                            W[p][q] *= axis(p == q ? (a == p ? 1 : 0) : a == p ? 2 : a == q ? 3 : 0, bm - bl, bl ? bf : 2 + bf);
+                            W[p][q] *= F[p == q ? (a == p ? 1 : 0) : a == p ? 2 : a == q ? 3 : 0][bm - bl + 1][bl ? bf : 2 + bf];
                         }
                     }
                 const double S = k.mu[0] * W[0][0] + k.mu[1] * W[1][1] + k.mu[2] * W[2][2];
