@@ -9,7 +9,7 @@
 // The work is O(n bw^2) instead of the O(n^3) of a dense factorisation. For the solves, the explicit dense
 // lower-triangular X = L^-1 is formed block row by block row, so a coarse solve x = X^T (X b) is two bandwidth-bound
 // triangular matrix-vector products instead of a chain of small sequential triangular solves.
-// One launch per block column (k_band_step) does all of that: the chain of block columns is what bounds the
+// One launch per block column (k_band_step) does all of that (two on wide bands): the chain of block columns is what bounds the
 // factorisation, so nothing that the next diagonal block does not need sits between two links of it.
 #include "vf_internal.hpp"
 
@@ -250,7 +250,7 @@ __device__ __forceinline__ void store_linv(const double *sX, double *__restrict_
     for (int e = t; e < BB; e += TPB) Lk[e] = sX[(e / NB) * LS + e % NB];
 }
 
-// ---- the first diagonal block (grid: systems); nbz (batched, optional): system z uses its first nbz[z] blocks only
+// ---- the first diagonal block (grid: systems)
 __global__ void __launch_bounds__(TPB) k_band_first(int kb, const double *__restrict__ B, double *__restrict__ Linv,
                                                     int *__restrict__ flag, size_t zB, size_t zL) {
     B += blockIdx.x * zB;
