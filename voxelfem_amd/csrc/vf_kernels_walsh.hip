@@ -23,13 +23,14 @@
 // Measured against one with both butterflies per element, all corners through LDS, two barriers a step and the addresses
 // formed in the loop (577 vector instructions a step, now 267), in us, K u / residual: 65x33x33 FP64 9.2 / 9.3 -> 7.1 /
 // 7.1; 209x113x97 FP64 54.3 / 55.9 -> 41.7 / 43.0, FP32 36.6 / 37.4 -> 28.1 / 27.3; 257x129x129 FP64 85.6 / 111.9 -> 64.9 /
-// 99.1, FP32 58.5 / 60.9 -> 45.1 / 45.0; 385x193x193 FP64 259 / 394 -> 259 / 332, FP32 173 / 227 -> 148 / 198. At the
-// largest, K u is bound by neither the vector units (about 45%) nor the bytes (3.1 TB/s): requesting the planes two steps
+// 99.1, FP32 58.5 / 60.9 -> 45.1 / 45.0; 385x193x193 FP64 268 / 394 -> 249 / 322, FP32 173 / 227 -> 148 / 198. At the
+// largest, K u is bound by neither the vector units (about 45%) nor the bytes (3.2 TB/s, 3.9 moved): requesting the planes two steps
 // ahead costs registers that spill, and waiting for all of a step's loads before the next ones are requested changes
 // nothing.
 #include "vf_internal.hpp"
 
 #include <algorithm>
+#include <climits>
 
 namespace vf {
 namespace {
@@ -309,9 +310,15 @@ inline int cdiv(int a, int b) { return (a + b - 1) / b; }
 
 }  // namespace
 
-static int walsh_xchunk_of(const Grid &g, const void *kern, int alignX) {
+// Four workgroups per compute unit, no more than run at once: a second round costs more than it hides, e.g. in FP64
+// (K u, us) 66 against 74 at 256x128x128 elements, 146 against 151 at 320x160x160. Where an FP64 field alone no longer fits
+// the 256 MB last-level cache the launch is bound by HBM and the other way round: as many as asked for 249 against 259 at
+// 384x192x192, 405 / 416 at 448x224x224, 673 / 732 at 512x256x256 (residuals 324 / 332, 512 / 521, 902 / 909); in FP32 the
+// cap stays the better one (512x256x256: 404 against 445).
+static int walsh_xchunk_of(const Grid &g, const void *kern, int alignX, size_t word) {
     const int tiles = cdiv(g.ydet, TN) * cdiv(g.nn[2], TN);
-    const int chunks0 = plane_chunks(tiles, g.nn[0], 4 * cu_count(), resident_workgroups(kern, NTW));
+    const bool hbm = word == sizeof(double) && (size_t)3 * g.nnodes * word > (size_t)256 << 20;
+    const int chunks0 = plane_chunks(tiles, g.nn[0], 4 * cu_count(), hbm ? INT_MAX : resident_workgroups(kern, NTW));
     int xchunk = cdiv(g.nn[0], chunks0);
     if (alignX > 0) {  // the largest divisor of alignX not above xchunk: no x-chunk straddles a multiple of alignX
         int best = 1;
@@ -323,7 +330,7 @@ static int walsh_xchunk_of(const Grid &g, const void *kern, int alignX) {
 }
 int walsh_xchunk(const Grid &g, int mode, int alignX) {
     const void *kern = mode == AM_RESIDUAL ? (const void *)k_ku_walsh<double, AM_RESIDUAL> : (const void *)k_ku_walsh<double, AM_SET>;
-    return walsh_xchunk_of(g, kern, alignX);
+    return walsh_xchunk_of(g, kern, alignX, sizeof(double));
 }
 
 size_t walsh_partials(const Grid &g) { return (size_t)cdiv(g.ydet, TN) * cdiv(g.nn[2], TN) * g.nn[0]; }
@@ -340,7 +347,7 @@ void launch_fine_apply_walsh(const Grid &g, const T *C, const T *E, const T *u, 
         const int ntY = cdiv(g.ydet, TN), ntZ = cdiv(g.nn[2], TN);
         const int tiles = ntY * ntZ;
         const void *kern = mode == AM_RESIDUAL ? (const void *)k_ku_walsh<T, AM_RESIDUAL> : (const void *)k_ku_walsh<T, AM_SET>;
-        const int xchunk = walsh_xchunk_of(g, kern, alignX);
+        const int xchunk = walsh_xchunk_of(g, kern, alignX, sizeof(T));
         const int chunks = cdiv(g.nn[0], xchunk);
         if (chunks > 65535) throw std::runtime_error("grid too large for the Walsh K u");
         if (dotOut && (size_t)tiles * chunks > dotCapacity)
